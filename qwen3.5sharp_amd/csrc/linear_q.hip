@@ -785,54 +785,110 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qt(const unsigned char* __r
 // y[t][o] = Ops.DotF32(x[t], W[o]) (Ops.cs:418-449) in its order: 16 FMA
 // lanes over 16-float strides (lane j takes elements 16 k + j), one 8-float
 // stride into lanes 0-7, then HorizontalSum(acc0 + acc1) and a scalar tail.
-// Four threads per output row, thread q holding reference lanes 4q .. 4q+3
-// (a float4 of each stride when rows are 16-byte aligned); 64 rows a
-// 256-thread workgroup, one token per grid row.
-template <bool VEC>
+// Thread (group, l16) holds reference lane l16 of RT rows x TT tokens (16
+// threads a group, GR x GT groups of a 256-thread workgroup), so the order's
+// long chains run in parallel over rows, tokens and lanes and their operands
+// come from LDS: a workgroup stages KC columns of its RT GR weight rows and
+// TT GT token rows, all loads in flight at once (the next chunk's during the
+// current one's chains).  In LDS the four elements a lane takes from 64
+// columns (64 q + 16 s + l16, s < 4) lie together, so a chain's next four
+// steps are one 16-byte read; they are loaded as four dwords of 16-lane runs,
+// which also makes any width and alignment the same path.
+template <int RT, int TT, int GR, int GT, int KC>
 __global__ __launch_bounds__(256) void linear_f32(const float* __restrict__ w, const float* __restrict__ x,
-                                                  float* __restrict__ y, int n_in, int n_out) {
+                                                  float* __restrict__ y, int n_in, int n_out, int tokens) {
 #pragma clang fp contract(off)
-    const int tid = threadIdx.x, q = tid & 3;
-    const int row = blockIdx.x * 64 + (tid >> 2), t = blockIdx.y;
-    const int rr = min(row, n_out - 1);            // rows past n_out compute row n_out - 1, not stored
-    const float* a = x + (size_t)t * n_in;
-    const float* b = w + (size_t)rr * n_in;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    int i = 0;
-    for (; i + 16 <= n_in; i += 16) {
-        float av[4], bv[4];
-        if constexpr (VEC) {
-            const float4 a4 = *reinterpret_cast<const float4*>(a + i + 4 * q);
-            const float4 b4 = *reinterpret_cast<const float4*>(b + i + 4 * q);
-            av[0] = a4.x; av[1] = a4.y; av[2] = a4.z; av[3] = a4.w;
-            bv[0] = b4.x; bv[1] = b4.y; bv[2] = b4.z; bv[3] = b4.w;
-        } else {
+    constexpr int RW = RT * GR, TW = TT * GT, C4 = KC / 4;
+    constexpr int NU = (RW + TW) * C4, NL = (NU + 255) / 256;
+    __shared__ float4 tile[RW + TW][C4];
+    const int tid = threadIdx.x, l16 = tid & 15, grp = tid >> 4;
+    const int gr = grp % GR, gt = grp / GR;
+    const int row0 = blockIdx.x * RW, tok0 = blockIdx.y * TW;
+    const int main = n_in & ~15;                  // columns of the 16-wide strides
+
+    // Unit e of the staging: tile row e / C4 (weight rows, then tokens; past
+    // the end the last one again), lane e % 16 of 64-column run (e % C4) / 16.
+    // Columns past `main` read its last one and are not used.
+    float4 v[NL];
+    auto unit = [&](int i) { return NU % 256 ? min(tid + 256 * i, NU - 1) : tid + 256 * i; };
+    auto load = [&](int k0) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) { av[k] = a[i + 4 * q + k]; bv[k] = b[i + 4 * q + k]; }
+        for (int i = 0; i < NL; ++i) {
+            const int e = unit(i), r = e / C4, c = k0 + 64 * (e % C4 / 16) + l16;
+            const float* src = r < RW ? w + (size_t)min(row0 + r, n_out - 1) * n_in
+                                      : x + (size_t)min(tok0 + r - RW, tokens - 1) * n_in;
+            v[i] = make_float4(src[min(c, main - 1)], src[min(c + 16, main - 1)], src[min(c + 32, main - 1)],
+                               src[min(c + 48, main - 1)]);
         }
+    };
+    auto stage = [&] {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) acc[k] = fmaf(av[k], bv[k], acc[k]);
+        for (int i = 0; i < NL; ++i) (&tile[0][0])[unit(i)] = v[i];
+        __syncthreads();
+    };
+    float acc[RT][TT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) acc[r][t] = 0.0f;
+    // n strides of 16 columns from the chunk's start (gt: groups past GT only stage)
+    auto chains = [&](int n) {
+        if (gt >= GT) return;
+        auto quad = [&](int q, int steps) {
+            float4 wv[RT], xv[TT];
+#pragma unroll
+            for (int r = 0; r < RT; ++r) wv[r] = tile[gr + GR * r][16 * q + l16];
+#pragma unroll
+            for (int t = 0; t < TT; ++t) xv[t] = tile[RW + gt + GT * t][16 * q + l16];
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                if (s < steps)
+#pragma unroll
+                    for (int r = 0; r < RT; ++r)
+#pragma unroll
+                        for (int t = 0; t < TT; ++t)
+                            acc[r][t] = fmaf(reinterpret_cast<const float*>(&xv[t])[s],
+                                             reinterpret_cast<const float*>(&wv[r])[s], acc[r][t]);
+        };
+        // unrolled so the LDS reads run ahead of the ordered chains
+        int q = 0;
+#pragma unroll 4
+        for (; 4 * q + 4 <= n; ++q) quad(q, 4);
+        if (4 * q < n) quad(q, n - 4 * q);
+    };
+    if (main > 0) {
+        int k0 = 0;
+        load(0);
+        for (; k0 + KC < main; k0 += KC) {
+            stage();
+            load(k0 + KC);
+            chains(KC / 16);
+            __syncthreads();
+        }
+        stage();
+        chains((main - k0) >> 4);
     }
-    if (i + 8 <= n_in) {
-        if (q < 2)
 #pragma unroll
-            for (int k = 0; k < 4; ++k) acc[k] = fmaf(a[i + 4 * q + k], b[i + 4 * q + k], acc[k]);
-        i += 8;
-    }
-    // s_j = acc0_j + acc1_j: threads 0, 1 hold acc0 lanes 0-7, threads 2, 3 acc1.
-    float s[4];
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) s[k] = acc[k] + __shfl_xor(acc[k], 2, kWave);
-    // HorizontalSum: (s_k + s_{k+4}) pairs, then (0 + 2) + (1 + 3).
-    float u[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) u[k] = s[k] + __shfl_xor(s[k], 1, kWave);
-    if (q == 0 && row < n_out) {
-        const float t0 = u[0] + u[2], t1 = u[1] + u[3];
-        float sum = t0 + t1;
-        for (; i < n_in; ++i) sum += a[i] * b[i];
-        y[(size_t)t * n_out + row] = sum;
-    }
+        for (int t = 0; t < TT; ++t) {
+            const int row = row0 + gr + GR * r, tok = tok0 + gt + GT * t;
+            const float* a = x + (size_t)min(tok, tokens - 1) * n_in;
+            const float* b = w + (size_t)min(row, n_out - 1) * n_in;
+            float s = acc[r][t];
+            int i = main;
+            if (i + 8 <= n_in) {
+                if (l16 < 8) s = fmaf(a[i + l16], b[i + l16], s);
+                i += 8;
+            }
+            // acc0 + acc1, then HorizontalSum: (s_k + s_{k+4}) pairs, (0 + 2) + (1 + 3).
+            s = s + __shfl_xor(s, 8, kWave);
+            s = s + __shfl_xor(s, 4, kWave);
+            s = s + __shfl_xor(s, 2, kWave);
+            s = s + __shfl_xor(s, 1, kWave);
+            for (; i < n_in; ++i) s += a[i] * b[i];
+            if (l16 == 0 && gt < GT && row < n_out && tok < tokens) y[(size_t)tok * n_out + row] = s;
+        }
 }
 
 // ---------------------------------------------------------------- Q4_K, several tokens
@@ -1673,13 +1729,27 @@ hipError_t launch_add_rmsnorm(q35m_ctx* c, float* hidden, const float* delta, co
 
 hipError_t launch_linear_f32(q35m_ctx* c, const float* w, const float* x, float* y, int n_in, int n_out,
                              int tokens) {
-    const bool vec = n_in % 4 == 0 && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15) == 0;
-    const dim3 grid((n_out + 63) / 64, tokens);
     ProfScope ps_(c, K_F32_LINEAR);
-    if (vec)
-        hipExtLaunchKernelGGL(linear_f32<true>, grid, dim3(256), 0, c->stream, ps_.a, ps_.b, 0, w, x, y, n_in, n_out);
-    else
-        hipExtLaunchKernelGGL(linear_f32<false>, grid, dim3(256), 0, c->stream, ps_.a, ps_.b, 0, w, x, y, n_in, n_out);
+    auto go = [&](auto kern, int rw, int tw) {
+        hipExtLaunchKernelGGL(kern, dim3((n_out + rw - 1) / rw, (tokens + tw - 1) / tw), dim3(256), 0, c->stream,
+                              ps_.a, ps_.b, 0, w, x, y, n_in, n_out, tokens);
+    };
+    // One token's rows, or one token a workgroup, while those workgroups fit
+    // the CUs once; else 4 x 4 tiles, the most chains in flight, up to four
+    // workgroups a CU; else 8 x 8 tiles, half the LDS reads a chain.  Measured
+    // (us; thread per four lanes from global memory before: 17.3 at 1 token,
+    // 18.0 at 64, 82.6 at 2048 of 2560 -> 32, 153 at 2048 of 1000 -> 250):
+    // 2560 -> 32 at 1 / 64 / 256 / 512 / 2048 tokens: 4.0 / 4.9 / 11.8 / 20.8
+    // / 73.4 as 4 x 1, 4.7 / 4.9 / 6.2 / 9.1 / 26.1 as 4 x 4, 8.3 / 8.6 / 8.4
+    // / 8.7 / 16.5 as 8 x 8; 1000 -> 250 at 64 / 128 / 2048 tokens: 5.1 / 7.1
+    // / 73 as 4 x 4, 5.6 / 6.5 / 43.8 as 8 x 8 (16 x 16: 37.0, but 16 at any
+    // token count of 2560 -> 32).
+    const long rows4 = (n_out + 3) / 4, toks4 = (tokens + 3) / 4;
+    // A chunk is staged whole, so rows narrower than it take a smaller one.
+    const bool few = rows4 * toks4 <= 4L * c->n_cu;
+    if (n_in > 512 && (tokens == 1 || rows4 * tokens <= c->n_cu)) go(linear_f32<1, 1, 4, 1, 2560>, 4, 1);
+    else if (n_in <= 128) few ? go(linear_f32<1, 1, 4, 4, 128>, 4, 4) : go(linear_f32<2, 2, 4, 4, 128>, 8, 8);
+    else few ? go(linear_f32<1, 1, 4, 4, 512>, 4, 4) : go(linear_f32<2, 2, 4, 4, 256>, 8, 8);
     return hipGetLastError();
 }
 

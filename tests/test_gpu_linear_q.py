@@ -162,6 +162,22 @@ def test_linear_f32_bit_exact(ctx, n_in, n_out, tokens):
         a.free()
 
 
+@pytest.mark.parametrize("n_in,n_out,tokens", [(2569, 5, 1), (5200, 3, 2), (64, 9, 33), (527, 261, 5), (600, 264, 70),
+                                               (283, 270, 65), (15, 300, 61), (256, 8, 4100), (129, 33, 9), (100, 300, 70)])
+def test_linear_f32_tiles(ctx, n_in, n_out, tokens):
+    """Each tile shape of the F32 projection (4 rows x 1 token, 4 x 4, 8 x 8)
+    at ragged rows and tokens and around its staged column chunks (2560, 512,
+    256, 128), bit for bit."""
+    rng = np.random.default_rng(n_in + 7 * n_out + tokens)
+    w = rng.standard_normal((n_out, n_in)).astype(np.float32)
+    x = rng.standard_normal((tokens, n_in)).astype(np.float32)
+    dw, dx, dy = ctx.array((n_out, n_in), w), ctx.array((tokens, n_in), x), ctx.array((tokens, n_out))
+    ctx.linear_f32(dw, dx, dy, n_in, n_out, tokens)
+    assert np.array_equal(dy.download().view(np.uint32), oracle.linear_f32(w, x, n_in, n_out).view(np.uint32))
+    for a in (dw, dx, dy):
+        a.free()
+
+
 @pytest.mark.parametrize("qtype", [4, 6])
 def test_tiled_pieces_match_whole_launch(monkeypatch, qtype):
     """The tiled Q4_K / Q6_K kernels go in pieces of whole row and token tiles
