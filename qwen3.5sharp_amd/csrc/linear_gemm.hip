@@ -1,0 +1,497 @@
+// Quantized projections of several tokens on the matrix cores, for the formats
+// whose reference result is one exact integer sum per block or sub-block
+// followed by an fp32 chain in block order (linear_q.hip states the formats,
+// the reference's functions and the one-token kernels):
+//
+//   Q5_K    per block  acc += d (sum_s sc_s dot_s) - dmin (sum_j min_j bsums)
+//   IQ4_XS  per 32-value sub-block  acc += (d (ls - 32) dot_s) dx
+//   Q2_0C   per 256 values T; panel rows acc = fma(T, dw dx, acc), raw rows
+//           per 512 values acc += dw (T0 dx0 + T1 dx1)
+//   STQ1_0  per 256 values T; panel rows acc = fma(T, dw dx, acc), raw rows
+//           acc += (dw dx) T
+//
+// (dot_s and T exact integers, no fused multiply-add but where written), so
+// results are the reference's bits at any tile shape.
+//
+// (linear_gemm_split, below, is the form for few outputs.)  A wave holds 16
+// weight rows x 16 TT tokens.  The dots are int8 MFMAs: A is
+// the tokens' Q8_K bytes from LDS, B the rows' values, decoded in registers
+// from each lane's own share of its row (no LDS, no exchange between waves;
+// the four lane groups of a row cover its block without overlap) and loaded
+// two or more blocks ahead.  So per block a wave spends its decode once for
+// all its token tiles, and per output one multiply-add a sub-block (Q5_K), or
+// the chain's own operations.  The workgroup's waves share the tokens, CH
+// blocks at a time through two LDS buffers filled by buffer loads straight
+// into LDS while the other one is worked on.  Bound by instruction issue: Q5_K
+// at 500 tokens of 2560 -> 8192 issues on 98 % of its cycles, 448 VALU and 40
+// MFMA instructions a block of 16 rows x 64 tokens.
+#include <algorithm>
+
+#include "common.h"
+#include "q35mix_internal.h"
+#include "quant_layout.h"
+
+namespace q35 {
+namespace {
+
+// Rows of the 2-byte aligned formats are read at their own addresses.
+typedef uint32_t u32_a2 __attribute__((aligned(2)));
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+
+// A lane's share (lane group lg) of one 256-value block of its row.
+template <int QT> struct RowBlock;
+
+template <> struct RowBlock<5> {       // header; qh and qs bytes 8 lg .. + 7 of each 32
+    uint4 hdr;
+    uint2 qh, qs[4];
+    __device__ __forceinline__ void load(const unsigned char* row, int b, int lg) {
+        const unsigned char* p = row + (size_t)b * Q5K_BYTES;
+        hdr = *reinterpret_cast<const uint4*>(p);
+        qh = *reinterpret_cast<const uint2*>(p + 16 + 8 * lg);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) qs[j] = *reinterpret_cast<const uint2*>(p + 48 + 32 * j + 8 * lg);
+    }
+};
+
+template <> struct RowBlock<14> {      // header; bytes 8 (lg % 2) .. + 7 of each sub-block's 16
+    uint2 hdr, qs[8];
+    __device__ __forceinline__ void load(const unsigned char* row, int b, int lg) {
+        const unsigned char* p = row + (size_t)b * IQ4XS_BYTES;
+        hdr = *reinterpret_cast<const uint2*>(p);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) qs[s] = *reinterpret_cast<const uint2*>(p + 8 + 16 * s + 8 * (lg & 1));
+    }
+};
+
+template <> struct RowBlock<2> {       // d; the 4 code bytes of values 64 s + 16 lg .. + 15
+    uint32_t d, qs[4];
+    __device__ __forceinline__ void load(const unsigned char* row, int b, int lg) {
+        const unsigned char* p = row + (size_t)(b >> 1) * Q2_BYTES;
+        d = *reinterpret_cast<const uint16_t*>(p);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) qs[s] = *reinterpret_cast<const u32_a2*>(p + 2 + 64 * (b & 1) + 16 * s + 4 * lg);
+    }
+};
+
+template <> struct RowBlock<1> {       // d; slots and signs of chunk lg (16 groups)
+    uint32_t d, sign;
+    u32x2_a2 qs;
+    __device__ __forceinline__ void load(const unsigned char* row, int b, int lg) {
+        const unsigned char* p = row + (size_t)b * STQ_BYTES;
+        qs = *reinterpret_cast<const u32x2_a2*>(p + 8 * lg);
+        sign = *reinterpret_cast<const uint16_t*>(p + 32 + 2 * lg);
+        d = *reinterpret_cast<const uint16_t*>(p + 40);
+    }
+};
+
+// Four IQ4_XS grid values (IQ4XS.cs:15-18) of four 4-bit indices, one a byte.
+__device__ __forceinline__ uint32_t iq4_grid(uint32_t idx) {
+    // grid bytes: -127 -104 -83 -65 | -49 -35 -22 -10 | 1 13 25 38 | 53 69 89 113
+    const uint32_t g0 = 0xBFAD9881u, g1 = 0xF6EADDCFu, g2 = 0x26190D01u, g3 = 0x71594535u;
+    const uint32_t sel = idx & 0x07070707u;
+    const uint32_t m = ((idx >> 3) & 0x01010101u) * 0xffu;
+    const uint32_t lo = __builtin_amdgcn_perm(g1, g0, sel), hi = __builtin_amdgcn_perm(g3, g2, sel);
+    return (lo & ~m) | (hi & m);
+}
+
+// The four-lane patterns of STQ1_0 groups 4 i .. + 3 of a chunk, one a byte
+// (see stq_unit_dot in linear_q.hip): h the groups' 4-bit slots, s4 their signs.
+__device__ __forceinline__ uint32_t stq_patterns(uint32_t h, uint32_t s4) {
+    constexpr uint32_t L0 = 0x092989A9u, L1 = 0x062686A6u, L2 = 0x121A929Au, L3 = 0x424A626Au;
+    constexpr uint32_t H0 = 0xA1812101u, H1 = 0xA4842404u, H2 = 0x98901810u, H3 = 0x68604840u;
+    const uint32_t idx = (h & 0xfu) | ((h & 0xf0u) << 4) | ((h & 0xf00u) << 8) | ((h & 0xf000u) << 12);
+    const uint32_t sel = idx & 0x07070707u;
+    const uint32_t hib = ((idx >> 3) & 0x01010101u) * 0xffu;
+    const uint32_t lo = (__builtin_amdgcn_perm(L1, L0, sel) & ~hib) | (__builtin_amdgcn_perm(L3, L2, sel) & hib);
+    const uint32_t hi = (__builtin_amdgcn_perm(H1, H0, sel) & ~hib) | (__builtin_amdgcn_perm(H3, H2, sel) & hib);
+    const uint32_t neg = ((s4 * 0x00204081u) & 0x01010101u) * 0xffu;
+    return (lo & ~neg) | (hi & neg);
+}
+
+// v of the four 16-lane groups, in every lane.
+__device__ __forceinline__ void lane_groups(uint32_t v, uint32_t (&r)[4]) {
+    const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    const auto a = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
+    r[0] = a[0]; r[1] = a[1]; r[2] = b[0]; r[3] = b[1];
+}
+
+// Terms of the fp32 chain a block adds to an output: (a, b) pairs, in order.
+template <int QT> constexpr int kTerms = QT == 14 ? 8 : 1;
+
+// The running values of 16 rows x 16 TT tokens: lane (l16, lg) holds tokens
+// 16 tt + 4 lg + r of weight row l16 (the layout of an MFMA result).  pend: a
+// raw Q2_0C row's first product of a 512-value pair.
+template <int QT, int TT> struct Acc {
+    float v[TT][4], pend[QT == 2 ? TT : 1][4];
+};
+
+// One term of the reference's chain.
+template <int QT, int TT>
+__device__ __forceinline__ void chain(Acc<QT, TT>& acc, int tt, int r, float a, float b, int blk, bool panel) {
+#pragma clang fp contract(off)
+    float& v = acc.v[tt][r];
+    if constexpr (QT == 5 || QT == 14) {
+        v = v + a;
+    } else if (panel) {
+        v = fmaf(a, b, v);
+    } else if constexpr (QT == 1) {
+        v = v + b * a;
+    } else {
+        if (blk & 1) v = v + b * (acc.pend[tt][r] + a);
+        else acc.pend[tt][r] = a;
+    }
+}
+
+// One block of 16 rows x 16 TT tokens: forms its chain terms and hands each to
+// term(s, tt, r, a, b), for every output in ascending s.  X: the block's
+// tokens in LDS, Q8K_WORDS apart.
+template <int QT, int TT, typename F>
+__device__ __forceinline__ void block_terms(const RowBlock<QT>& w, const uint32_t* X, int l16, int lg, bool panel, F&& term) {
+#pragma clang fp contract(off)
+    const uint32_t* xa = X + l16 * Q8K_WORDS;                    // A rows: token 16 tt + l16
+    auto dx = [&](int tt, int r) { return __builtin_bit_cast(float, X[(16 * tt + 4 * lg + r) * Q8K_WORDS]); };
+    const i32x4 zero = {0, 0, 0, 0};
+    if constexpr (QT == 5) {
+        const uint32_t S0 = w.hdr.y, S1 = w.hdr.z, S2 = w.hdr.w;
+        const uint32_t sl = S0 & 0x3f3f3f3fu;                                  // scales 0-3
+        const uint32_t sh = (S2 & 0x0f0f0f0fu) | ((S0 >> 2) & 0x30303030u);    // scales 4-7
+        int isum[TT][4];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) isum[tt][r] = 0;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            auto val = [&](uint32_t q, uint32_t h) {
+                const uint32_t h4 = s < 4 ? h << (4 - s) : h >> (s - 4);       // qh bit s to bit 4
+                return (((s & 1) ? q >> 4 : q) & 0x0f0f0f0fu) | (h4 & 0x10101010u);
+            };
+            const uint32_t b0 = val(w.qs[s >> 1].x, w.qh.x), b1 = val(w.qs[s >> 1].y, w.qh.y);
+            const long bv = (long)(((unsigned long)b1 << 32) | b0);
+            const int sc = (int)(((s < 4 ? sl : sh) >> (8 * (s & 3))) & 0xffu);
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+                const long av = *reinterpret_cast<const long*>(xa + 16 * tt * Q8K_WORDS + Q8K_QS + 8 * s + 2 * lg);
+                const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bv, zero, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    isum[tt][r] += __mul24(d[r], sc);
+                    // one multiply-add each (summed in pairs it takes three operations for two)
+                    asm volatile("" : "+v"(isum[tt][r]));
+                }
+            }
+        }
+        // Min term: j = lg and lg + 4 of this lane's row (B) and token (A);
+        // at most 8 x 63 x 4064, exact in fp32.
+        const float m0 = (float)((S1 >> (8 * lg)) & 63);
+        const float m1 = (float)(((S2 >> (8 * lg + 4)) & 15) | (((S1 >> (8 * lg + 6)) & 3) << 4));
+        const float dw = half_bits_to_float(w.hdr.x & 0xffff), dmw = half_bits_to_float(w.hdr.x >> 16);
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) {
+            const uint32_t* xb = xa + 16 * tt * Q8K_WORDS + Q8K_BS;
+            float pa[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t p = xb[lg + 4 * h];
+                pa[h] = (float)((int)(int16_t)(p & 0xffff) + (int)(int16_t)(p >> 16));
+            }
+            f32x4 md = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[0], m0, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            md = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[1], m1, md, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float yd = dx(tt, r), d = dw * yd, dmin = dmw * yd;
+                term(0, tt, r, d * (float)isum[tt][r] - dmin * md[r], 0.0f);
+            }
+        }
+    } else if constexpr (QT == 14) {
+        const float d = half_bits_to_float(w.hdr.x & 0xffff);
+        const uint32_t sh = 4 * (lg >> 1);                       // low or high nibbles
+        float yd[TT][4];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) yd[tt][r] = dx(tt, r);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const uint32_t b0 = iq4_grid((w.qs[s].x >> sh) & 0x0f0f0f0fu), b1 = iq4_grid((w.qs[s].y >> sh) & 0x0f0f0f0fu);
+            const long bv = (long)(((unsigned long)b1 << 32) | b0);
+            const int ls = (int)(((w.hdr.y >> (8 * (s >> 1) + 4 * (s & 1))) & 0xf) | (((w.hdr.x >> (16 + 2 * s)) & 3) << 4));
+            const float dl = d * (float)(ls - 32);
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+                const long av = *reinterpret_cast<const long*>(xa + 16 * tt * Q8K_WORDS + Q8K_QS + 8 * s + 2 * lg);
+                const i32x4 dot = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bv, zero, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) term(s, tt, r, dl * (float)dot[r] * yd[tt][r], 0.0f);
+            }
+        }
+    } else {
+        i32x4 t[TT];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) t[tt] = zero;
+        uint32_t pat[4][4];            // STQ1_0: [i][chunk]
+        if constexpr (QT == 1)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                lane_groups(stq_patterns((w.qs[i >> 1] >> (16 * (i & 1))) & 0xffffu, (w.sign >> (4 * i)) & 0xfu), pat[i]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            i32x4 bv;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (QT == 1) {
+                    // lane lg of each pattern, less 1
+                    bv[i] = (int)__builtin_amdgcn_perm(0u, 0x020100FFu, (pat[i][s] >> (2 * lg)) & 0x03030303u);
+                } else {
+                    // the byte's four codes spread over four bytes, then 2 code - 3
+                    const uint32_t c = (w.qs[s] >> (8 * i)) & 0xffu, c2 = c | (c << 12);
+                    bv[i] = (int)__builtin_amdgcn_perm(0u, 0x0301FFFDu, (c2 | (c2 << 6)) & 0x03030303u);
+                }
+            }
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+                const i32x4 av = *reinterpret_cast<const i32x4*>(xa + 16 * tt * Q8K_WORDS + Q8K_QS + 16 * s + 4 * lg);
+                t[tt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, t[tt], 0, 0, 0);
+            }
+        }
+        const float dw = half_bits_to_float(w.d);
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float T = (float)t[tt][r], x = dx(tt, r);
+                if (QT == 1 || panel) term(0, tt, r, T, dw * x);
+                else term(0, tt, r, T * x, dw);
+            }
+    }
+}
+
+template <int QT>
+__host__ __device__ constexpr size_t row_bytes(int nb) {
+    return QT == 5 ? (size_t)nb * Q5K_BYTES : QT == 14 ? (size_t)nb * IQ4XS_BYTES : QT == 2 ? (size_t)(nb >> 1) * Q2_BYTES
+                                                                                            : (size_t)nb * STQ_BYTES;
+}
+
+// Blocks of the tokens in one LDS buffer: two buffers are 76 KiB, two
+// workgroups a CU.
+template <int TT> constexpr int kChunk = 8 / TT;
+
+template <int QT, int TT, int NW>
+__global__ __launch_bounds__(64 * NW) void linear_gemm(const unsigned char* __restrict__ w, const uint32_t* __restrict__ q8,
+                                                       float* __restrict__ y, int n_in, int n_rows, int n_out, int tokens,
+                                                       int panel_rows) {
+    constexpr int TOK = 16 * TT, CH = kChunk<TT>, PF = CH < 4 ? CH : 4;
+    constexpr int XW = Q8K_WORDS / 4;                            // 16-byte pieces of a Q8_K block
+    constexpr int RUNS = (TOK * XW + 63) / 64;                   // wave-wide loads of one block's tokens
+    __shared__ uint4 xsh[2][CH][TOK * XW];
+    const int nb = n_in / QK;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row0 = (blockIdx.x * NW + wave) * 16, tok0 = blockIdx.y * TOK;
+    const int row = row0 + l16;
+    const unsigned char* wrow = w + (size_t)min(row, n_rows - 1) * row_bytes<QT>(nb);
+    const bool panel = row < panel_rows;
+
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t*>(q8), 0, (int)((uint32_t)tokens * nb * Q8K_WORDS * 4), 0x00020000);
+    auto stage = [&](int b0, int buf) {
+        for (int u = wave; u < CH * RUNS; u += NW) {
+            const int k = u / RUNS, q = u % RUNS, i = 64 * q + lane, b = b0 + k;
+            const uint32_t vo = (uint32_t)min(tok0 + i / XW, tokens - 1) * nb * Q8K_WORDS * 4 + 16 * (i % XW);
+            if (b < nb && i < TOK * XW) dma_b128(xrs, &xsh[buf][k][64 * q], vo, (uint32_t)b * Q8K_WORDS * 4);
+        }
+    };
+    RowBlock<QT> wq[PF];
+#pragma unroll
+    for (int u = 0; u < PF; ++u) wq[u].load(wrow, min(u, nb - 1), lg);
+    Acc<QT, TT> acc = {};
+
+    stage(0, 0);
+    for (int b0 = 0, buf = 0; b0 < nb; b0 += CH, buf ^= 1) {
+        // This chunk's tokens have landed, and every wave is past the last one.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (b0 + CH < nb) stage(b0 + CH, buf ^ 1);
+#pragma unroll 1
+        for (int k0 = 0; k0 < CH; k0 += PF)
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+                const int k = k0 + u, b = b0 + k;
+                if (b < nb) {
+                    // The next load goes out before the block's work: the chunk's
+                    // closing wait covers it.
+                    const RowBlock<QT> wb = wq[u];
+                    wq[u].load(wrow, min(b + PF, nb - 1), lg);
+                    block_terms<QT, TT>(wb, reinterpret_cast<const uint32_t*>(xsh[buf][k]), l16, lg, panel,
+                                        [&](int, int tt, int r, float a, float f) { chain<QT, TT>(acc, tt, r, a, f, b, panel); });
+                }
+            }
+    }
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = tok0 + 16 * tt + 4 * lg + r;
+            if (row < n_rows && t < tokens) y[(size_t)t * n_out + row] = acc.v[tt][r];
+        }
+}
+
+// The same for few outputs (few tokens, or few rows): a workgroup takes 16 RG
+// rows x 16 TT tokens and its waves split the blocks, KW at a time, wave (rg,
+// kw) forming block p KW + kw's terms.  The chain then passes from wave to
+// wave in block order through LDS, a barrier a step.
+constexpr int kSplitWaves = 10;
+
+template <int QT, int TT, int RG>
+__global__ __launch_bounds__(64 * kSplitWaves) void linear_gemm_split(const unsigned char* __restrict__ w,
+                                                                      const uint32_t* __restrict__ q8, float* __restrict__ y,
+                                                                      int n_in, int n_rows, int n_out, int tokens,
+                                                                      int panel_rows, int KW) {
+    constexpr int TOK = 16 * TT, XW = Q8K_WORDS / 4, XB = TOK * XW, RUNS = (XB + 63) / 64;
+    constexpr int NT = kTerms<QT>, NV = QT == 2 ? 2 : 1;
+    extern __shared__ uint4 split_smem[];                        // two buffers of KW blocks' tokens, then the chain
+    const int nb = n_in / QK, passes = (nb + KW - 1) / KW;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kw = wave % KW, rg = wave / KW;
+    const int row = (blockIdx.x * RG + rg) * 16 + l16, tok0 = blockIdx.y * TOK;
+    const unsigned char* wrow = w + (size_t)min(row, n_rows - 1) * row_bytes<QT>(nb);
+    const bool panel = row < panel_rows;
+    float4* relay = reinterpret_cast<float4*>(split_smem + (passes > 1 ? 2 : 1) * KW * XB) + rg * NV * TT * 64 + lane;
+
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint32_t*>(q8), 0, (int)((uint32_t)tokens * nb * Q8K_WORDS * 4), 0x00020000);
+    // A row group's share of block b's tokens (past the last token: not loaded, not stored).
+    const int nchunk = min(tokens - tok0, TOK) * XW;
+    auto stage = [&](int b, int buf) {
+        if (b >= nb) return;
+#pragma unroll
+        for (int q0 = 0; q0 < RUNS; q0 += RG) {
+            const int q = q0 + rg, i = 64 * q + lane;
+            if (i < nchunk)
+                dma_b128(xrs, split_smem + (buf * KW + kw) * XB + 64 * q,
+                         (uint32_t)(tok0 + i / XW) * nb * Q8K_WORDS * 4 + 16 * (i % XW), (uint32_t)b * Q8K_WORDS * 4);
+        }
+    };
+    RowBlock<QT> wn;
+    wn.load(wrow, min(kw, nb - 1), lg);
+    stage(kw, 0);
+    Acc<QT, TT> acc = {};
+    for (int p = 0; p < passes; ++p) {
+        const int b = p * KW + kw;
+        // This pass's tokens have landed, and every wave is past the last one's.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        const RowBlock<QT> wb = wn;
+        if (p + 1 < passes) {
+            stage(b + KW, (p + 1) & 1);
+            wn.load(wrow, min(b + KW, nb - 1), lg);
+        }
+        float ta[NT][TT][4], tb[NT][TT][4];
+        if (b < nb)
+            block_terms<QT, TT>(wb, reinterpret_cast<const uint32_t*>(split_smem + ((p & 1) * KW + kw) * XB), l16, lg, panel,
+                                [&](int s, int tt, int r, float a, float f) { ta[s][tt][r] = a; tb[s][tt][r] = f; });
+        const int steps = min(KW, nb - p * KW);
+        for (int k = 0; k < steps; ++k) {
+            if (kw == k) {
+                if (b > 0)
+#pragma unroll
+                    for (int tt = 0; tt < TT; ++tt) {
+                        *reinterpret_cast<float4*>(acc.v[tt]) = relay[64 * tt];
+                        if constexpr (QT == 2) *reinterpret_cast<float4*>(acc.pend[tt]) = relay[64 * (TT + tt)];
+                    }
+#pragma unroll
+                for (int s = 0; s < NT; ++s)
+#pragma unroll
+                    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) chain<QT, TT>(acc, tt, r, ta[s][tt][r], tb[s][tt][r], b, panel);
+                if (b + 1 < nb) {
+#pragma unroll
+                    for (int tt = 0; tt < TT; ++tt) {
+                        relay[64 * tt] = *reinterpret_cast<const float4*>(acc.v[tt]);
+                        if constexpr (QT == 2) relay[64 * (TT + tt)] = *reinterpret_cast<const float4*>(acc.pend[tt]);
+                    }
+                } else {
+#pragma unroll
+                    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int t = tok0 + 16 * tt + 4 * lg + r;
+                            if (row < n_rows && t < tokens) y[(size_t)t * n_out + row] = acc.v[tt][r];
+                        }
+                }
+            }
+            if (k + 1 < steps) lds_barrier();
+        }
+    }
+}
+
+template <int QT>
+hipError_t go(q35m_ctx* c, int kid, const unsigned char* w, const uint32_t* q8, float* y, int n_in, int n_out, int tokens,
+              int panel_rows) {
+    const int nb = n_in / QK;
+    auto pieces = [&](int tok, auto one) {
+        // The tokens are addressed through a buffer descriptor: at most 2 GiB a launch.
+        const size_t lim = (c->tile_limit - 1) / ((size_t)nb * Q8K_WORDS * 4) / tok * tok;
+        const int tmax = (int)std::min<size_t>(tokens, std::max<size_t>(lim, tok));
+        for (int t0 = 0; t0 < tokens; t0 += tmax) {
+            const int nt = std::min(tmax, tokens - t0);
+            ProfScope ps_(c, kid);
+            one(ps_, q8 + (size_t)t0 * nb * Q8K_WORDS, y + (size_t)t0 * n_out, nt);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    };
+    auto whole = [&](auto kern, int tok, int nw) {
+        return pieces(tok, [&](ProfScope& ps, const uint32_t* qt, float* yt, int nt) {
+            hipExtLaunchKernelGGL(kern, dim3((n_out + 16 * nw - 1) / (16 * nw), (nt + tok - 1) / tok), dim3(64 * nw), 0,
+                                  c->stream, ps.a, ps.b, 0, w, qt, yt, n_in, n_out, n_out, nt, panel_rows);
+        });
+    };
+    auto split = [&](auto kern, int tt, int rg) {
+        const int wmax = kSplitWaves / rg, passes = (nb + wmax - 1) / wmax, kw = (nb + passes - 1) / passes;
+        const size_t lds = ((passes > 1 ? 2 : 1) * (size_t)kw * tt * 16 * Q8K_WORDS / 4 + (size_t)rg * (QT == 2 ? 2 : 1) * tt * 64) * 16;
+        return pieces(16 * tt, [&](ProfScope& ps, const uint32_t* qt, float* yt, int nt) {
+            hipExtLaunchKernelGGL(kern, dim3((n_out + 16 * rg - 1) / (16 * rg), (nt + 16 * tt - 1) / (16 * tt)),
+                                  dim3(64 * kw * rg), lds, c->stream, ps.a, ps.b, 0, w, qt, yt, n_in, n_out, n_out, nt,
+                                  panel_rows, kw);
+        });
+    };
+    // By the 16 x 16 tiles of the result.  Few: every tile its own workgroup,
+    // the blocks split over its waves; then pairs of them; then waves that
+    // run whole rows of blocks, of 32 and of 64 tokens (least decode a token,
+    // but a serial 3 us a block where the waves are few).  Measured (us, in
+    // that order; 2560 -> 8192 unless said): Q5_K 16 tokens (512 tiles) 7.9 /
+    // 9.9 / 19 / 32, 32 (1024) 16 / 10.4 / 19 / 32, 64 (2048) 27 / 17.3 / 22 /
+    // 33, 128 (4096) 48 / 33 / 22 / 33, 500 177 / 127 / 61 / 48, 2048 tokens -
+    // / 500 / 218 / 170; 4096 -> 2560 at 64 tokens (640) 14.9 / 14.7 / 30 /
+    // 51, at 200 (2080) 36 / 29 / 32 / 51; IQ4_XS at 200 (6656) - / 67 / 46 /
+    // 35; Q2_0C at 200 - / 57 / 26 / 19.  One thread a block and a serial
+    // chain a row for 8 tokens at a time took 7.1 at 2 tokens, 17.6 at 16, 310
+    // at 500, 1246 at 2048 (IQ4_XS 373, Q2_0C 422, STQ1_0 770 at 500).
+    const long tiles = (long)((n_out + 15) / 16) * ((tokens + 15) / 16);
+    if (tiles <= 640) return split(linear_gemm_split<QT, 1, 1>, 1, 1);
+    if (tiles <= 2304) return split(linear_gemm_split<QT, 2, 2>, 2, 2);
+    if (tiles <= 4608) return whole(linear_gemm<QT, 2, 8>, 32, 8);
+    return whole(linear_gemm<QT, 4, 8>, 64, 8);
+}
+
+}  // namespace
+
+hipError_t launch_linear_gemm(q35m_ctx* c, int qtype, const void* w, const void* q8, float* y, int n_in, int n_out,
+                              int tokens, int panel_rows) {
+    const unsigned char* wb = reinterpret_cast<const unsigned char*>(w);
+    const uint32_t* qb = reinterpret_cast<const uint32_t*>(q8);
+    switch (qtype) {
+        case 5: return go<5>(c, K_Q5K_GEMM, wb, qb, y, n_in, n_out, tokens, 0);
+        case 14: return go<14>(c, K_IQ4XS_GEMM, wb, qb, y, n_in, n_out, tokens, 0);
+        case 2: return go<2>(c, K_Q2_0C_GEMM, wb, qb, y, n_in, n_out, tokens, panel_rows);
+        default: return go<1>(c, K_STQ1_0_GEMM, wb, qb, y, n_in, n_out, tokens, panel_rows);
+    }
+}
+
+}  // namespace q35

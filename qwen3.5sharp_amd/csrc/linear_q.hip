@@ -33,23 +33,14 @@
 // tokens reuse the staged weights.
 #include "common.h"
 #include "q35mix_internal.h"
+#include "quant_layout.h"
 
 namespace q35 {
 namespace {
 
-constexpr int QK = 256;
-constexpr int Q4K_BYTES = 144, Q6K_BYTES = 210;
-// Workspace form of a Q8_K block, 304 bytes (19 x 16): dword 0 d, dwords 4..67
-// qs (16-byte aligned), dwords 68..75 bsums; dwords 1..3 unused.
-constexpr int Q8K_WORDS = 76;
-constexpr int Q8K_QS = 4, Q8K_BS = 68;
 constexpr int LQ_THREADS = 64;
 constexpr int LQ_MAX_ROWS = 8;     // rows per workgroup (8 threads a row in the fp32 pass)
 constexpr int LANES_LD = 13;       // padded stride of the per-block integer lanes in LDS
-
-__device__ __forceinline__ float half_bits_to_float(uint32_t h) {
-    return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(h)));
-}
 
 // The Q8_K block of 256 values held 16 a lane by a 16-lane group (lane li of
 // the group: values 16 li .. 16 li + 15, one bsums group); every lane of the
@@ -383,11 +374,10 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_q(const unsigned char* __re
 // Kernels/Q5K.cs:45-95; IQ4XS.Dot, IQ4XS.cs:49-73): exact integer sums per
 // block (Q5_K) or per 32-value sub-block (IQ4_XS), then one fp32 chain per
 // output in block order with no fused multiply-add.  Their Gemm runs the GEMV
-// per token (Q5K.cs:112-117, IQ4XS.cs:99-104), so every token is a GEMV here
-// too.  Block formats (BlockLayout.cs:49-66):
+// per token (Q5K.cs:112-117, IQ4XS.cs:99-104): several tokens keep the same
+// arithmetic (linear_gemm.hip).  Block formats (BlockLayout.cs:49-66):
 //   Q5_K (176 B): f16 d, f16 dmin, u8 scales[12], u8 qh[32], u8 qs[128]
 //   IQ4_XS (136 B): f16 d, u16 scales_h, u8 scales_l[4], u8 qs[128]
-constexpr int Q5K_BYTES = 176, IQ4XS_BYTES = 136;
 constexpr int QS_TLD = 9;            // LDS stride of a block's chain terms
 
 // Q5_K x Q8_K block: acc = sum_j scale_j (q8 . a over sub-block j) with the
@@ -467,16 +457,14 @@ __device__ __forceinline__ void iq4xs_block_terms(const uint32_t* __restrict__ w
     }
 }
 
-// One 64-thread workgroup per group of up to 8 whole rows (at most 64
-// blocks, a block a thread, held in registers) and `tok_per_wg` tokens.  Per
-// token: the token's Q8_K row is staged in LDS, every thread forms its
-// block's integer terms, and one thread per row runs the reference's fp32
-// chain over the row's blocks in order.
+// One token: one 64-thread workgroup per group of up to 8 whole rows (at most
+// 64 blocks, a block a thread, held in registers).  The token's Q8_K row is
+// staged in LDS, every thread forms its block's integer terms, and one thread
+// per row runs the reference's fp32 chain over the row's blocks in order.
 template <int QT>
 __global__ __launch_bounds__(LQ_THREADS) void linear_qs(const unsigned char* __restrict__ w,
                                                         const uint32_t* __restrict__ q8,
-                                                        float* __restrict__ y, int n_in, int n_out,
-                                                        int tokens, int rows_per_wg, int tok_per_wg) {
+                                                        float* __restrict__ y, int n_in, int n_out, int rows_per_wg) {
 #pragma clang fp contract(off)
     constexpr int BB = QT == 5 ? Q5K_BYTES : IQ4XS_BYTES;
     extern __shared__ uint4 smem[];
@@ -484,7 +472,6 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qs(const unsigned char* __r
     const int row0 = blockIdx.x * rows_per_wg;
     const int nrows = min(rows_per_wg, n_out - row0);
     const int nblk = nrows * nb;
-    const int t_begin = blockIdx.y * tok_per_wg, t_end = min(tokens, t_begin + tok_per_wg);
     uint32_t* q8s = reinterpret_cast<uint32_t*>(smem);
     float* terms = reinterpret_cast<float*>(q8s + nb * Q8K_WORDS);
 
@@ -501,62 +488,59 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qs(const unsigned char* __r
             for (int c = 0; c < BB / 8; ++c) reinterpret_cast<uint2*>(wb)[c] = reinterpret_cast<const uint2*>(src)[c];
         }
     }
-    for (int t = t_begin; t < t_end; ++t) {
-        {
-            const uint4* src = reinterpret_cast<const uint4*>(q8 + (size_t)t * nb * Q8K_WORDS);
-            uint4* dst = reinterpret_cast<uint4*>(q8s);
-            const int n4 = nb * (Q8K_WORDS / 4);
-            for (int i0 = 0; i0 < n4; i0 += 8 * LQ_THREADS) {
-                uint4 qv[8];
+    {
+        const uint4* src = reinterpret_cast<const uint4*>(q8);
+        uint4* dst = reinterpret_cast<uint4*>(q8s);
+        const int n4 = nb * (Q8K_WORDS / 4);
+        for (int i0 = 0; i0 < n4; i0 += 8 * LQ_THREADS) {
+            uint4 qv[8];
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    qv[c] = make_uint4(0u, 0u, 0u, 0u);
-                    if (i0 + lane + LQ_THREADS * c < n4) qv[c] = src[i0 + lane + LQ_THREADS * c];
-                }
+            for (int c = 0; c < 8; ++c) {
+                qv[c] = make_uint4(0u, 0u, 0u, 0u);
+                if (i0 + lane + LQ_THREADS * c < n4) qv[c] = src[i0 + lane + LQ_THREADS * c];
+            }
 #pragma unroll
-                for (int c = 0; c < 8; ++c)
-                    if (i0 + lane + LQ_THREADS * c < n4) dst[i0 + lane + LQ_THREADS * c] = qv[c];
+            for (int c = 0; c < 8; ++c)
+                if (i0 + lane + LQ_THREADS * c < n4) dst[i0 + lane + LQ_THREADS * c] = qv[c];
+        }
+    }
+    __syncthreads();
+    // Each thread forms its block's terms of the reference's chain (they do
+    // not depend on the running sum); one thread per row then adds them in
+    // order.
+    if (lane < nblk) {
+        const uint32_t* q8b = q8s + (lane % nb) * Q8K_WORDS;
+        const float yd = __builtin_bit_cast(float, q8b[0]);
+        float* out = terms + lane * QS_TLD;
+        if constexpr (QT == 5) {
+            int acc, sumi;
+            q5k_block_terms(wb, q8b, acc, sumi);
+            const float d = half_bits_to_float(wb[0] & 0xffff) * yd;
+            const float dmin = half_bits_to_float(wb[0] >> 16) * yd;
+            out[0] = d * (float)acc - dmin * (float)sumi;
+        } else {
+            int acc[8];
+            iq4xs_block_terms(wb, q8b, acc);
+            const uint32_t hdr = wb[0], sl = wb[1];
+            const float d = half_bits_to_float(hdr & 0xffff);
+#pragma unroll
+            for (int ib = 0; ib < 8; ++ib) {
+                const int ls = (int)(((sl >> (8 * (ib >> 1) + 4 * (ib & 1))) & 0xf) |
+                                     (((hdr >> (16 + 2 * ib)) & 3) << 4));
+                const float dl = d * (float)(ls - 32);
+                out[ib] = dl * (float)acc[ib] * yd;
             }
         }
-        __syncthreads();
-        // Each thread forms its block's terms of the reference's chain (they do
-        // not depend on the running sum); one thread per row then adds them in
-        // order.
-        if (lane < nblk) {
-            const uint32_t* q8b = q8s + (lane % nb) * Q8K_WORDS;
-            const float yd = __builtin_bit_cast(float, q8b[0]);
-            float* out = terms + lane * QS_TLD;
-            if constexpr (QT == 5) {
-                int acc, sumi;
-                q5k_block_terms(wb, q8b, acc, sumi);
-                const float d = half_bits_to_float(wb[0] & 0xffff) * yd;
-                const float dmin = half_bits_to_float(wb[0] >> 16) * yd;
-                out[0] = d * (float)acc - dmin * (float)sumi;
-            } else {
-                int acc[8];
-                iq4xs_block_terms(wb, q8b, acc);
-                const uint32_t hdr = wb[0], sl = wb[1];
-                const float d = half_bits_to_float(hdr & 0xffff);
+    }
+    __syncthreads();
+    if (lane < nrows) {
+        constexpr int NTERM = QT == 5 ? 1 : 8;
+        float sumf = 0.0f;
+        const float* T = terms + lane * nb * QS_TLD;
+        for (int b = 0; b < nb; ++b)
 #pragma unroll
-                for (int ib = 0; ib < 8; ++ib) {
-                    const int ls = (int)(((sl >> (8 * (ib >> 1) + 4 * (ib & 1))) & 0xf) |
-                                         (((hdr >> (16 + 2 * ib)) & 3) << 4));
-                    const float dl = d * (float)(ls - 32);
-                    out[ib] = dl * (float)acc[ib] * yd;
-                }
-            }
-        }
-        __syncthreads();
-        if (lane < nrows) {
-            constexpr int NTERM = QT == 5 ? 1 : 8;
-            float sumf = 0.0f;
-            const float* T = terms + lane * nb * QS_TLD;
-            for (int b = 0; b < nb; ++b)
-#pragma unroll
-                for (int k = 0; k < NTERM; ++k) sumf += T[b * QS_TLD + k];
-            y[(size_t)t * n_out + row0 + lane] = sumf;
-        }
-        __syncthreads();
+            for (int k = 0; k < NTERM; ++k) sumf += T[b * QS_TLD + k];
+        y[row0 + lane] = sumf;
     }
 }
 
@@ -578,7 +562,6 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qs(const unsigned char* __r
 // other rows, Q2_0C.DotAvx2 (Q2_0C.cs:67-79): acc += dw * ((float)T0 * dx0
 // + (float)T1 * dx1) per 512 values, and STQ1_0.DotAvx2 (STQ1_0.cs:120-138):
 // acc += (dw * dx) * (float)T.  Rows below panel_rows take the panel order.
-constexpr int Q2_BYTES = 130, STQ_BYTES = 42;
 
 // Bytes k of the four dwords q[0..3] gathered into dword k (a 4 x 4 byte
 // transpose): Q2_0C's byte c of a qs dword holds values 4c .. 4c + 3, so its
@@ -656,16 +639,15 @@ __device__ __forceinline__ int stq_unit_dot(const uint32_t* __restrict__ base, i
     return enc - q8k_bsum_total(q8b);
 }
 
-// One 64-thread workgroup per group of up to 8 whole rows (at most 64 units,
-// one a thread) and tok_per_wg tokens: the rows' contiguous weight bytes are
-// staged in LDS once (as for Q6_K), then per token the Q8_K row is staged,
-// every thread forms its unit's T, and one thread per row runs the chain.
+// One token: one 64-thread workgroup per group of up to 8 whole rows (at most
+// 64 units, one a thread): the rows' contiguous weight bytes are staged in LDS
+// (as for Q6_K) and the token's Q8_K row, every thread forms its unit's T, and
+// one thread per row runs the chain.
 template <int QT>
 __global__ __launch_bounds__(LQ_THREADS) void linear_qt(const unsigned char* __restrict__ w,
                                                         const uint32_t* __restrict__ q8,
                                                         float* __restrict__ y, int n_in, int n_out,
-                                                        int tokens, int rows_per_wg, int tok_per_wg,
-                                                        int panel_rows) {
+                                                        int rows_per_wg, int panel_rows) {
 #pragma clang fp contract(off)
     constexpr int UB = QT == 2 ? Q2_BYTES / 2 : STQ_BYTES;   // weight bytes per unit
     extern __shared__ uint4 smem[];
@@ -673,7 +655,6 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qt(const unsigned char* __r
     const int row0 = blockIdx.x * rows_per_wg;
     const int nrows = min(rows_per_wg, n_out - row0);
     const int nunit = nrows * nb;
-    const int t_begin = blockIdx.y * tok_per_wg, t_end = min(tokens, t_begin + tok_per_wg);
     const size_t row_bytes = (size_t)nb * UB;
     const int nchunk_max = (rows_per_wg * nb * UB + 31) / 16 + 1;
     uint4* wsh = smem;
@@ -715,67 +696,64 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qt(const unsigned char* __r
         }
     }
 
-    for (int t = t_begin; t < t_end; ++t) {
-        {
-            const uint4* src = reinterpret_cast<const uint4*>(q8 + (size_t)t * nb * Q8K_WORDS);
-            uint4* dst = reinterpret_cast<uint4*>(q8s);
-            const int n4 = nb * (Q8K_WORDS / 4);
-            for (int i0 = 0; i0 < n4; i0 += 8 * LQ_THREADS) {
-                uint4 qv[8];
+    {
+        const uint4* src = reinterpret_cast<const uint4*>(q8);
+        uint4* dst = reinterpret_cast<uint4*>(q8s);
+        const int n4 = nb * (Q8K_WORDS / 4);
+        for (int i0 = 0; i0 < n4; i0 += 8 * LQ_THREADS) {
+            uint4 qv[8];
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    qv[c] = make_uint4(0u, 0u, 0u, 0u);
-                    if (i0 + lane + LQ_THREADS * c < n4) qv[c] = src[i0 + lane + LQ_THREADS * c];
-                }
+            for (int c = 0; c < 8; ++c) {
+                qv[c] = make_uint4(0u, 0u, 0u, 0u);
+                if (i0 + lane + LQ_THREADS * c < n4) qv[c] = src[i0 + lane + LQ_THREADS * c];
+            }
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    const int i = i0 + lane + LQ_THREADS * c;
-                    if (i < n4) {
-                        const int part = i % (Q8K_WORDS / 4);     // 1..16: qs, 0 and 17..18: d, bsums
-                        dst[i] = (QT == 2 && part >= 1 && part <= 16) ? byte_transpose(qv[c]) : qv[c];
-                    }
+            for (int c = 0; c < 8; ++c) {
+                const int i = i0 + lane + LQ_THREADS * c;
+                if (i < n4) {
+                    const int part = i % (Q8K_WORDS / 4);     // 1..16: qs, 0 and 17..18: d, bsums
+                    dst[i] = (QT == 2 && part >= 1 && part <= 16) ? byte_transpose(qv[c]) : qv[c];
                 }
             }
         }
-        __syncthreads();
-        if (lane < nunit) {
-            const int r = lane / nb, b = lane % nb;
-            const uint32_t* q8b = q8s + b * Q8K_WORDS;
-            if constexpr (QT == 2)
-                tv[lane] = q2_unit_dot(wbase, shift + (int)(r * row_bytes) + (b >> 1) * Q2_BYTES + 2 + 64 * (b & 1), q8b);
-            else
-                tv[lane] = stq_unit_dot(wbase, shift + (int)(r * row_bytes) + b * STQ_BYTES, q8b);
-        }
-        __syncthreads();
-        if (lane < nrows) {
-            const int row = row0 + lane;
-            const int* T = tv + lane * nb;
-            const int o = shift + (int)(lane * row_bytes);
-            float acc = 0.0f;
-            if (row < panel_rows) {
-                for (int b = 0; b < nb; ++b) {
-                    const int dof = QT == 2 ? o + (b >> 1) * Q2_BYTES : o + b * STQ_BYTES + 40;
-                    const float dw = half_bits_to_float(lds_word(wbase, dof) & 0xffff);
-                    const float dx = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
-                    acc = fmaf((float)T[b], dw * dx, acc);
-                }
-            } else if constexpr (QT == 2) {
-                for (int b = 0; b < nb; b += 2) {
-                    const float dw = half_bits_to_float(lds_word(wbase, o + (b >> 1) * Q2_BYTES) & 0xffff);
-                    const float dx0 = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
-                    const float dx1 = __builtin_bit_cast(float, q8s[(b + 1) * Q8K_WORDS]);
-                    acc = acc + dw * ((float)T[b] * dx0 + (float)T[b + 1] * dx1);
-                }
-            } else {
-                for (int b = 0; b < nb; ++b) {
-                    const float dw = half_bits_to_float(lds_word(wbase, o + b * STQ_BYTES + 40) & 0xffff);
-                    const float dx = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
-                    acc = acc + (dw * dx) * (float)T[b];
-                }
+    }
+    __syncthreads();
+    if (lane < nunit) {
+        const int r = lane / nb, b = lane % nb;
+        const uint32_t* q8b = q8s + b * Q8K_WORDS;
+        if constexpr (QT == 2)
+            tv[lane] = q2_unit_dot(wbase, shift + (int)(r * row_bytes) + (b >> 1) * Q2_BYTES + 2 + 64 * (b & 1), q8b);
+        else
+            tv[lane] = stq_unit_dot(wbase, shift + (int)(r * row_bytes) + b * STQ_BYTES, q8b);
+    }
+    __syncthreads();
+    if (lane < nrows) {
+        const int row = row0 + lane;
+        const int* T = tv + lane * nb;
+        const int o = shift + (int)(lane * row_bytes);
+        float acc = 0.0f;
+        if (row < panel_rows) {
+            for (int b = 0; b < nb; ++b) {
+                const int dof = QT == 2 ? o + (b >> 1) * Q2_BYTES : o + b * STQ_BYTES + 40;
+                const float dw = half_bits_to_float(lds_word(wbase, dof) & 0xffff);
+                const float dx = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
+                acc = fmaf((float)T[b], dw * dx, acc);
             }
-            y[(size_t)t * n_out + row] = acc;
+        } else if constexpr (QT == 2) {
+            for (int b = 0; b < nb; b += 2) {
+                const float dw = half_bits_to_float(lds_word(wbase, o + (b >> 1) * Q2_BYTES) & 0xffff);
+                const float dx0 = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
+                const float dx1 = __builtin_bit_cast(float, q8s[(b + 1) * Q8K_WORDS]);
+                acc = acc + dw * ((float)T[b] * dx0 + (float)T[b + 1] * dx1);
+            }
+        } else {
+            for (int b = 0; b < nb; ++b) {
+                const float dw = half_bits_to_float(lds_word(wbase, o + b * STQ_BYTES + 40) & 0xffff);
+                const float dx = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
+                acc = acc + (dw * dx) * (float)T[b];
+            }
         }
-        __syncthreads();
+        y[row] = acc;
     }
 }
 
@@ -920,9 +898,6 @@ constexpr int GWAVES = GTHREADS / 64;
 constexpr int GRUNS = (GX_CHUNKS + 64 * GWAVES - 1) / (64 * GWAVES);   // wave-wide loads a wave: 3
 constexpr int kMagic = 0x4B400000;                      // bits of 1.5 * 2^23
 constexpr float kMagicF = 12582912.0f;
-
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(GTHREADS) __attribute__((amdgpu_waves_per_eu(2)))
 void q4k_gemm(const unsigned char* __restrict__ w, const uint32_t* __restrict__ q8,
@@ -1621,35 +1596,33 @@ hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const
         // else none.
         int panel_rows = n_out & ~7;
         if (qtype == 1 && tokens > 1) panel_rows = ((tokens & 3) == 0 && (n_out & 7) == 0) ? n_out : 0;
+        if (tokens >= 2) return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, tokens, panel_rows);
         const int rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
-        const int tok_per_wg = 8;
         const int ub = qtype == 2 ? Q2_BYTES / 2 : STQ_BYTES;
         const int nchunk_max = (rows_per_wg * nb * ub + 31) / 16 + 1;
-        const dim3 grid((n_out + rows_per_wg - 1) / rows_per_wg, (tokens + tok_per_wg - 1) / tok_per_wg);
+        const dim3 grid((n_out + rows_per_wg - 1) / rows_per_wg);
         const size_t lds = 16 * (size_t)nchunk_max + (size_t)nb * Q8K_WORDS * 4 + (size_t)LQ_THREADS * 4;
         ProfScope ps_(c, qtype == 2 ? K_Q2_0C_LINEAR : K_STQ1_0_LINEAR);
         if (qtype == 2)
             hipExtLaunchKernelGGL(linear_qt<2>, grid, dim3(LQ_THREADS), lds, c->stream, ps_.a, ps_.b, 0, wb, qb, y,
-                                  n_in, n_out, tokens, rows_per_wg, tok_per_wg, panel_rows);
+                                  n_in, n_out, rows_per_wg, panel_rows);
         else
             hipExtLaunchKernelGGL(linear_qt<1>, grid, dim3(LQ_THREADS), lds, c->stream, ps_.a, ps_.b, 0, wb, qb, y,
-                                  n_in, n_out, tokens, rows_per_wg, tok_per_wg, panel_rows);
+                                  n_in, n_out, rows_per_wg, panel_rows);
         return hipGetLastError();
     }
     if (qtype == 5 || qtype == 14) {
-        // Per-token GEMV; up to 8 tokens a workgroup (the weights stay in
-        // registers across them), more tokens over the grid's second axis.
+        if (tokens >= 2) return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, tokens, 0);
         const int rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
-        const int tok_per_wg = 8;
-        const dim3 grid((n_out + rows_per_wg - 1) / rows_per_wg, (tokens + tok_per_wg - 1) / tok_per_wg);
+        const dim3 grid((n_out + rows_per_wg - 1) / rows_per_wg);
         const size_t lds = (size_t)nb * Q8K_WORDS * 4 + (size_t)LQ_THREADS * QS_TLD * 4;
         ProfScope ps_(c, qtype == 5 ? K_Q5K_LINEAR : K_IQ4XS_LINEAR);
         if (qtype == 5)
             hipExtLaunchKernelGGL(linear_qs<5>, grid, dim3(LQ_THREADS), lds, c->stream, ps_.a, ps_.b, 0, wb, qb, y,
-                                  n_in, n_out, tokens, rows_per_wg, tok_per_wg);
+                                  n_in, n_out, rows_per_wg);
         else
             hipExtLaunchKernelGGL(linear_qs<14>, grid, dim3(LQ_THREADS), lds, c->stream, ps_.a, ps_.b, 0, wb, qb, y,
-                                  n_in, n_out, tokens, rows_per_wg, tok_per_wg);
+                                  n_in, n_out, rows_per_wg);
         return hipGetLastError();
     }
     // The tiled kernels address their operands through buffer descriptors

@@ -91,6 +91,10 @@ enum KernelId {
     K_ATTN_DECODE_PARTIAL4R16,   // attn_decode_partial, 4 sub-chunks of 16 rows per workgroup
     K_ATTN_DECODE_PARTIAL8R16,   // attn_decode_partial, up to 8 sub-chunks of 16 rows per workgroup
     K_Q6K_GEMM_BLK,              // block-order Q6_K projection (q35m_set_projection_order)
+    K_Q5K_GEMM,                  // linear_gemm and linear_gemm_split of the format
+    K_IQ4XS_GEMM,
+    K_Q2_0C_GEMM,
+    K_STQ1_0_GEMM,
     K_COUNT
 };
 const char* kernel_name(int id);
@@ -196,6 +200,10 @@ hipError_t launch_attn_prefill(q35m_ctx* c, int layer, int seq, int start, int T
 size_t attn_prefill_work_bytes(const Dims& d, int T);
 hipError_t launch_linear_q(q35m_ctx* c, int qtype, const void* w, const float* x, float* y,
                            int n_in, int n_out, int tokens);
+// Q5_K, IQ4_XS, Q2_0C and STQ1_0 projections of several tokens on the matrix
+// cores; rows below panel_rows take the eight-row panel order (Q2_0C, STQ1_0).
+hipError_t launch_linear_gemm(q35m_ctx* c, int qtype, const void* w, const void* q8, float* y, int n_in, int n_out,
+                              int tokens, int panel_rows);
 hipError_t launch_add_rmsnorm(q35m_ctx* c, float* hidden, const float* delta, const float* w, float* y, void* q8,
                               int dim, int tokens, float eps);
 size_t linear_q_work_bytes(int n_in, int tokens);

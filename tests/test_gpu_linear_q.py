@@ -73,6 +73,20 @@ def test_linear_q_bit_exact(ctx, qtype, n_in, n_out, tokens):
     assert bad.size == 0
 
 
+@pytest.mark.parametrize("qtype", [1, 2, 5, 14])
+@pytest.mark.parametrize("n_in,n_out,tokens", [(512, 15, 2), (2560, 63, 16), (4608, 65, 17), (1024, 130, 32),
+                                               (3584, 17, 33), (512, 257, 64), (5120, 34, 65), (1536, 129, 191)])
+def test_linear_gemm_tiles(ctx, qtype, n_in, n_out, tokens):
+    """The matrix-core tiles of Q5_K, IQ4_XS, Q2_0C and STQ1_0 at the edges of
+    their rows (16 a wave), tokens (16, 32, 64) and block pipelines, bit for
+    bit (STQ1_0: panel and raw row orders by the token count)."""
+    rng = np.random.default_rng(31 * qtype + n_in + n_out + tokens)
+    w = qb.random_blocks(rng, qtype, qb.nblocks(qtype, n_out * n_in))
+    x = rng.standard_normal((tokens, n_in)).astype(np.float32)
+    got = run(ctx, qtype, w, x, n_in, n_out)
+    assert np.array_equal(got.view(np.uint32), oracle.linear_q(qtype, w, x, n_in, n_out).view(np.uint32))
+
+
 @pytest.mark.parametrize("qtype", TYPES)
 def test_linear_q_activation_edges(ctx, qtype):
     """Zero blocks (scale 0), a first extremum that is positive (negative
