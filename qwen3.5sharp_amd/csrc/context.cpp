@@ -200,7 +200,8 @@ const char* kernel_name(int id) {
         "q8k_quantize",           "linear_q<4>",             "linear_q<6>",
         "q4k_gemm", "q6k_gemm", "add_rmsnorm", "linear_qs<5>", "linear_qs<14>", "linear_f32", "linear_qt<2>",
         "linear_qt<1>", "attn_decode_partial<4,16>", "attn_decode_partial<8,16>", "q6k_gemm_blk",
-        "linear_gemm<5>", "linear_gemm<14>", "linear_gemm<2>", "linear_gemm<1>"};
+        "linear_gemm<5>", "linear_gemm<14>", "linear_gemm<2>", "linear_gemm<1>",
+        "attn_split_prep", "attn_split_flash", "attn_split_merge"};
     return (id >= 0 && id < K_COUNT) ? names[id] : nullptr;
 }
 
@@ -601,8 +602,11 @@ int q35m_attn_prefill(q35m_ctx* ctx, int layer, int seq, int T, const float* q_g
     if ((long)start + T > q35::kPrefillMaxRows)
         return fail(Q35M_ERR_UNSUPPORTED, "attention prefill reads at most %d cached rows (sequence %d "
                     "would reach %d)", q35::kPrefillMaxRows, seq, start + T);
-    HIP_TRY(q35::ensure_work(ctx, q35::attn_prefill_work_bytes(ctx->d, T)), "workspace");
-    HIP_TRY(q35::launch_attn_prefill(ctx, layer, seq, start, T, q_gate, k, v, out), "attn_prefill");
+    // Without room for the split form's workspace the call takes the fp32 form.
+    const size_t split = q35::attn_prefill_split_bytes(ctx, start, T);
+    const bool ok = split && q35::ensure_work(ctx, split) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    HIP_TRY(q35::launch_attn_prefill(ctx, layer, seq, start, T, q_gate, k, v, out, ok), "attn_prefill");
     return Q35M_OK;
 }
 

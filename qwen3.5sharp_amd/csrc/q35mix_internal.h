@@ -95,6 +95,9 @@ enum KernelId {
     K_IQ4XS_GEMM,
     K_Q2_0C_GEMM,
     K_STQ1_0_GEMM,
+    K_ATTN_SPLIT_PREP,
+    K_ATTN_SPLIT_FLASH,
+    K_ATTN_SPLIT_MERGE,
     K_COUNT
 };
 const char* kernel_name(int id);
@@ -196,8 +199,10 @@ constexpr size_t kNoAllocScratchBytes = Q35M_NOALLOC_SCRATCH_BYTES;
 // current; each device has its own copy).
 hipError_t attn_decode_scratch_address(float** ptr);
 hipError_t launch_attn_prefill(q35m_ctx* c, int layer, int seq, int start, int T,
-                               const float* q_gate, const float* k, const float* v, float* out);
-size_t attn_prefill_work_bytes(const Dims& d, int T);
+                               const float* q_gate, const float* k, const float* v, float* out, bool split);
+// Workspace of the split-fp16 form (0: the call takes the fp32 form, which
+// needs none).
+size_t attn_prefill_split_bytes(const q35m_ctx* c, int start, int T);
 hipError_t launch_linear_q(q35m_ctx* c, int qtype, const void* w, const float* x, float* y,
                            int n_in, int n_out, int tokens);
 // Q5_K, IQ4_XS, Q2_0C and STQ1_0 projections of several tokens on the matrix

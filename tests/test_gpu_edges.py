@@ -236,3 +236,67 @@ def test_deltanet_prefill_long_context():
         say(f"  out rel err {e_out:.2e} (last chunk {e_last:.2e}), state rel err {e_st:.2e}")
         assert e_out <= TOL and e_last <= TOL and e_st <= TOL
         np.testing.assert_array_equal(c.state_read(0, 0, q35mix.STATE_CONV), cs_ref)
+
+
+def _attn_prefill_case(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None):
+    """One attention prefill of T tokens behind `start` cached rows against
+    the oracle; kmul / vmul scale single cached rows, (row, factor)."""
+    dims = oracle.dims(n_heads=nh, n_kv_heads=nkv)
+    rng = np.random.default_rng(1000 * nh + 10 * start + T)
+    wts = synth.attn_weights(256)
+    if q_norm is not None:
+        wts["q_norm"] = np.full(256, q_norm, np.float32)
+    ck = np.zeros((start + T, nkv * 256), np.float32)
+    cv = np.zeros_like(ck)
+    ck[:start] = rng.standard_normal((start, nkv * 256))
+    cv[:start] = rng.standard_normal((start, nkv * 256))
+    for arr, mul in ((ck, kmul), (cv, vmul)):
+        for row, f in mul or ():
+            arr[row] *= np.float32(f)
+    x = synth.attn_inputs(T, nh, nkv, 256, salt=3 + T)
+    with q35mix.Context(q35mix.qwen35_config(num_layers=1, num_heads=nh, num_kv_heads=nkv, is_recurrent=[0]), n_seqs=1,
+                        kv_capacity=start + T) as c:
+        c.set_attn_weights(0, wts)
+        if start:
+            c.state_write(0, 0, q35mix.STATE_KEYS, ck[:start])
+            c.state_write(0, 0, q35mix.STATE_VALUES, cv[:start])
+            if c.kv_len(0) < start:
+                c.advance(0, start - c.kv_len(0))
+        out = c.array((T, nh * 256))
+        c.attn_prefill(0, 0, T, c.array((T, 2 * nh * 256), x["q_gate"]), c.array((T, nkv * 256), x["k"]),
+                       c.array((T, nkv * 256), x["v"]), out)
+        got = out.download()
+    with np.errstate(all="ignore"):
+        want, _, _ = oracle.attn_prefill(dims, start, T, x["q_gate"], x["k"], x["v"], wts, ck, cv, n_threads=8)
+    return got, want
+
+
+@pytest.mark.parametrize("nh,nkv,start,T", [(16, 4, 0, 1), (16, 4, 31, 33), (16, 4, 32, 32), (16, 4, 33, 31), (16, 4, 300, 65),
+                                            (16, 4, 4000, 3), (16, 4, 0, 1100), (4, 4, 100, 129), (8, 4, 63, 65),
+                                            (8, 1, 700, 40), (16, 2, 0, 34)])
+def test_attn_prefill_chunks(nh, nkv, start, T):
+    """Query blocks and key tiles (32 rows) at their edges, blocks of one and
+    of many chunks, 1, 2, 4 and 8 q heads a kv head."""
+    got, want = _attn_prefill_case(nh, nkv, start, T)
+    e = np.max(np.abs(got - want)) / np.max(np.abs(want))
+    say(f"attn_prefill {nh}/{nkv} start {start} T {T}: {e:.2e}")
+    assert e <= 1e-5
+
+
+@pytest.mark.parametrize("case", ["v_spread", "k_spread", "v_zero_rows", "huge_v", "q_huge", "v_inf", "v_nan"])
+def test_attn_prefill_value_ranges(case):
+    """Cached rows whose magnitudes lie far apart, huge or not finite, and q
+    beyond the split's range: the query blocks that meet them take the fp32
+    form (one chunk and many), the others keep theirs."""
+    for start, T in ((200, 40), (3000, 37)):
+        kw = {"v_spread": {"vmul": [(50, 2.0 ** 20)]}, "k_spread": {"kmul": [(60, 2.0 ** -15)]},
+              "v_zero_rows": {"vmul": [(r, 0.0) for r in range(64, 96)]}, "huge_v": {"vmul": [(r, 1e25) for r in range(start)]},
+              "q_huge": {"q_norm": 2.0 ** 66, "kmul": [(r, 2.0 ** -66) for r in range(start)]},
+              "v_inf": {"vmul": [(50, np.inf)]}, "v_nan": {"vmul": [(50, np.nan)]}}[case]
+        got, want = _attn_prefill_case(16, 4, start, T, **kw)
+        fin = np.isfinite(want)
+        assert np.array_equal(np.isfinite(got), fin) and np.array_equal(np.isnan(got), np.isnan(want))
+        if fin.any():
+            e = np.max(np.abs(got - want)[fin]) / np.max(np.abs(want[fin]))
+            say(f"attn_prefill {case} start {start}: {e:.2e}")
+            assert e <= 1e-5
