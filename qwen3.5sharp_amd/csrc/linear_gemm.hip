@@ -1,8 +1,11 @@
-// Quantized projections of several tokens on the matrix cores, for the formats
-// whose reference result is one exact integer sum per block or sub-block
-// followed by an fp32 chain in block order (linear_q.hip states the formats,
-// the reference's functions and the one-token kernels):
+// Quantized projections of several tokens on the matrix cores.  The reference's
+// result is exact integer sums per block or sub-block followed by fp32 chains
+// in block order (linear_q.hip states the formats, the reference's functions,
+// the one-token kernels and the tiles of many tokens of Q4_K and Q6_K):
 //
+//   Q4_K    per 32-value sub-block  acc = fma(sc_s dot_s, dw dx, acc); per block
+//           mn = fma(sum_j min_j bsums, dmin dx, mn); acc - mn
+//   Q6_K    per block and lane k < 8  acc_k = fma(dw dx, sumi_k, acc_k)
 //   Q5_K    per block  acc += d (sum_s sc_s dot_s) - dmin (sum_j min_j bsums)
 //   IQ4_XS  per 32-value sub-block  acc += (d (ls - 32) dot_s) dx
 //   Q2_0C   per 256 values T; panel rows acc = fma(T, dw dx, acc), raw rows
@@ -10,7 +13,7 @@
 //   STQ1_0  per 256 values T; panel rows acc = fma(T, dw dx, acc), raw rows
 //           acc += (dw dx) T
 //
-// (dot_s and T exact integers, no fused multiply-add but where written), so
+// (dots, sums and T exact integers, no fused multiply-add but where written), so
 // results are the reference's bits at any tile shape.
 //
 // (linear_gemm_split, below, is the form for few outputs.)  A wave holds 16
@@ -37,10 +40,47 @@ namespace {
 // Rows of the 2-byte aligned formats are read at their own addresses.
 typedef uint32_t u32_a2 __attribute__((aligned(2)));
 typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
-typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 // A lane's share (lane group lg) of one 256-value block of its row.
 template <int QT> struct RowBlock;
+
+template <> struct RowBlock<4> {       // header; qs bytes 8 lg .. + 7 of each 32
+    uint4 hdr;
+    uint2 qs[4];
+    __device__ __forceinline__ void load(const unsigned char* row, int b, int lg) {
+        const unsigned char* p = row + (size_t)b * Q4K_BYTES;
+        hdr = *reinterpret_cast<const uint4*>(p);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) qs[j] = *reinterpret_cast<const uint2*>(p + 16 + 32 * j + 8 * lg);
+    }
+};
+
+// Half lg / 2 of ql and qh, the scales and d, as the dwords from the 4-byte
+// boundary below the 2-byte aligned block (16-byte loads at 2-byte aligned
+// addresses cost 1.5-2.7 us more a call); the rows of a launch end on a 4-byte
+// boundary.
+template <> struct RowBlock<6> {
+    uint32_t ql[17], qh[9], sc[5];
+    uint32_t sh;
+    __device__ __forceinline__ void load(const unsigned char* row, int b, int lg) {
+        const size_t at = reinterpret_cast<size_t>(row) + (size_t)b * Q6K_BYTES;
+        const unsigned char* p = reinterpret_cast<const unsigned char*>(at & ~(size_t)3);
+        const int j = lg >> 1;
+        sh = (uint32_t)at & 3;
+        words<17>(ql, p + 64 * j);
+        words<9>(qh, p + 128 + 32 * j);
+        words<5>(sc, p + 192);
+    }
+    template <int N> static __device__ __forceinline__ void words(uint32_t (&v)[N], const unsigned char* p) {
+#pragma unroll
+        for (int i = 0; i + 4 <= N; i += 4) {
+            const u32x4_a4 x = *reinterpret_cast<const u32x4_a4*>(p + 4 * i);
+            v[i] = x[0]; v[i + 1] = x[1]; v[i + 2] = x[2]; v[i + 3] = x[3];
+        }
+        v[N - 1] = *reinterpret_cast<const uint32_t*>(p + 4 * (N - 1));
+    }
+};
 
 template <> struct RowBlock<5> {       // header; qh and qs bytes 8 lg .. + 7 of each 32
     uint4 hdr;
@@ -118,29 +158,46 @@ __device__ __forceinline__ void lane_groups(uint32_t v, uint32_t (&r)[4]) {
 }
 
 // Terms of the fp32 chain a block adds to an output: (a, b) pairs, in order.
-template <int QT> constexpr int kTerms = QT == 14 ? 8 : 1;
+template <int QT> constexpr int kTerms = QT == 4 ? 9 : QT == 14 || QT == 6 ? 8 : 1;
 
 // The running values of 16 rows x 16 TT tokens: lane (l16, lg) holds tokens
-// 16 tt + 4 lg + r of weight row l16 (the layout of an MFMA result).  pend: a
-// raw Q2_0C row's first product of a 512-value pair.
+// 16 tt + 4 lg + r of weight row l16 (the layout of an MFMA result).  v[1]:
+// Q4_K's min sum, or a raw Q2_0C row's first product of a 512-value pair;
+// v[0..7]: Q6_K's lanes.
+template <int QT> constexpr int kAccs = QT == 6 ? 8 : QT == 4 || QT == 2 ? 2 : 1;
 template <int QT, int TT> struct Acc {
-    float v[TT][4], pend[QT == 2 ? TT : 1][4];
+    float v[kAccs<QT>][TT][4];
+    __device__ __forceinline__ float result(int tt, int r) const {
+#pragma clang fp contract(off)
+        if constexpr (QT == 4) {
+            return v[0][tt][r] - v[1][tt][r];
+        } else if constexpr (QT == 6) {    // VecDotQ4K.HorizontalSum (VecDotQ4K.cs:145-151)
+            const float s0 = v[0][tt][r] + v[4][tt][r], s1 = v[1][tt][r] + v[5][tt][r];
+            const float s2 = v[2][tt][r] + v[6][tt][r], s3 = v[3][tt][r] + v[7][tt][r];
+            return (s0 + s2) + (s1 + s3);
+        } else {
+            return v[0][tt][r];
+        }
+    }
 };
 
-// One term of the reference's chain.
+// Term s of a block in the reference's chain.
 template <int QT, int TT>
-__device__ __forceinline__ void chain(Acc<QT, TT>& acc, int tt, int r, float a, float b, int blk, bool panel) {
+__device__ __forceinline__ void chain(Acc<QT, TT>& acc, int s, int tt, int r, float a, float b, int blk, bool panel) {
 #pragma clang fp contract(off)
-    float& v = acc.v[tt][r];
-    if constexpr (QT == 5 || QT == 14) {
+    float& v = acc.v[QT == 6 ? s : QT == 4 ? s >> 3 : 0][tt][r];
+    if constexpr (QT == 4 || QT == 6) {
+        v = fmaf(a, b, v);
+    } else if constexpr (QT == 5 || QT == 14) {
         v = v + a;
     } else if (panel) {
         v = fmaf(a, b, v);
     } else if constexpr (QT == 1) {
         v = v + b * a;
     } else {
-        if (blk & 1) v = v + b * (acc.pend[tt][r] + a);
-        else acc.pend[tt][r] = a;
+        float& pend = acc.v[QT == 2 ? 1 : 0][tt][r];
+        if (blk & 1) v = v + b * (pend + a);
+        else pend = a;
     }
 }
 
@@ -153,7 +210,97 @@ __device__ __forceinline__ void block_terms(const RowBlock<QT>& w, const uint32_
     const uint32_t* xa = X + l16 * Q8K_WORDS;                    // A rows: token 16 tt + l16
     auto dx = [&](int tt, int r) { return __builtin_bit_cast(float, X[(16 * tt + 4 * lg + r) * Q8K_WORDS]); };
     const i32x4 zero = {0, 0, 0, 0};
-    if constexpr (QT == 5) {
+    // Q4_K / Q5_K min sum of a token tile, sum_j min_j (bsums 2j, 2j + 1): j =
+    // lg and lg + 4 of this lane's row (B) and token (A); at most 8 x 63 x
+    // 4064, exact in fp32.
+    auto min_sum = [&](int tt, uint32_t S1, uint32_t S2) {
+        const float m0 = (float)((S1 >> (8 * lg)) & 63);
+        const float m1 = (float)(((S2 >> (8 * lg + 4)) & 15) | (((S1 >> (8 * lg + 6)) & 3) << 4));
+        const uint32_t* xb = xa + 16 * tt * Q8K_WORDS + Q8K_BS;
+        float pa[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t p = xb[lg + 4 * h];
+            pa[h] = (float)((int)(int16_t)(p & 0xffff) + (int)(int16_t)(p >> 16));
+        }
+        const f32x4 md = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[0], m0, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(pa[1], m1, md, 0, 0, 0);
+    };
+    if constexpr (QT == 4) {
+        // The dot starts at the bits of 1.5 * 2^23 and is read as fp32, so that
+        // fma(dot, sc, -1.5 * 2^23 sc) = sc dot exactly (as in q4k_gemm).
+        const int m = 0x4B400000;
+        const i32x4 magic = {m, m, m, m};
+        const uint32_t S0 = w.hdr.y, S1 = w.hdr.z, S2 = w.hdr.w;
+        const uint32_t sl = S0 & 0x3f3f3f3fu, sh = (S2 & 0x0f0f0f0fu) | ((S0 >> 2) & 0x30303030u);
+        const float dw = half_bits_to_float(w.hdr.x & 0xffff), dmw = half_bits_to_float(w.hdr.x >> 16);
+        float cs[TT][4];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) cs[tt][r] = dw * dx(tt, r);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const uint32_t q0 = w.qs[s >> 1].x, q1 = w.qs[s >> 1].y;
+            const uint32_t b0 = ((s & 1) ? q0 >> 4 : q0) & 0x0f0f0f0fu, b1 = ((s & 1) ? q1 >> 4 : q1) & 0x0f0f0f0fu;
+            const long bv = (long)(((unsigned long)b1 << 32) | b0);
+            const float scf = (float)(((s < 4 ? sl : sh) >> (8 * (s & 3))) & 0xffu), negc = scf * -12582912.0f;
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+                const long av = *reinterpret_cast<const long*>(xa + 16 * tt * Q8K_WORDS + Q8K_QS + 8 * s + 2 * lg);
+                const i32x4 d = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bv, magic, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) term(s, tt, r, fmaf(__int_as_float(d[r]), scf, negc), cs[tt][r]);
+            }
+        }
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) {
+            const f32x4 md = min_sum(tt, S1, S2);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) term(8, tt, r, md[r], dmw * dx(tt, r));
+        }
+    } else if constexpr (QT == 6) {
+        // Lane k's sum as two planes of one 16x16x64 product each (the notes
+        // at q6k_gemm in linear_q.hip): lane group lg brings parts (j, m0),
+        // (j, m0 + 1) at bytes 4k .. + 3 and the bsums term.
+        const int j = lg >> 1, odd = lg & 1;
+        auto at = [&](const uint32_t* v, int i) { return __builtin_amdgcn_alignbyte(v[i + 1], v[i], w.sh); };
+        const float dw = half_bits_to_float((w.sc[4] >> (8 * w.sh)) & 0xffff);
+        float d[TT][4];
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) d[tt][r] = dx(tt, r) * dw;
+        const uint32_t rq = odd ? 3 : 31, rh0 = odd ? 31 : 27, rh1 = odd ? 1 : 29;
+        const uint32_t sc4[4] = {at(w.sc, 0), at(w.sc, 1), at(w.sc, 2), at(w.sc, 3)};
+        const uint32_t scw = lg < 2 ? (lg ? sc4[1] : sc4[0]) : (lg & 1 ? sc4[3] : sc4[2]);   // scales 4 lg .. + 3
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const uint32_t qa = at(w.ql, k), qb = at(w.ql, 8 + k), qh = at(w.qh, k);
+            const uint32_t v0 = (__builtin_amdgcn_alignbit(qa, qa, rq) & 0x1e1e1e1eu) |
+                                (__builtin_amdgcn_alignbit(qh, qh, rh0) & 0x60606060u);
+            const uint32_t v1 = (__builtin_amdgcn_alignbit(qb, qb, rq) & 0x1e1e1e1eu) |
+                                (__builtin_amdgcn_alignbit(qh, qh, rh1) & 0x60606060u);
+            uint32_t l0, h0, l1, h1;
+            q6k_split(v0, (int)(int8_t)(scw >> (8 * (k >> 2))), l0, h0);
+            q6k_split(v1, (int)(int8_t)(scw >> (8 * (2 + (k >> 2)))), l1, h1);
+            // -32 scales[2k + j] = 128 ((-s) >> 2) + 32 ((-s) & 3), bytes replicated
+            const int neg = -(int)(int8_t)(sc4[k >> 1] >> (16 * (k & 1) + 8 * j));
+            const uint32_t elo = __builtin_amdgcn_perm(0u, (uint32_t)((neg & 3) << 5), 0u);
+            const uint32_t ehi = __builtin_amdgcn_perm(0u, (uint32_t)(neg >> 2), 0u);
+            const i32x4 bh = {(int)h0, (int)h1, (int)ehi, (int)ehi}, bl = {(int)l0, (int)l1, (int)elo, (int)elo};
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+                const uint32_t* xt = xa + 16 * tt * Q8K_WORDS + Q8K_QS;
+                const int qv = 32 * j + 16 * odd + k, qe = 8 * k + 4 * j + 2 * odd;
+                const i32x4 av = {(int)xt[qv], (int)xt[qv + 8], (int)xt[qe], (int)xt[qe + 1]};
+                const i32x4 dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bh, zero, 0, 0, 0);
+                const i32x4 dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bl, zero, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) term(k, tt, r, d[tt][r], (float)((int)((unsigned)dh[r] << 7) + dl[r]));
+            }
+        }
+    } else if constexpr (QT == 5) {
         const uint32_t S0 = w.hdr.y, S1 = w.hdr.z, S2 = w.hdr.w;
         const uint32_t sl = S0 & 0x3f3f3f3fu;                                  // scales 0-3
         const uint32_t sh = (S2 & 0x0f0f0f0fu) | ((S0 >> 2) & 0x30303030u);    // scales 4-7
@@ -183,22 +330,10 @@ __device__ __forceinline__ void block_terms(const RowBlock<QT>& w, const uint32_
                 }
             }
         }
-        // Min term: j = lg and lg + 4 of this lane's row (B) and token (A);
-        // at most 8 x 63 x 4064, exact in fp32.
-        const float m0 = (float)((S1 >> (8 * lg)) & 63);
-        const float m1 = (float)(((S2 >> (8 * lg + 4)) & 15) | (((S1 >> (8 * lg + 6)) & 3) << 4));
         const float dw = half_bits_to_float(w.hdr.x & 0xffff), dmw = half_bits_to_float(w.hdr.x >> 16);
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt) {
-            const uint32_t* xb = xa + 16 * tt * Q8K_WORDS + Q8K_BS;
-            float pa[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const uint32_t p = xb[lg + 4 * h];
-                pa[h] = (float)((int)(int16_t)(p & 0xffff) + (int)(int16_t)(p >> 16));
-            }
-            f32x4 md = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[0], m0, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            md = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[1], m1, md, 0, 0, 0);
+            const f32x4 md = min_sum(tt, S1, S2);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float yd = dx(tt, r), d = dw * yd, dmin = dmw * yd;
@@ -270,8 +405,20 @@ __device__ __forceinline__ void block_terms(const RowBlock<QT>& w, const uint32_
 
 template <int QT>
 __host__ __device__ constexpr size_t row_bytes(int nb) {
-    return QT == 5 ? (size_t)nb * Q5K_BYTES : QT == 14 ? (size_t)nb * IQ4XS_BYTES : QT == 2 ? (size_t)(nb >> 1) * Q2_BYTES
+    return QT == 4 ? (size_t)nb * Q4K_BYTES : QT == 6 ? (size_t)nb * Q6K_BYTES : QT == 5 ? (size_t)nb * Q5K_BYTES : QT == 14 ? (size_t)nb * IQ4XS_BYTES : QT == 2 ? (size_t)(nb >> 1) * Q2_BYTES
                                                                                             : (size_t)nb * STQ_BYTES;
+}
+
+template <int QT, int TT>
+__device__ __forceinline__ void store_tile(const Acc<QT, TT>& acc, float* y, int row, int n_rows, int n_out, int tok0,
+                                           int tokens, int lg) {
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = tok0 + 16 * tt + 4 * lg + r;
+            if (row < n_rows && t < tokens) y[(size_t)t * n_out + row] = acc.result(tt, r);
+        }
 }
 
 // Blocks of the tokens in one LDS buffer: two buffers are 76 KiB, two
@@ -325,17 +472,11 @@ __global__ __launch_bounds__(64 * NW) void linear_gemm(const unsigned char* __re
                     const RowBlock<QT> wb = wq[u];
                     wq[u].load(wrow, min(b + PF, nb - 1), lg);
                     block_terms<QT, TT>(wb, reinterpret_cast<const uint32_t*>(xsh[buf][k]), l16, lg, panel,
-                                        [&](int, int tt, int r, float a, float f) { chain<QT, TT>(acc, tt, r, a, f, b, panel); });
+                                        [&](int s, int tt, int r, float a, float f) { chain<QT, TT>(acc, s, tt, r, a, f, b, panel); });
                 }
             }
     }
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int t = tok0 + 16 * tt + 4 * lg + r;
-            if (row < n_rows && t < tokens) y[(size_t)t * n_out + row] = acc.v[tt][r];
-        }
+    store_tile(acc, y, row, n_rows, n_out, tok0, tokens, lg);
 }
 
 // The same for few outputs (few tokens, or few rows): a workgroup takes 16 RG
@@ -350,7 +491,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void linear_gemm_split(const unsi
                                                                       int n_in, int n_rows, int n_out, int tokens,
                                                                       int panel_rows, int KW) {
     constexpr int TOK = 16 * TT, XW = Q8K_WORDS / 4, XB = TOK * XW, RUNS = (XB + 63) / 64;
-    constexpr int NT = kTerms<QT>, NV = QT == 2 ? 2 : 1;
+    constexpr int NT = kTerms<QT>, NV = kAccs<QT>;
     extern __shared__ uint4 split_smem[];                        // two buffers of KW blocks' tokens, then the chain
     const int nb = n_in / QK, passes = (nb + KW - 1) / KW;
     const int lane = threadIdx.x & 63, l16 = lane & 15, lg = lane >> 4;
@@ -394,34 +535,56 @@ __global__ __launch_bounds__(64 * kSplitWaves) void linear_gemm_split(const unsi
             block_terms<QT, TT>(wb, reinterpret_cast<const uint32_t*>(split_smem + ((p & 1) * KW + kw) * XB), l16, lg, panel,
                                 [&](int s, int tt, int r, float a, float f) { ta[s][tt][r] = a; tb[s][tt][r] = f; });
         const int steps = min(KW, nb - p * KW);
+        if constexpr (QT == 6) {
+            // Eight chains an output: every wave's terms to LDS, and each wave
+            // then runs its share of the lanes over the pass's blocks (passed
+            // from wave to wave, the chains took 0.4 us a block).
+            static_assert(TT == 1 && RG == 1, "one tile a workgroup");
+            if (b < nb) {
+#pragma unroll
+                for (int s = 0; s < 8; ++s) relay[(kw * 9 + s) * 64] = *reinterpret_cast<const float4*>(tb[s][0]);
+                relay[(kw * 9 + 8) * 64] = *reinterpret_cast<const float4*>(ta[0][0]);
+            }
+            lds_barrier();
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                if (s % KW == kw)
+#pragma unroll 4
+                    for (int k = 0; k < steps; ++k) {
+                        const float4 x = relay[(k * 9 + s) * 64], d = relay[(k * 9 + 8) * 64];
+                        chain<QT, TT>(acc, s, 0, 0, d.x, x.x, b, panel);
+                        chain<QT, TT>(acc, s, 0, 1, d.y, x.y, b, panel);
+                        chain<QT, TT>(acc, s, 0, 2, d.z, x.z, b, panel);
+                        chain<QT, TT>(acc, s, 0, 3, d.w, x.w, b, panel);
+                    }
+            if (p + 1 < passes) continue;
+            lds_barrier();
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                if (s % KW == kw) relay[s * 64] = *reinterpret_cast<const float4*>(acc.v[s][0]);
+            lds_barrier();
+            if (kw > 0) return;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) *reinterpret_cast<float4*>(acc.v[s][0]) = relay[s * 64];
+            store_tile(acc, y, row, n_rows, n_out, tok0, tokens, lg);
+            continue;
+        }
         for (int k = 0; k < steps; ++k) {
             if (kw == k) {
                 if (b > 0)
 #pragma unroll
-                    for (int tt = 0; tt < TT; ++tt) {
-                        *reinterpret_cast<float4*>(acc.v[tt]) = relay[64 * tt];
-                        if constexpr (QT == 2) *reinterpret_cast<float4*>(acc.pend[tt]) = relay[64 * (TT + tt)];
-                    }
+                    for (int i = 0; i < NV * TT; ++i) *reinterpret_cast<float4*>(acc.v[i / TT][i % TT]) = relay[64 * i];
 #pragma unroll
                 for (int s = 0; s < NT; ++s)
 #pragma unroll
                     for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) chain<QT, TT>(acc, tt, r, ta[s][tt][r], tb[s][tt][r], b, panel);
+                        for (int r = 0; r < 4; ++r) chain<QT, TT>(acc, s, tt, r, ta[s][tt][r], tb[s][tt][r], b, panel);
                 if (b + 1 < nb) {
 #pragma unroll
-                    for (int tt = 0; tt < TT; ++tt) {
-                        relay[64 * tt] = *reinterpret_cast<const float4*>(acc.v[tt]);
-                        if constexpr (QT == 2) relay[64 * (TT + tt)] = *reinterpret_cast<const float4*>(acc.pend[tt]);
-                    }
+                    for (int i = 0; i < NV * TT; ++i) relay[64 * i] = *reinterpret_cast<const float4*>(acc.v[i / TT][i % TT]);
                 } else {
-#pragma unroll
-                    for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int t = tok0 + 16 * tt + 4 * lg + r;
-                            if (row < n_rows && t < tokens) y[(size_t)t * n_out + row] = acc.v[tt][r];
-                        }
+                    store_tile(acc, y, row, n_rows, n_out, tok0, tokens, lg);
                 }
             }
             if (k + 1 < steps) lds_barrier();
@@ -430,8 +593,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) void linear_gemm_split(const unsi
 }
 
 template <int QT>
-hipError_t go(q35m_ctx* c, int kid, const unsigned char* w, const uint32_t* q8, float* y, int n_in, int n_out, int tokens,
-              int panel_rows) {
+hipError_t go(q35m_ctx* c, int kid, const unsigned char* w, const uint32_t* q8, float* y, int n_in, int n_rows, int n_out,
+              int tokens, int panel_rows) {
     const int nb = n_in / QK;
     auto pieces = [&](int tok, auto one) {
         // The tokens are addressed through a buffer descriptor: at most 2 GiB a launch.
@@ -448,16 +611,19 @@ hipError_t go(q35m_ctx* c, int kid, const unsigned char* w, const uint32_t* q8, 
     };
     auto whole = [&](auto kern, int tok, int nw) {
         return pieces(tok, [&](ProfScope& ps, const uint32_t* qt, float* yt, int nt) {
-            hipExtLaunchKernelGGL(kern, dim3((n_out + 16 * nw - 1) / (16 * nw), (nt + tok - 1) / tok), dim3(64 * nw), 0,
-                                  c->stream, ps.a, ps.b, 0, w, qt, yt, n_in, n_out, n_out, nt, panel_rows);
+            hipExtLaunchKernelGGL(kern, dim3((n_rows + 16 * nw - 1) / (16 * nw), (nt + tok - 1) / tok), dim3(64 * nw), 0,
+                                  c->stream, ps.a, ps.b, 0, w, qt, yt, n_in, n_rows, n_out, nt, panel_rows);
         });
     };
     auto split = [&](auto kern, int tt, int rg) {
-        const int wmax = kSplitWaves / rg, passes = (nb + wmax - 1) / wmax, kw = (nb + passes - 1) / passes;
-        const size_t lds = ((passes > 1 ? 2 : 1) * (size_t)kw * tt * 16 * Q8K_WORDS / 4 + (size_t)rg * (QT == 2 ? 2 : 1) * tt * 64) * 16;
+        // Q6_K: two passes' tokens and the terms of eight waves fill the LDS.
+        const int wmax = QT == 6 && nb > kSplitWaves ? 8 : kSplitWaves / rg;
+        const int passes = (nb + wmax - 1) / wmax, kw = (nb + passes - 1) / passes;
+        const size_t chains = QT == 6 ? (size_t)std::max(kw * 9, 8) : (size_t)rg * kAccs<QT> * tt;
+        const size_t lds = ((passes > 1 ? 2 : 1) * (size_t)kw * tt * 16 * Q8K_WORDS / 4 + chains * 64) * 16;
         return pieces(16 * tt, [&](ProfScope& ps, const uint32_t* qt, float* yt, int nt) {
-            hipExtLaunchKernelGGL(kern, dim3((n_out + 16 * rg - 1) / (16 * rg), (nt + 16 * tt - 1) / (16 * tt)),
-                                  dim3(64 * kw * rg), lds, c->stream, ps.a, ps.b, 0, w, qt, yt, n_in, n_out, n_out, nt,
+            hipExtLaunchKernelGGL(kern, dim3((n_rows + 16 * rg - 1) / (16 * rg), (nt + 16 * tt - 1) / (16 * tt)),
+                                  dim3(64 * kw * rg), lds, c->stream, ps.a, ps.b, 0, w, qt, yt, n_in, n_rows, n_out, nt,
                                   panel_rows, kw);
         });
     };
@@ -473,24 +639,33 @@ hipError_t go(q35m_ctx* c, int kid, const unsigned char* w, const uint32_t* q8, 
     // 35; Q2_0C at 200 - / 57 / 26 / 19.  One thread a block and a serial
     // chain a row for 8 tokens at a time took 7.1 at 2 tokens, 17.6 at 16, 310
     // at 500, 1246 at 2048 (IQ4_XS 373, Q2_0C 422, STQ1_0 770 at 500).
-    const long tiles = (long)((n_out + 15) / 16) * ((tokens + 15) / 16);
-    if (tiles <= 640) return split(linear_gemm_split<QT, 1, 1>, 1, 1);
-    if (tiles <= 2304) return split(linear_gemm_split<QT, 2, 2>, 2, 2);
-    if (tiles <= 4608) return whole(linear_gemm<QT, 2, 8>, 32, 8);
-    return whole(linear_gemm<QT, 4, 8>, 64, 8);
+    const long tiles = (long)((n_rows + 15) / 16) * ((tokens + 15) / 16);
+    if constexpr (QT == 6) {
+        return split(linear_gemm_split<QT, 1, 1>, 1, 1);
+    } else {
+        // Q4_K at 16 tokens 10.9 / 9.3 / 18 / 25, at 64 34 / 17.6 / 18 / 25, at
+        // 128 66 / 32 / 19 / 26, at 256 131 / 63 / 34 / 27; 2560 -> 1024 at 64
+        // tokens (256 tiles) 6.8 / 9.7 / 18 / 24.
+        if (tiles <= (QT == 4 ? 400 : 640)) return split(linear_gemm_split<QT, 1, 1>, 1, 1);
+        if (tiles <= (QT == 4 ? 1536 : 2304)) return split(linear_gemm_split<QT, 2, 2>, 2, 2);
+        if (tiles <= 4608) return whole(linear_gemm<QT, 2, 8>, 32, 8);
+        return whole(linear_gemm<QT, 4, 8>, 64, 8);
+    }
 }
 
 }  // namespace
 
-hipError_t launch_linear_gemm(q35m_ctx* c, int qtype, const void* w, const void* q8, float* y, int n_in, int n_out,
-                              int tokens, int panel_rows) {
+hipError_t launch_linear_gemm(q35m_ctx* c, int qtype, const void* w, const void* q8, float* y, int n_in, int n_rows,
+                              int n_out, int tokens, int panel_rows) {
     const unsigned char* wb = reinterpret_cast<const unsigned char*>(w);
     const uint32_t* qb = reinterpret_cast<const uint32_t*>(q8);
     switch (qtype) {
-        case 5: return go<5>(c, K_Q5K_GEMM, wb, qb, y, n_in, n_out, tokens, 0);
-        case 14: return go<14>(c, K_IQ4XS_GEMM, wb, qb, y, n_in, n_out, tokens, 0);
-        case 2: return go<2>(c, K_Q2_0C_GEMM, wb, qb, y, n_in, n_out, tokens, panel_rows);
-        default: return go<1>(c, K_STQ1_0_GEMM, wb, qb, y, n_in, n_out, tokens, panel_rows);
+        case 4: return go<4>(c, K_Q4K_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, 0);
+        case 6: return go<6>(c, K_Q6K_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, 0);
+        case 5: return go<5>(c, K_Q5K_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, 0);
+        case 14: return go<14>(c, K_IQ4XS_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, 0);
+        case 2: return go<2>(c, K_Q2_0C_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, panel_rows);
+        default: return go<1>(c, K_STQ1_0_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, panel_rows);
     }
 }
 

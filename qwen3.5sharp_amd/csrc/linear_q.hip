@@ -233,7 +233,7 @@ template <int QT, int NB>
 __global__ __launch_bounds__(LQ_THREADS) void linear_q(const unsigned char* __restrict__ w,
                                                        const uint32_t* __restrict__ q8,
                                                        float* __restrict__ y, int n_in, int n_out,
-                                                       int tokens, int rows_per_wg, int row_base) {
+                                                       int tokens, int rows_per_wg, int row_base, int tok_per_wg) {
 #pragma clang fp contract(off)
     constexpr int BB = QT == 4 ? Q4K_BYTES : Q6K_BYTES;
     constexpr int NL = QT == 4 ? 12 : 8;          // integer lanes per block
@@ -292,7 +292,8 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_q(const unsigned char* __re
         }
     }
 
-    for (int t = 0; t < tokens; ++t) {
+    const int t_end = min(tokens, ((int)blockIdx.y + 1) * tok_per_wg);
+    for (int t = blockIdx.y * tok_per_wg; t < t_end; ++t) {
         {
             // The token's Q8_K row, nb x 19 16-byte chunks, 8 loads a lane in flight.
             const uint4* src = reinterpret_cast<const uint4*>(q8 + (size_t)t * nb * Q8K_WORDS);
@@ -1107,21 +1108,6 @@ struct Q6Stage {
 
 typedef const volatile __attribute__((address_space(3))) uint32_t lds_cvu32;
 
-typedef short s16x2 __attribute__((ext_vector_type(2)));
-
-// Four unsigned 6-bit values given doubled (bytes of v2 = 2 v) times sc, as
-// the low (& 127) and high (>> 7, two's complement) int8 planes of the
-// products sc v.  The doubled 16-bit products 2 sc v are formed in pairs:
-// the high plane is their high bytes, the low plane bits 1-7 of their low
-// bytes.
-__device__ __forceinline__ void q6k_split(uint32_t v2, int sc, uint32_t& lo, uint32_t& hi) {
-    const s16x2 s2 = {(short)sc, (short)sc};
-    const uint32_t a = __builtin_bit_cast(uint32_t, __builtin_bit_cast(s16x2, __builtin_amdgcn_perm(0u, v2, 0x0c010c00u)) * s2);
-    const uint32_t b = __builtin_bit_cast(uint32_t, __builtin_bit_cast(s16x2, __builtin_amdgcn_perm(0u, v2, 0x0c030c02u)) * s2);
-    lo = (__builtin_amdgcn_perm(b, a, 0x06040200u) >> 1) & 0x7f7f7f7fu;
-    hi = __builtin_amdgcn_perm(b, a, 0x07050301u);
-}
-
 // A operand of lane k = 2 KH + (kk & 1) + 4 (kk >> 1) for token tile tt:
 // qs dwords 32j + 8 m0 + k and + 8 (the values' q8), then 8k + 4j + (g & 1)
 // and + 2 (sub-block 2k + j: lane groups 2j and 2j + 1 read opposite bank
@@ -1596,7 +1582,7 @@ hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const
         // else none.
         int panel_rows = n_out & ~7;
         if (qtype == 1 && tokens > 1) panel_rows = ((tokens & 3) == 0 && (n_out & 7) == 0) ? n_out : 0;
-        if (tokens >= 2) return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, tokens, panel_rows);
+        if (tokens >= 2) return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, n_out, tokens, panel_rows);
         const int rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
         const int ub = qtype == 2 ? Q2_BYTES / 2 : STQ_BYTES;
         const int nchunk_max = (rows_per_wg * nb * ub + 31) / 16 + 1;
@@ -1612,7 +1598,7 @@ hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const
         return hipGetLastError();
     }
     if (qtype == 5 || qtype == 14) {
-        if (tokens >= 2) return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, tokens, 0);
+        if (tokens >= 2) return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, n_out, tokens, 0);
         const int rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
         const dim3 grid((n_out + rows_per_wg - 1) / rows_per_wg);
         const size_t lds = (size_t)nb * Q8K_WORDS * 4 + (size_t)LQ_THREADS * QS_TLD * 4;
@@ -1648,29 +1634,52 @@ hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const
         return hipSuccess;
     };
     // Q4_K with several tokens: the panel order for the first n_out & ~7 rows
-    // (the reference's MulMatQ4K.Gemm), the GEMV for the rest.
-    const int row_base = (qtype == 4 && tokens > 1) ? (n_out & ~7) : 0;
-    if (row_base > 0) {
-        const hipError_t e = tiled(q4k_gemm, K_Q4K_GEMM, Q4K_BYTES, GR, GT, GTHREADS, row_base);
+    // (the reference's MulMatQ4K.Gemm), the GEMV for the rest.  Q6_K keeps one
+    // token's arithmetic in every form; with an odd number of blocks its last
+    // row stays out of the tiled kernels, whose 4-byte loads could not reach
+    // the end of it.
+    const int rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
+    int row_base = 0;
+    if (tokens > 1) {
+        // The GEMV takes a few tokens while its workgroups fit the CUs about
+        // once; the matrix cores the rest: linear_gemm's small tiles while they
+        // are few, else 64-token tiles.  Measured (us; GEMV / small / 64-token
+        // tiles): Q6_K 4096 -> 2560 at 2 tokens 6.8 / 12 / 29, at 4 9.8 / 12 /
+        // 29, at 8 17 / 12 / 29, at 32 - / 22 / 29; 2560 -> 8192 at 2 11 / 16.5
+        // / 20, at 16 - / 16.5 / 20, at 32 - / 36 / 20; 2560 -> 1024 at 4 6.0 /
+        // 9.3 / 19, at 16 10.4 / 9.5 / 19 (a workgroup's tokens one after the
+        // other: 11.6 at 4, 47 at 15 of 2560 -> 8192).  Q4_K (GEMV order in no
+        // whole panel: small tiles / 64-token tiles) 2560 -> 8192 at 8 9.1 / 30,
+        // at 128 19 / 32, at 256 27 / 32, at 500 49 / 44.
+        const long groups = (n_out + rows_per_wg - 1) / rows_per_wg;
+        const long tiles = (long)((n_out + 15) / 16) * ((tokens + 15) / 16);
+        if (qtype == 4) {
+            row_base = n_out & ~7;
+        } else if (c->proj_order == Q35M_PROJ_BLOCK && tokens >= 16 && (((size_t)n_out * nb) & 1) == 0) {
+            return tiled(q6k_gemm_blk, K_Q6K_GEMM_BLK, Q6K_BYTES, BR, BT, BTHREADS, n_out);
+        } else if (groups * tokens > 4000 || tokens > 16) {
+            row_base = n_out - (int)(((size_t)n_out * nb) & 1);
+        }
+        hipError_t e = hipSuccess;
+        if (row_base > 0) {
+            const bool small = qtype == 4 ? tiles <= 8192 : tiles * nb <= 5120;
+            if (small) e = launch_linear_gemm(c, qtype, w, q8, y, n_in, row_base, n_out, tokens, 0);
+            else if (qtype == 4) e = tiled(q4k_gemm, K_Q4K_GEMM, Q4K_BYTES, GR, GT, GTHREADS, row_base);
+            else e = tiled(q6k_gemm, K_Q6K_GEMM, Q6K_BYTES, SGR, SGT, 256, row_base);
+        }
         if (e != hipSuccess || row_base == n_out) return e;
     }
-    // Q6_K: the tiled kernel from 16 tokens when n_out * n_in / 256 is even
-    // (see q6k_gemm), the per-token GEMV otherwise; both keep the same
-    // per-token arithmetic, so the results are identical.
-    if (qtype == 6 && tokens >= 16 && (((size_t)n_out * nb) & 1) == 0) {
-        if (c->proj_order == Q35M_PROJ_BLOCK)
-            return tiled(q6k_gemm_blk, K_Q6K_GEMM_BLK, Q6K_BYTES, BR, BT, BTHREADS, n_out);
-        return tiled(q6k_gemm, K_Q6K_GEMM, Q6K_BYTES, SGR, SGT, 256, n_out);
-    }
-    const int rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
+    // Tokens a workgroup: one while the workgroups fit the CUs about once (a
+    // tiled call's last rows, many tokens of few rows, took 0.75 us a token).
     const int grid = (n_out - row_base + rows_per_wg - 1) / rows_per_wg;
+    const int tok_per_wg = (int)(((long)tokens * grid + 1499) / 1500);
     const int bb = qtype == 4 ? Q4K_BYTES : Q6K_BYTES;
     const size_t lds = 16 * (size_t)lq_wchunks(qtype, rows_per_wg, nb, bb) + (size_t)nb * Q8K_WORDS * 4 +
                        (size_t)LQ_THREADS * LANES_LD * 4 + (size_t)LQ_MAX_ROWS * 12 * 4;
     auto launch = [&](auto kern, int kid) {
         ProfScope ps_(c, kid);
-        hipExtLaunchKernelGGL(kern, dim3(grid), dim3(LQ_THREADS), lds, c->stream, ps_.a, ps_.b, 0, wb, qb, y,
-                              n_in, n_out, tokens, rows_per_wg, row_base);
+        hipExtLaunchKernelGGL(kern, dim3(grid, (tokens + tok_per_wg - 1) / tok_per_wg), dim3(LQ_THREADS), lds, c->stream,
+                              ps_.a, ps_.b, 0, wb, qb, y, n_in, n_out, tokens, rows_per_wg, row_base, tok_per_wg);
     };
     if (qtype == 4)
         launch(nb == 10 ? linear_q<4, 10> : nb == 16 ? linear_q<4, 16> : linear_q<4, 0>, K_Q4K_LINEAR);

@@ -207,8 +207,8 @@ hipError_t launch_linear_q(q35m_ctx* c, int qtype, const void* w, const float* x
                            int n_in, int n_out, int tokens);
 // Q5_K, IQ4_XS, Q2_0C and STQ1_0 projections of several tokens on the matrix
 // cores; rows below panel_rows take the eight-row panel order (Q2_0C, STQ1_0).
-hipError_t launch_linear_gemm(q35m_ctx* c, int qtype, const void* w, const void* q8, float* y, int n_in, int n_out,
-                              int tokens, int panel_rows);
+hipError_t launch_linear_gemm(q35m_ctx* c, int qtype, const void* w, const void* q8, float* y, int n_in, int n_rows,
+                              int n_out, int tokens, int panel_rows);
 hipError_t launch_add_rmsnorm(q35m_ctx* c, float* hidden, const float* delta, const float* w, float* y, void* q8,
                               int dim, int tokens, float eps);
 size_t linear_q_work_bytes(int n_in, int tokens);

@@ -73,13 +73,17 @@ def test_linear_q_bit_exact(ctx, qtype, n_in, n_out, tokens):
     assert bad.size == 0
 
 
-@pytest.mark.parametrize("qtype", [1, 2, 5, 14])
+@pytest.mark.parametrize("qtype", TYPES)
 @pytest.mark.parametrize("n_in,n_out,tokens", [(512, 15, 2), (2560, 63, 16), (4608, 65, 17), (1024, 130, 32),
-                                               (3584, 17, 33), (512, 257, 64), (5120, 34, 65), (1536, 129, 191)])
+                                               (3584, 17, 33), (512, 257, 64), (5120, 34, 65), (1536, 129, 191),
+                                               (512, 8190, 33), (1024, 2047, 100), (512, 3001, 700), (2304, 2111, 20),
+                                               (16384, 4111, 3), (2560, 1701, 16)])
 def test_linear_gemm_tiles(ctx, qtype, n_in, n_out, tokens):
-    """The matrix-core tiles of Q5_K, IQ4_XS, Q2_0C and STQ1_0 at the edges of
-    their rows (16 a wave), tokens (16, 32, 64) and block pipelines, bit for
-    bit (STQ1_0: panel and raw row orders by the token count)."""
+    """The matrix-core tiles of each rule at the edges of their rows (16 a
+    wave), tokens (16, 32, 64) and block pipelines, and the rows the tiles
+    leave to the GEMV, bit for bit (STQ1_0: panel and raw row orders by the
+    token count)."""
+    n_in += -n_in % qb.VALUES[qtype]
     rng = np.random.default_rng(31 * qtype + n_in + n_out + tokens)
     w = qb.random_blocks(rng, qtype, qb.nblocks(qtype, n_out * n_in))
     x = rng.standard_normal((tokens, n_in)).astype(np.float32)
