@@ -383,9 +383,14 @@ __device__ __forceinline__ uint32_t abs_bits(float x) { return __float_as_uint(x
 __device__ __forceinline__ int exp_of(uint32_t bits) { return max((int)(bits >> 23) - 126, kMinExp); }
 
 __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, kWave));
-    return v;
+    const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    v = max(h[0], h[1]);
+    const auto q = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = max(q[0], q[1]);
+    v = max(v, row_xor_bits<8>(v));
+    v = max(v, row_xor_bits<4>(v));
+    v = max(v, row_xor_bits<2>(v));
+    return max(v, row_xor_bits<1>(v));
 }
 
 __device__ __forceinline__ float pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
@@ -632,8 +637,10 @@ __global__ __launch_bounds__(64 * SWAVES, 2) void attn_split_flash(
                 x[k][j] = x[k][j] * scale * (1.0f + Q.q_norm[32 * k + 8 * g + j]) * post;
                 m = max(m, abs_bits(x[k][j]));
             }
-        m = max(m, (uint32_t)__shfl_xor((int)m, 16, kWave));
-        m = max(m, (uint32_t)__shfl_xor((int)m, 32, kWave));
+        const auto mh = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+        m = max(mh[0], mh[1]);
+        const auto mq = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+        m = max(mq[0], mq[1]);
         const int eq = min(exp_of(m), kMaxExp);
         bad = exp_of(m) > kMaxExp;
         const float qs = pow2(kScaleTop - eq);

@@ -58,31 +58,55 @@ __device__ __forceinline__ float xor32_sum(float v) { const float2 p = lanes_xor
 __device__ __forceinline__ float xor16_max(float v) { const float2 p = lanes_xor16(v); return fmaxf(p.x, p.y); }
 __device__ __forceinline__ float xor32_max(float v) { const float2 p = lanes_xor32(v); return fmaxf(p.x, p.y); }
 
-// Butterfly sum over all 64 lanes of a wave (the 32- and 16-lane steps by
-// lane swaps, the rest by shuffles within rows).
-__device__ __forceinline__ float wave_sum(float v) {
-    v = xor32_sum(v);
-    v = xor16_sum(v);
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
+// The value of lane l ^ K of the same 16-lane row (K = 1, 2, 4, 8), by data
+// parallel primitives: VALU moves of a few cycles, where a shuffle is an LDS
+// round trip of over a hundred (K = 4 is two moves: lanes 7 - l, then 3 - l).
+template <int CTRL>
+__device__ __forceinline__ uint32_t row_move(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+template <int K>
+__device__ __forceinline__ uint32_t row_xor_bits(uint32_t v) {
+    static_assert(K == 1 || K == 2 || K == 4 || K == 8, "within a row");
+    if constexpr (K == 1) return row_move<0xB1>(v);              // quad_perm 1 0 3 2
+    else if constexpr (K == 2) return row_move<0x4E>(v);         // quad_perm 2 3 0 1
+    else if constexpr (K == 4) return row_move<0x1B>(row_move<0x141>(v));   // row_half_mirror, quad_perm 3 2 1 0
+    else return row_move<0x128>(v);                              // row_ror 8
+}
+template <int K>
+__device__ __forceinline__ float row_xor(float v) { return __uint_as_float(row_xor_bits<K>(__float_as_uint(v))); }
+
+// Lane l - 4 of the row: where lanes l and l + 8 agree, as after a butterfly's
+// step 8, the value of lane l ^ 4 in one move.
+__device__ __forceinline__ float row_ror4(float v) { return __uint_as_float(row_move<0x124>(__float_as_uint(v))); }
+
+// Sums / maximum over each 16-lane row, the steps 8, 4, 2, 1 of a butterfly.
+__device__ __forceinline__ float row_sum(float v) {
+    v += row_xor<8>(v);
+    v += row_ror4(v);
+    v += row_xor<2>(v);
+    return v + row_xor<1>(v);
+}
+__device__ __forceinline__ float row_max(float v) {
+    v = fmaxf(v, row_xor<8>(v));
+    v = fmaxf(v, row_ror4(v));
+    v = fmaxf(v, row_xor<2>(v));
+    return fmaxf(v, row_xor<1>(v));
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-    v = xor32_max(v);
-    v = xor16_max(v);
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-    return v;
-}
+// Butterfly sum / maximum over all 64 lanes of a wave.
+__device__ __forceinline__ float wave_sum(float v) { return row_sum(xor16_sum(xor32_sum(v))); }
+__device__ __forceinline__ float wave_max(float v) { return row_max(xor16_max(xor32_max(v))); }
 
 // Sum over lane groups of `width` consecutive lanes (width a power of two <= 64).
 template <int width>
 __device__ __forceinline__ float group_sum(float v) {
     if constexpr (width >= 64) v = xor32_sum(v);
     if constexpr (width >= 32) v = xor16_sum(v);
-#pragma unroll
-    for (int o = (width < 16 ? width : 16) / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+    if constexpr (width >= 16) return row_sum(v);
+    if constexpr (width >= 8) v += row_xor<4>(v);
+    if constexpr (width >= 4) v += row_xor<2>(v);
+    if constexpr (width >= 2) v += row_xor<1>(v);
     return v;
 }
 
@@ -130,10 +154,10 @@ __device__ __forceinline__ int xcd_remap(int b, int total) {
 __device__ __forceinline__ float4 rope_norm_regs(float4 x, float4 c, float4 s, float4 ww, int lane,
                                                  float eps, float post_scale) {
     float4 p;
-    p.x = __shfl_xor(x.x, 8, kWave);
-    p.y = __shfl_xor(x.y, 8, kWave);
-    p.z = __shfl_xor(x.z, 8, kWave);
-    p.w = __shfl_xor(x.w, 8, kWave);
+    p.x = row_xor<8>(x.x);
+    p.y = row_xor<8>(x.y);
+    p.z = row_xor<8>(x.z);
+    p.w = row_xor<8>(x.w);
     float4 lo, hi;      // x0' = x0 c - x1 s (lanes 0-7), x1' = x0 s + x1 c (lanes 8-15)
     lo.x = x.x * c.x - p.x * s.x;
     lo.y = x.y * c.y - p.y * s.y;

@@ -177,13 +177,12 @@ __global__ __launch_bounds__(NT) void deltanet_decode_kernel(
         sqp[0] += s[j].x * qa; sqp[1] += s[j].y * qa; sqp[2] += s[j].z * qa; sqp[3] += s[j].w * qa;
     }
     // Lanes c4 + C4N*r of a wave share columns: fold them, then the waves.
+    static_assert(C4N == 32, "two lanes share a column");
 #pragma unroll
-    for (int m = C4N; m < kWave; m <<= 1)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            kvp[c] += __shfl_xor(kvp[c], m, kWave);
-            sqp[c] += __shfl_xor(sqp[c], m, kWave);
-        }
+    for (int c = 0; c < 4; ++c) {
+        kvp[c] = xor32_sum(kvp[c]);
+        sqp[c] = xor32_sum(sqp[c]);
+    }
     if (lane < C4N)
 #pragma unroll
         for (int c = 0; c < 4; ++c) {

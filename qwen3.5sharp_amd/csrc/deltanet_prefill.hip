@@ -843,8 +843,11 @@ __global__ __launch_bounds__(256, 3) void dn_chunk_out(PrefillWork w, const floa
         const int o4 = tid + 256 * i, row = o4 >> 5, c4 = o4 & 31, t = t0 + row;
         const float4 o = *reinterpret_cast<const float4*>(&o_s[row][4 * c4]);
         float ss = o.x * o.x + o.y * o.y + o.z * o.z + o.w * o.w;
-#pragma unroll
-        for (int m = 1; m < 32; m <<= 1) ss += __shfl_xor(ss, m, kWave);
+        ss += row_xor<1>(ss);
+        ss += row_xor<2>(ss);
+        ss += row_xor<4>(ss);
+        ss += row_xor<8>(ss);
+        ss = xor16_sum(ss);
         if (t >= T) continue;
         const float rs = 1.0f / sqrtf(ss / (float)kDk + eps);
         float4 r;
