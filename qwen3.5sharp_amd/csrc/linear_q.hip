@@ -50,18 +50,17 @@ __device__ __forceinline__ void q8k_from16(const float (&v)[16], int lane, uint3
     float amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[i]));
+    amax = row_max(amax);
+    // The first element of that magnitude, its sign in the index's low bit.
+    int first = 2 * QK;
 #pragma unroll
-    for (int m = 1; m < 16; m <<= 1) amax = fmaxf(amax, __shfl_xor(amax, m, kWave));
-    int e = 16;
-#pragma unroll
-    for (int i = 15; i >= 0; --i) e = fabsf(v[i]) == amax ? i : e;
-    int first = e < 16 ? 16 * li + e : QK;
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) first = min(first, __shfl_xor(first, m, kWave));
-    float mine = v[0];
-#pragma unroll
-    for (int i = 1; i < 16; ++i) mine = (first & 15) == i ? v[i] : mine;
-    const float mx = __shfl(mine, (lane & ~15) + min(first >> 4, 15), kWave);
+    for (int i = 15; i >= 0; --i)
+        if (fabsf(v[i]) == amax) first = 2 * (16 * li + i) + (int)(__float_as_uint(v[i]) >> 31);
+    first = min(first, (int)row_xor_bits<8>(first));
+    first = min(first, (int)row_xor_bits<4>(first));
+    first = min(first, (int)row_xor_bits<2>(first));
+    first = min(first, (int)row_xor_bits<1>(first));
+    const float mx = first & 1 ? -amax : amax;
     uint32_t pk[4] = {0u, 0u, 0u, 0u};
     int bsum = 0;
     float delta = 0.0f;
@@ -82,6 +81,35 @@ __device__ __forceinline__ void q8k_from16(const float (&v)[16], int lane, uint3
     }
 }
 
+// Bytes k of the four dwords q[0..3] gathered into dword k (a 4 x 4 byte
+// transpose): Q2_0C's byte c of a qs dword holds values 4c .. 4c + 3, so its
+// bit pair k of every byte meets the activations 16 i + 4c + k.
+__device__ __forceinline__ uint4 byte_transpose(uint4 q) {
+    const uint32_t a = __builtin_amdgcn_perm(q.y, q.x, 0x05010400u), b = __builtin_amdgcn_perm(q.y, q.x, 0x07030602u);
+    const uint32_t c = __builtin_amdgcn_perm(q.w, q.z, 0x05010400u), d = __builtin_amdgcn_perm(q.w, q.z, 0x07030602u);
+    return make_uint4(__builtin_amdgcn_perm(c, a, 0x05040100u), __builtin_amdgcn_perm(c, a, 0x07060302u),
+                      __builtin_amdgcn_perm(d, b, 0x05040100u), __builtin_amdgcn_perm(d, b, 0x07060302u));
+}
+
+// One-token projections from the fp32 row: a workgroup of FW waves quantizes
+// the row itself, a 16-lane group a block, and its waves then share it.  The
+// quantizer as a kernel of its own costs a launch (about 3 us of host time
+// and 4 us on the device before the weights are asked for); repeated by every
+// workgroup it is 120 VALU instructions a wave per 4 blocks, behind the
+// weights' loads.
+constexpr int FW = 4;
+
+// A thread's values of blocks grp, grp + 16, .. (16 FW / 4 blocks a pass): the
+// first pass's loads, issued before the weights'.
+struct RowLoads { float4 f[4]; };
+__device__ __forceinline__ void row_load(RowLoads& r, const float* __restrict__ x, int b, int nb) {
+    const float4* src = reinterpret_cast<const float4*>(x + (size_t)min(b, nb - 1) * QK + 16 * (threadIdx.x & 15));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.f[i] = src[i];
+}
+template <bool TRANSPOSE>
+__device__ __forceinline__ void quantize_row(RowLoads& r, const float* __restrict__ x, int nb, uint32_t* q8s);
+
 // Q8K.QuantizeRow / ScaleBlock (Q8K.cs:12-146), four 256-value blocks of one
 // token per wave: a 16-lane group per block, 16 consecutive values a lane (so
 // a lane's values are exactly one bsums group).  amax = max |x|; the scale's
@@ -100,6 +128,26 @@ __global__ __launch_bounds__(kWave) void q8k_quantize(const float* __restrict__ 
         v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
     }
     q8k_from16(v, lane, b < nb ? q8 + ((size_t)t * nb + b) * Q8K_WORDS : nullptr);
+}
+
+template <bool TRANSPOSE>
+__device__ __forceinline__ void quantize_row(RowLoads& r, const float* __restrict__ x, int nb, uint32_t* q8s) {
+    const int grp = threadIdx.x >> 4, li = threadIdx.x & 15;
+    for (int b0 = 0; b0 < nb; b0 += 4 * FW) {
+        const int b = b0 + grp;
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[4 * i] = r.f[i].x; v[4 * i + 1] = r.f[i].y; v[4 * i + 2] = r.f[i].z; v[4 * i + 3] = r.f[i].w;
+        }
+        if (b0 + 4 * FW < nb) row_load(r, x, b + 4 * FW, nb);
+        uint32_t* blk = b < nb ? q8s + b * Q8K_WORDS : nullptr;
+        q8k_from16(v, threadIdx.x & 63, blk);
+        if (TRANSPOSE && blk) {
+            uint4* q = reinterpret_cast<uint4*>(blk + Q8K_QS + 4 * li);
+            *q = byte_transpose(*q);
+        }
+    }
 }
 
 // VecDotQ4K.HorizontalSum (VecDotQ4K.cs:145-151).
@@ -226,26 +274,38 @@ __device__ __forceinline__ void q6k_block_lanes(const uint32_t* __restrict__ bas
 __host__ __device__ constexpr int lq_wchunks(int qtype, int rows, int nb, int bytes) {
     return qtype == 4 ? 0 : (rows * nb * bytes + 31) / 16 + 1;
 }
+// 16-byte pieces of LDS of one wave (beside the token's row).
+__host__ __device__ constexpr int lq_wave_chunks(int qtype, int rows, int nb, int bytes) {
+    return lq_wchunks(qtype, rows, nb, bytes) + (LQ_THREADS * LANES_LD + LQ_MAX_ROWS * 12) / 4;
+}
 
 // NB > 0 fixes the blocks per row at compile time (n_in = 256 NB), so the
 // fp32 pass unrolls and issues its LDS reads together; NB = 0 is generic.
-template <int QT, int NB>
-__global__ __launch_bounds__(LQ_THREADS) void linear_q(const unsigned char* __restrict__ w,
-                                                       const uint32_t* __restrict__ q8,
+// FUSED: one token from the fp32 row x (q8 unused), FW waves of rows_per_wg
+// rows; else one wave and tok_per_wg tokens.
+template <int QT, int NB, bool FUSED>
+__global__ __launch_bounds__(FUSED ? FW * LQ_THREADS : LQ_THREADS) void linear_q(const unsigned char* __restrict__ w,
+                                                       const uint32_t* __restrict__ q8, const float* __restrict__ x,
                                                        float* __restrict__ y, int n_in, int n_out,
                                                        int tokens, int rows_per_wg, int row_base, int tok_per_wg) {
 #pragma clang fp contract(off)
     constexpr int BB = QT == 4 ? Q4K_BYTES : Q6K_BYTES;
     constexpr int NL = QT == 4 ? 12 : 8;          // integer lanes per block
     extern __shared__ uint4 smem[];
-    const int nb = NB > 0 ? NB : n_in / QK, lane = threadIdx.x;
-    const int row0 = row_base + blockIdx.x * rows_per_wg;
-    const int nrows = min(rows_per_wg, n_out - row0);
+    const int nb = NB > 0 ? NB : n_in / QK, lane = threadIdx.x & 63;
+    const int wave = FUSED ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    // A wave past the last row (FUSED) reads it and stores nothing.
+    const int first = row_base + (blockIdx.x * (FUSED ? FW : 1) + wave) * rows_per_wg;
+    const int row0 = min(first, n_out - 1);
+    const int nrows = first < n_out ? min(rows_per_wg, n_out - row0) : 0;
     const int nblk = nrows * nb;
-    uint4* wsh = smem;
-    uint32_t* q8s = reinterpret_cast<uint32_t*>(smem + lq_wchunks(QT, rows_per_wg, nb, BB));
-    int* lanes = reinterpret_cast<int*>(q8s + nb * Q8K_WORDS);
+    // The token's Q8_K row, then each wave's weights (Q6_K), lanes and sums.
+    uint32_t* q8s = reinterpret_cast<uint32_t*>(smem);
+    uint4* wsh = smem + nb * (Q8K_WORDS / 4) + wave * lq_wave_chunks(QT, rows_per_wg, nb, BB);
+    int* lanes = reinterpret_cast<int*>(wsh + lq_wchunks(QT, rows_per_wg, nb, BB));
     float* accs = reinterpret_cast<float*>(lanes + LQ_THREADS * LANES_LD);
+    RowLoads rl;
+    if constexpr (FUSED) row_load(rl, x, threadIdx.x >> 4, nb);
 
     // Q4_K: each thread loads its block (16-byte aligned, 144 B) straight
     // into registers.  Q6_K blocks are 2-byte aligned: the workgroup's rows,
@@ -256,7 +316,7 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_q(const unsigned char* __re
     const uint32_t* wbase = reinterpret_cast<const uint32_t*>(wsh);
     int shift = 0;
     if constexpr (QT == 4) {
-        const uint4* src = reinterpret_cast<const uint4*>(w + ((size_t)row0 * nb + min(lane, nblk - 1)) * BB);
+        const uint4* src = reinterpret_cast<const uint4*>(w + ((size_t)row0 * nb + max(min(lane, nblk - 1), 0)) * BB);
 #pragma unroll
         for (int c = 0; c < Q4K_BYTES / 16; ++c) wreg[c] = src[c];
     } else {
@@ -292,9 +352,11 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_q(const unsigned char* __re
         }
     }
 
-    const int t_end = min(tokens, ((int)blockIdx.y + 1) * tok_per_wg);
-    for (int t = blockIdx.y * tok_per_wg; t < t_end; ++t) {
-        {
+    const int t_end = FUSED ? 1 : min(tokens, ((int)blockIdx.y + 1) * tok_per_wg);
+    for (int t = FUSED ? 0 : blockIdx.y * tok_per_wg; t < t_end; ++t) {
+        if constexpr (FUSED) {
+            quantize_row<false>(rl, x, nb, q8s);
+        } else {
             // The token's Q8_K row, nb x 19 16-byte chunks, 8 loads a lane in flight.
             const uint4* src = reinterpret_cast<const uint4*>(q8 + (size_t)t * nb * Q8K_WORDS);
             uint4* dst = reinterpret_cast<uint4*>(q8s);
@@ -311,7 +373,7 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_q(const unsigned char* __re
                     if (i0 + lane + LQ_THREADS * c < n4) dst[i0 + lane + LQ_THREADS * c] = qv[c];
             }
         }
-        __syncthreads();
+        lds_barrier();
         if (lane < nblk) {
             const uint32_t* q8b = q8s + (lane % nb) * Q8K_WORDS;
             int* out = lanes + lane * LANES_LD;
@@ -332,7 +394,7 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_q(const unsigned char* __re
                 out[8] = (int)(lds_word(wbase, shift + lane * BB + 208) & 0xffff);   // d of the block
             }
         }
-        __syncthreads();
+        lds_barrier();
         // Row r's lane k: one FMA per block in block order (and, for Q4_K,
         // lanes 0..3 also run the min term's multiply-add).
         const int r = lane >> 3, k = lane & 7;
@@ -357,7 +419,7 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_q(const unsigned char* __re
             accs[r * NL + k] = acc;
             if (QT == 4 && k < 4) accs[r * NL + 8 + k] = accm;
         }
-        __syncthreads();
+        lds_barrier();
         if (lane < nrows) {
             const float* a = accs + lane * NL;
             const float h[8] = {a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7]};
@@ -365,7 +427,7 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_q(const unsigned char* __re
             if constexpr (QT == 4) o = o + ((a[8] + a[10]) + (a[9] + a[11]));
             y[(size_t)t * n_out + row0 + lane] = o;
         }
-        __syncthreads();
+        lds_barrier();
     }
 }
 
@@ -458,29 +520,32 @@ __device__ __forceinline__ void iq4xs_block_terms(const uint32_t* __restrict__ w
     }
 }
 
-// One token: one 64-thread workgroup per group of up to 8 whole rows (at most
-// 64 blocks, a block a thread, held in registers).  The token's Q8_K row is
-// staged in LDS, every thread forms its block's integer terms, and one thread
+// One token: a wave per group of up to 8 whole rows (at most 64 blocks, a
+// block a thread, held in registers); one wave a workgroup, or FW with FUSED
+// (see linear_q).  The token's Q8_K row is staged or formed in LDS, every thread forms its block's integer terms, and one thread
 // per row runs the reference's fp32 chain over the row's blocks in order.
-template <int QT>
-__global__ __launch_bounds__(LQ_THREADS) void linear_qs(const unsigned char* __restrict__ w,
-                                                        const uint32_t* __restrict__ q8,
+template <int QT, bool FUSED>
+__global__ __launch_bounds__(FUSED ? FW * LQ_THREADS : LQ_THREADS) void linear_qs(const unsigned char* __restrict__ w,
+                                                        const uint32_t* __restrict__ q8, const float* __restrict__ x,
                                                         float* __restrict__ y, int n_in, int n_out, int rows_per_wg) {
 #pragma clang fp contract(off)
     constexpr int BB = QT == 5 ? Q5K_BYTES : IQ4XS_BYTES;
     extern __shared__ uint4 smem[];
-    const int nb = n_in / QK, lane = threadIdx.x;
-    const int row0 = blockIdx.x * rows_per_wg;
-    const int nrows = min(rows_per_wg, n_out - row0);
+    const int nb = n_in / QK, lane = threadIdx.x & 63;
+    const int wave = FUSED ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    const int first = (blockIdx.x * (FUSED ? FW : 1) + wave) * rows_per_wg, row0 = min(first, n_out - 1);
+    const int nrows = first < n_out ? min(rows_per_wg, n_out - row0) : 0;
     const int nblk = nrows * nb;
     uint32_t* q8s = reinterpret_cast<uint32_t*>(smem);
-    float* terms = reinterpret_cast<float*>(q8s + nb * Q8K_WORDS);
+    float* terms = reinterpret_cast<float*>(q8s + nb * Q8K_WORDS) + wave * LQ_THREADS * QS_TLD;
+    RowLoads rl;
+    if constexpr (FUSED) row_load(rl, x, threadIdx.x >> 4, nb);
 
     // The thread's block straight into registers (Q5_K blocks are 16-byte
     // multiples, IQ4_XS blocks 8-byte multiples from a 16-byte aligned base).
     uint32_t wb[BB / 4];
     {
-        const unsigned char* src = w + ((size_t)row0 * nb + min(lane, nblk - 1)) * BB;
+        const unsigned char* src = w + ((size_t)row0 * nb + max(min(lane, nblk - 1), 0)) * BB;
         if constexpr (QT == 5) {
 #pragma unroll
             for (int c = 0; c < BB / 16; ++c) reinterpret_cast<uint4*>(wb)[c] = reinterpret_cast<const uint4*>(src)[c];
@@ -489,7 +554,9 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qs(const unsigned char* __r
             for (int c = 0; c < BB / 8; ++c) reinterpret_cast<uint2*>(wb)[c] = reinterpret_cast<const uint2*>(src)[c];
         }
     }
-    {
+    if constexpr (FUSED) {
+        quantize_row<false>(rl, x, nb, q8s);
+    } else {
         const uint4* src = reinterpret_cast<const uint4*>(q8);
         uint4* dst = reinterpret_cast<uint4*>(q8s);
         const int n4 = nb * (Q8K_WORDS / 4);
@@ -505,7 +572,7 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qs(const unsigned char* __r
                 if (i0 + lane + LQ_THREADS * c < n4) dst[i0 + lane + LQ_THREADS * c] = qv[c];
         }
     }
-    __syncthreads();
+    lds_barrier();
     // Each thread forms its block's terms of the reference's chain (they do
     // not depend on the running sum); one thread per row then adds them in
     // order.
@@ -533,7 +600,7 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qs(const unsigned char* __r
             }
         }
     }
-    __syncthreads();
+    lds_barrier();
     if (lane < nrows) {
         constexpr int NTERM = QT == 5 ? 1 : 8;
         float sumf = 0.0f;
@@ -563,16 +630,6 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qs(const unsigned char* __r
 // other rows, Q2_0C.DotAvx2 (Q2_0C.cs:67-79): acc += dw * ((float)T0 * dx0
 // + (float)T1 * dx1) per 512 values, and STQ1_0.DotAvx2 (STQ1_0.cs:120-138):
 // acc += (dw * dx) * (float)T.  Rows below panel_rows take the panel order.
-
-// Bytes k of the four dwords q[0..3] gathered into dword k (a 4 x 4 byte
-// transpose): Q2_0C's byte c of a qs dword holds values 4c .. 4c + 3, so its
-// bit pair k of every byte meets the activations 16 i + 4c + k.
-__device__ __forceinline__ uint4 byte_transpose(uint4 q) {
-    const uint32_t a = __builtin_amdgcn_perm(q.y, q.x, 0x05010400u), b = __builtin_amdgcn_perm(q.y, q.x, 0x07030602u);
-    const uint32_t c = __builtin_amdgcn_perm(q.w, q.z, 0x05010400u), d = __builtin_amdgcn_perm(q.w, q.z, 0x07030602u);
-    return make_uint4(__builtin_amdgcn_perm(c, a, 0x05040100u), __builtin_amdgcn_perm(c, a, 0x07060302u),
-                      __builtin_amdgcn_perm(d, b, 0x05040100u), __builtin_amdgcn_perm(d, b, 0x07060302u));
-}
 
 // Sum of a Q8_K block's 16 bsums (the workspace form).
 __device__ __forceinline__ int q8k_bsum_total(const uint32_t* __restrict__ q8b) {
@@ -640,29 +697,32 @@ __device__ __forceinline__ int stq_unit_dot(const uint32_t* __restrict__ base, i
     return enc - q8k_bsum_total(q8b);
 }
 
-// One token: one 64-thread workgroup per group of up to 8 whole rows (at most
-// 64 units, one a thread): the rows' contiguous weight bytes are staged in LDS
+// One token: a wave per group of up to 8 whole rows (at most 64 units, one a
+// thread), one wave a workgroup, or FW with FUSED (see linear_q): the rows' contiguous weight bytes are staged in LDS
 // (as for Q6_K) and the token's Q8_K row, every thread forms its unit's T, and
 // one thread per row runs the chain.
-template <int QT>
-__global__ __launch_bounds__(LQ_THREADS) void linear_qt(const unsigned char* __restrict__ w,
-                                                        const uint32_t* __restrict__ q8,
+template <int QT, bool FUSED>
+__global__ __launch_bounds__(FUSED ? FW * LQ_THREADS : LQ_THREADS) void linear_qt(const unsigned char* __restrict__ w,
+                                                        const uint32_t* __restrict__ q8, const float* __restrict__ x,
                                                         float* __restrict__ y, int n_in, int n_out,
                                                         int rows_per_wg, int panel_rows) {
 #pragma clang fp contract(off)
     constexpr int UB = QT == 2 ? Q2_BYTES / 2 : STQ_BYTES;   // weight bytes per unit
     extern __shared__ uint4 smem[];
-    const int nb = n_in / QK, lane = threadIdx.x;
-    const int row0 = blockIdx.x * rows_per_wg;
-    const int nrows = min(rows_per_wg, n_out - row0);
+    const int nb = n_in / QK, lane = threadIdx.x & 63;
+    const int wave = FUSED ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    const int first = (blockIdx.x * (FUSED ? FW : 1) + wave) * rows_per_wg, row0 = min(first, n_out - 1);
+    const int nrows = first < n_out ? min(rows_per_wg, n_out - row0) : 0;
     const int nunit = nrows * nb;
     const size_t row_bytes = (size_t)nb * UB;
     const int nchunk_max = (rows_per_wg * nb * UB + 31) / 16 + 1;
-    uint4* wsh = smem;
-    uint32_t* q8s = reinterpret_cast<uint32_t*>(smem + nchunk_max);
-    int* tv = reinterpret_cast<int*>(q8s + nb * Q8K_WORDS);
+    uint32_t* q8s = reinterpret_cast<uint32_t*>(smem);
+    uint4* wsh = smem + nb * (Q8K_WORDS / 4) + wave * (nchunk_max + LQ_THREADS / 4);
+    int* tv = reinterpret_cast<int*>(wsh + nchunk_max);
     const uint32_t* wbase = reinterpret_cast<const uint32_t*>(wsh);
 
+    RowLoads rl;
+    if constexpr (FUSED) row_load(rl, x, threadIdx.x >> 4, nb);
     // The rows' bytes from the 16-byte boundary below their even start; only
     // the buffer's last chunk can be partial, read with 2-byte loads.
     const size_t total = (size_t)n_out * row_bytes;
@@ -697,7 +757,9 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qt(const unsigned char* __r
         }
     }
 
-    {
+    if constexpr (FUSED) {
+        quantize_row<QT == 2>(rl, x, nb, q8s);
+    } else {
         const uint4* src = reinterpret_cast<const uint4*>(q8);
         uint4* dst = reinterpret_cast<uint4*>(q8s);
         const int n4 = nb * (Q8K_WORDS / 4);
@@ -718,7 +780,7 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qt(const unsigned char* __r
             }
         }
     }
-    __syncthreads();
+    lds_barrier();
     if (lane < nunit) {
         const int r = lane / nb, b = lane % nb;
         const uint32_t* q8b = q8s + b * Q8K_WORDS;
@@ -727,7 +789,7 @@ __global__ __launch_bounds__(LQ_THREADS) void linear_qt(const unsigned char* __r
         else
             tv[lane] = stq_unit_dot(wbase, shift + (int)(r * row_bytes) + b * STQ_BYTES, q8b);
     }
-    __syncthreads();
+    lds_barrier();
     if (lane < nrows) {
         const int row = row0 + lane;
         const int* T = tv + lane * nb;
@@ -861,10 +923,7 @@ __global__ __launch_bounds__(256) void linear_f32(const float* __restrict__ w, c
                 i += 8;
             }
             // acc0 + acc1, then HorizontalSum: (s_k + s_{k+4}) pairs, (0 + 2) + (1 + 3).
-            s = s + __shfl_xor(s, 8, kWave);
-            s = s + __shfl_xor(s, 4, kWave);
-            s = s + __shfl_xor(s, 2, kWave);
-            s = s + __shfl_xor(s, 1, kWave);
+            s = row_sum(s);
             for (; i < n_in; ++i) s += a[i] * b[i];
             if (l16 == 0 && gt < GT && row < n_out && tok < tokens) y[(size_t)tok * n_out + row] = s;
         }
@@ -1514,7 +1573,7 @@ __global__ __launch_bounds__(kWave) void add_rmsnorm(float* hidden, const float*
         }
     float a[8];
 #pragma unroll
-    for (int l = 0; l < 8; ++l) a[l] = __shfl(acc, l, kWave);
+    for (int l = 0; l < 8; ++l) a[l] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane(__float_as_uint(acc), l));
     float sum = hsum8(a);
     for (int i = dim & ~7; i < dim; ++i) {
         const float sq = row[i] * row[i];
@@ -1570,47 +1629,63 @@ hipError_t launch_q8k_quantize(q35m_ctx* c, const float* x, void* q8, int n_in, 
     return hipGetLastError();
 }
 
+// The one-token kernels, from the Q8_K row q8 or (q8 null) the fp32 row x; also
+// rows from row_base on of several tokens of Q4_K and Q6_K, tok_per_wg a
+// workgroup.
+static hipError_t launch_gemv(q35m_ctx* c, int qtype, const unsigned char* w, const uint32_t* q8, const float* x, float* y,
+                              int n_in, int n_out, int tokens, int row_base, int tok_per_wg) {
+    const int nb = n_in / QK, rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS), waves = q8 ? 1 : FW;
+    const dim3 grid(((n_out - row_base + rows_per_wg - 1) / rows_per_wg + waves - 1) / waves,
+                    (tokens + tok_per_wg - 1) / tok_per_wg);
+    const dim3 block(LQ_THREADS * waves);
+    const size_t row_lds = (size_t)nb * Q8K_WORDS * 4;
+    auto go = [&](auto kern, int kid, size_t wave_lds, auto... args) {
+        ProfScope ps_(c, kid);
+        hipExtLaunchKernelGGL(kern, grid, block, row_lds + waves * wave_lds, c->stream, ps_.a, ps_.b, 0, w, q8, x, y, n_in,
+                              n_out, args...);
+        return hipGetLastError();
+    };
+    if (qtype == 1 || qtype == 2) {
+        // Eight-row panels (see launch_linear_q_prequant) of one token.
+        const int ub = qtype == 2 ? Q2_BYTES / 2 : STQ_BYTES;
+        const size_t lds = 16 * (size_t)((rows_per_wg * nb * ub + 31) / 16 + 1) + LQ_THREADS * 4;
+        const int kid = qtype == 2 ? K_Q2_0C_LINEAR : K_STQ1_0_LINEAR, panel_rows = n_out & ~7;
+        if (qtype == 2) return go(q8 ? linear_qt<2, false> : linear_qt<2, true>, kid, lds, rows_per_wg, panel_rows);
+        return go(q8 ? linear_qt<1, false> : linear_qt<1, true>, kid, lds, rows_per_wg, panel_rows);
+    }
+    if (qtype == 5 || qtype == 14) {
+        const size_t lds = (size_t)LQ_THREADS * QS_TLD * 4;
+        if (qtype == 5) return go(q8 ? linear_qs<5, false> : linear_qs<5, true>, K_Q5K_LINEAR, lds, rows_per_wg);
+        return go(q8 ? linear_qs<14, false> : linear_qs<14, true>, K_IQ4XS_LINEAR, lds, rows_per_wg);
+    }
+    const int bb = qtype == 4 ? Q4K_BYTES : Q6K_BYTES;
+    const size_t lds = 16 * (size_t)lq_wave_chunks(qtype, rows_per_wg, nb, bb);
+    auto pick = [&](auto k10, auto k16, auto k0, int kid) {
+        return go(nb == 10 ? k10 : nb == 16 ? k16 : k0, kid, lds, tokens, rows_per_wg, row_base, tok_per_wg);
+    };
+    if (qtype == 4)
+        return q8 ? pick(linear_q<4, 10, false>, linear_q<4, 16, false>, linear_q<4, 0, false>, K_Q4K_LINEAR)
+                  : pick(linear_q<4, 10, true>, linear_q<4, 16, true>, linear_q<4, 0, true>, K_Q4K_LINEAR);
+    return q8 ? pick(linear_q<6, 10, false>, linear_q<6, 16, false>, linear_q<6, 0, false>, K_Q6K_LINEAR)
+              : pick(linear_q<6, 10, true>, linear_q<6, 16, true>, linear_q<6, 0, true>, K_Q6K_LINEAR);
+}
+
 hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const void* q8, float* y,
                                     int n_in, int n_out, int tokens) {
     const int nb = n_in / QK;
     const unsigned char* wb = reinterpret_cast<const unsigned char*>(w);
     const uint32_t* qb = reinterpret_cast<const uint32_t*>(q8);
+    if (tokens == 1) return launch_gemv(c, qtype, wb, qb, nullptr, y, n_in, n_out, 1, 0, 1);
     if (qtype == 1 || qtype == 2) {
         // Which rows take the eight-row panel order (MulMatQ2.cs:25-40,
         // MulMatSTQ.cs:25-64): the first n_out & ~7, except STQ1_0 with
         // several tokens: all rows when tokens % 4 == 0 and n_out % 8 == 0,
         // else none.
         int panel_rows = n_out & ~7;
-        if (qtype == 1 && tokens > 1) panel_rows = ((tokens & 3) == 0 && (n_out & 7) == 0) ? n_out : 0;
-        if (tokens >= 2) return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, n_out, tokens, panel_rows);
-        const int rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
-        const int ub = qtype == 2 ? Q2_BYTES / 2 : STQ_BYTES;
-        const int nchunk_max = (rows_per_wg * nb * ub + 31) / 16 + 1;
-        const dim3 grid((n_out + rows_per_wg - 1) / rows_per_wg);
-        const size_t lds = 16 * (size_t)nchunk_max + (size_t)nb * Q8K_WORDS * 4 + (size_t)LQ_THREADS * 4;
-        ProfScope ps_(c, qtype == 2 ? K_Q2_0C_LINEAR : K_STQ1_0_LINEAR);
-        if (qtype == 2)
-            hipExtLaunchKernelGGL(linear_qt<2>, grid, dim3(LQ_THREADS), lds, c->stream, ps_.a, ps_.b, 0, wb, qb, y,
-                                  n_in, n_out, rows_per_wg, panel_rows);
-        else
-            hipExtLaunchKernelGGL(linear_qt<1>, grid, dim3(LQ_THREADS), lds, c->stream, ps_.a, ps_.b, 0, wb, qb, y,
-                                  n_in, n_out, rows_per_wg, panel_rows);
-        return hipGetLastError();
+        if (qtype == 1) panel_rows = ((tokens & 3) == 0 && (n_out & 7) == 0) ? n_out : 0;
+        return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, n_out, tokens, panel_rows);
     }
-    if (qtype == 5 || qtype == 14) {
-        if (tokens >= 2) return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, n_out, tokens, 0);
-        const int rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
-        const dim3 grid((n_out + rows_per_wg - 1) / rows_per_wg);
-        const size_t lds = (size_t)nb * Q8K_WORDS * 4 + (size_t)LQ_THREADS * QS_TLD * 4;
-        ProfScope ps_(c, qtype == 5 ? K_Q5K_LINEAR : K_IQ4XS_LINEAR);
-        if (qtype == 5)
-            hipExtLaunchKernelGGL(linear_qs<5>, grid, dim3(LQ_THREADS), lds, c->stream, ps_.a, ps_.b, 0, wb, qb, y,
-                                  n_in, n_out, rows_per_wg);
-        else
-            hipExtLaunchKernelGGL(linear_qs<14>, grid, dim3(LQ_THREADS), lds, c->stream, ps_.a, ps_.b, 0, wb, qb, y,
-                                  n_in, n_out, rows_per_wg);
-        return hipGetLastError();
-    }
+    if (qtype == 5 || qtype == 14) return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, n_out, tokens, 0);
     // The tiled kernels address their operands through buffer descriptors
     // (32-bit offsets): calls with more than 2 GiB of weight rows or of
     // activations go in pieces of whole row and token tiles (even rows), each
@@ -1640,56 +1715,49 @@ hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const
     // the end of it.
     const int rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
     int row_base = 0;
-    if (tokens > 1) {
-        // The GEMV takes a few tokens while its workgroups fit the CUs about
-        // once; the matrix cores the rest: linear_gemm's small tiles while they
-        // are few, else 64-token tiles.  Measured (us; GEMV / small / 64-token
-        // tiles): Q6_K 4096 -> 2560 at 2 tokens 6.8 / 12 / 29, at 4 9.8 / 12 /
-        // 29, at 8 17 / 12 / 29, at 32 - / 22 / 29; 2560 -> 8192 at 2 11 / 16.5
-        // / 20, at 16 - / 16.5 / 20, at 32 - / 36 / 20; 2560 -> 1024 at 4 6.0 /
-        // 9.3 / 19, at 16 10.4 / 9.5 / 19 (a workgroup's tokens one after the
-        // other: 11.6 at 4, 47 at 15 of 2560 -> 8192).  Q4_K (GEMV order in no
-        // whole panel: small tiles / 64-token tiles) 2560 -> 8192 at 8 9.1 / 30,
-        // at 128 19 / 32, at 256 27 / 32, at 500 49 / 44.
-        const long groups = (n_out + rows_per_wg - 1) / rows_per_wg;
-        const long tiles = (long)((n_out + 15) / 16) * ((tokens + 15) / 16);
-        if (qtype == 4) {
-            row_base = n_out & ~7;
-        } else if (c->proj_order == Q35M_PROJ_BLOCK && tokens >= 16 && (((size_t)n_out * nb) & 1) == 0) {
-            return tiled(q6k_gemm_blk, K_Q6K_GEMM_BLK, Q6K_BYTES, BR, BT, BTHREADS, n_out);
-        } else if (groups * tokens > 4000 || tokens > 16) {
-            row_base = n_out - (int)(((size_t)n_out * nb) & 1);
-        }
-        hipError_t e = hipSuccess;
-        if (row_base > 0) {
-            const bool small = qtype == 4 ? tiles <= 8192 : tiles * nb <= 5120;
-            if (small) e = launch_linear_gemm(c, qtype, w, q8, y, n_in, row_base, n_out, tokens, 0);
-            else if (qtype == 4) e = tiled(q4k_gemm, K_Q4K_GEMM, Q4K_BYTES, GR, GT, GTHREADS, row_base);
-            else e = tiled(q6k_gemm, K_Q6K_GEMM, Q6K_BYTES, SGR, SGT, 256, row_base);
-        }
-        if (e != hipSuccess || row_base == n_out) return e;
+    // The GEMV takes a few tokens while its workgroups fit the CUs about
+    // once; the matrix cores the rest: linear_gemm's small tiles while they
+    // are few, else 64-token tiles.  Measured (us; GEMV / small / 64-token
+    // tiles): Q6_K 4096 -> 2560 at 2 tokens 6.8 / 12 / 29, at 4 9.8 / 12 /
+    // 29, at 8 17 / 12 / 29, at 32 - / 22 / 29; 2560 -> 8192 at 2 11 / 16.5
+    // / 20, at 16 - / 16.5 / 20, at 32 - / 36 / 20; 2560 -> 1024 at 4 6.0 /
+    // 9.3 / 19, at 16 10.4 / 9.5 / 19 (a workgroup's tokens one after the
+    // other: 11.6 at 4, 47 at 15 of 2560 -> 8192).  Q4_K (GEMV order in no
+    // whole panel: small tiles / 64-token tiles) 2560 -> 8192 at 8 9.1 / 30,
+    // at 128 19 / 32, at 256 27 / 32, at 500 49 / 44.
+    const long groups = (n_out + rows_per_wg - 1) / rows_per_wg;
+    const long tiles = (long)((n_out + 15) / 16) * ((tokens + 15) / 16);
+    if (qtype == 4) {
+        row_base = n_out & ~7;
+    } else if (c->proj_order == Q35M_PROJ_BLOCK && tokens >= 16 && (((size_t)n_out * nb) & 1) == 0) {
+        return tiled(q6k_gemm_blk, K_Q6K_GEMM_BLK, Q6K_BYTES, BR, BT, BTHREADS, n_out);
+    } else if (groups * tokens > 4000 || tokens > 16) {
+        row_base = n_out - (int)(((size_t)n_out * nb) & 1);
     }
+    hipError_t e = hipSuccess;
+    if (row_base > 0) {
+        const bool small = qtype == 4 ? tiles <= 8192 : tiles * nb <= 5120;
+        if (small) e = launch_linear_gemm(c, qtype, w, q8, y, n_in, row_base, n_out, tokens, 0);
+        else if (qtype == 4) e = tiled(q4k_gemm, K_Q4K_GEMM, Q4K_BYTES, GR, GT, GTHREADS, row_base);
+        else e = tiled(q6k_gemm, K_Q6K_GEMM, Q6K_BYTES, SGR, SGT, 256, row_base);
+    }
+    if (e != hipSuccess || row_base == n_out) return e;
     // Tokens a workgroup: one while the workgroups fit the CUs about once (a
     // tiled call's last rows, many tokens of few rows, took 0.75 us a token).
     const int grid = (n_out - row_base + rows_per_wg - 1) / rows_per_wg;
     const int tok_per_wg = (int)(((long)tokens * grid + 1499) / 1500);
-    const int bb = qtype == 4 ? Q4K_BYTES : Q6K_BYTES;
-    const size_t lds = 16 * (size_t)lq_wchunks(qtype, rows_per_wg, nb, bb) + (size_t)nb * Q8K_WORDS * 4 +
-                       (size_t)LQ_THREADS * LANES_LD * 4 + (size_t)LQ_MAX_ROWS * 12 * 4;
-    auto launch = [&](auto kern, int kid) {
-        ProfScope ps_(c, kid);
-        hipExtLaunchKernelGGL(kern, dim3(grid, (tokens + tok_per_wg - 1) / tok_per_wg), dim3(LQ_THREADS), lds, c->stream,
-                              ps_.a, ps_.b, 0, wb, qb, y, n_in, n_out, tokens, rows_per_wg, row_base, tok_per_wg);
-    };
-    if (qtype == 4)
-        launch(nb == 10 ? linear_q<4, 10> : nb == 16 ? linear_q<4, 16> : linear_q<4, 0>, K_Q4K_LINEAR);
-    else
-        launch(nb == 10 ? linear_q<6, 10> : nb == 16 ? linear_q<6, 16> : linear_q<6, 0>, K_Q6K_LINEAR);
-    return hipGetLastError();
+    return launch_gemv(c, qtype, wb, qb, nullptr, y, n_in, n_out, tokens, row_base, tok_per_wg);
 }
+
+// One token of Q6_K keeps the quantizer apart where the row and four waves'
+// weights would leave one workgroup a CU (29.8 against 27.5 us at 16384 ->
+// 2560; Q4_K, whose weights are in registers, 19.5 against 23.2).
+bool linear_q_fused(int qtype, int n_in, int tokens) { return tokens == 1 && !(qtype == 6 && n_in > 40 * QK); }
 
 hipError_t launch_linear_q(q35m_ctx* c, int qtype, const void* w, const float* x, float* y,
                            int n_in, int n_out, int tokens) {
+    if (linear_q_fused(qtype, n_in, tokens))
+        return launch_gemv(c, qtype, reinterpret_cast<const unsigned char*>(w), nullptr, x, y, n_in, n_out, 1, 0, 1);
     hipError_t e = launch_q8k_quantize(c, x, c->work, n_in, tokens);
     if (e != hipSuccess) return e;
     return launch_linear_q_prequant(c, qtype, w, c->work, y, n_in, n_out, tokens);

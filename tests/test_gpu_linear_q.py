@@ -92,6 +92,28 @@ def test_linear_gemm_tiles(ctx, qtype, n_in, n_out, tokens):
 
 
 @pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("n_in,n_out", [(512, 1), (512, 33), (4096, 17), (4608, 129), (10240, 5), (10752, 9), (16384, 3)])
+def test_linear_q_one_token_quantizes(ctx, qtype, n_in, n_out):
+    """One token, the row quantized by the projection's own workgroups (four
+    waves of rows, a last one with waves past the end; one, two and four
+    passes of blocks), bit for bit, and the same as with the row quantized
+    before."""
+    rng = np.random.default_rng(11 * qtype + n_in + n_out)
+    w = qb.random_blocks(rng, qtype, qb.nblocks(qtype, n_out * n_in))
+    x = rng.standard_normal((1, n_in)).astype(np.float32)
+    x[0, 256:512] = 0.0
+    x[0, 40] = -x[0, 30]
+    got = run(ctx, qtype, w, x, n_in, n_out)
+    assert np.array_equal(got.view(np.uint32), oracle.linear_q(qtype, w, x, n_in, n_out).view(np.uint32))
+    dw, dx, dy = ctx.bytes_array(w), ctx.array((1, n_in), x), ctx.array((1, n_out))
+    q8 = ctx.quantize_q8k(dx, n_in, 1)
+    ctx.linear_q_prequant(qtype, dw, q8, dy, n_in, n_out, 1)
+    assert np.array_equal(dy.download().view(np.uint32), got.view(np.uint32))
+    for a in (dw, dx, dy, q8):
+        a.free()
+
+
+@pytest.mark.parametrize("qtype", TYPES)
 def test_linear_q_activation_edges(ctx, qtype):
     """Zero blocks (scale 0), a first extremum that is positive (negative
     scale) or repeated with both signs, ties at .5 after scaling, huge and tiny
