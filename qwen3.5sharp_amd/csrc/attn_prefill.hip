@@ -363,7 +363,7 @@ typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int ST = 32;                       // key rows a tile
 constexpr int SFRAGS = 64;                   // 1 KiB operand fragments a tile: 32 K, 32 V
-constexpr int SPREP = 256, SWAVES = 8;
+constexpr int SPREP = 512, SWAVES = 8;
 // Largest workspace the split form takes (a sequence's planes are as large as
 // its K and V rows); calls past it take the fp32 form.
 constexpr size_t kSplitMaxBytes = (size_t)2 << 30;
@@ -395,21 +395,24 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
 
 __device__ __forceinline__ float pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
 
-// Workgroup: one 32-row tile of one kv head.  Wave a holds its rows 4a .. 4a +
-// 3 and 16 + 4a .. + 3, the eight keys that lane group a of a V operand takes.
+// Workgroup: one 32-row tile of one kv head.  Wave a + 4 half holds its rows 16
+// half + 4a .. + 3, half of the eight keys that lane group a of a V operand
+// takes: 11.6 us for 2048 rows and 24.2 for 8133 (all eight rows in four
+// waves: 13.7 and 27.5).
 __global__ __launch_bounds__(SPREP) void attn_split_prep(
     const float* __restrict__ knew, const float* __restrict__ vnew, const float* __restrict__ k_norm, float* __restrict__ K,
     float* __restrict__ V, const float* __restrict__ rope_cos, const float* __restrict__ rope_sin,
     uint4* __restrict__ planes, TileMeta* __restrict__ meta, int start, int T, int nkv, int cap, float eps) {
     __shared__ uint4 frag[SFRAGS][64];
-    __shared__ uint32_t red[4][4];
-    const int lane = threadIdx.x & 63, a = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    __shared__ uint32_t red[8][4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int a = wave & 3, half = wave >> 2;
     const int len = start + T, ntile = (len + ST - 1) / ST;
     const int tile = blockIdx.x / nkv, kvh = blockIdx.x % nkv, kv_dim = nkv * kHd;
-    float4 kx[8], vx[8];
+    float4 kx[4], vx[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int p = ST * tile + (i < 4 ? 4 * a + i : 12 + 4 * a + i);
+    for (int i = 0; i < 4; ++i) {
+        const int p = ST * tile + 16 * half + 4 * a + i;
         const size_t row = ((size_t)kvh * cap + p) * kHd + 4 * lane;
         const size_t nrow = (size_t)(p - start) * kv_dim + kvh * kHd + 4 * lane;
         kx[i] = vx[i] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -421,8 +424,8 @@ __global__ __launch_bounds__(SPREP) void attn_split_prep(
     // Largest absolute value of the tile's K and V, smallest nonzero row's.
     uint32_t kmax = 0, vmax = 0, kmin = ~0u, vmin = ~0u;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int p = ST * tile + (i < 4 ? 4 * a + i : 12 + 4 * a + i);
+    for (int i = 0; i < 4; ++i) {
+        const int p = ST * tile + 16 * half + 4 * a + i;
         if (p >= start && p < len) {
             const size_t row = ((size_t)kvh * cap + p) * kHd + 4 * lane;
             kx[i] = rope_norm_row(kx[i], lane, rope_cos + (size_t)p * kRopeHalf, rope_sin + (size_t)p * kRopeHalf, k_norm,
@@ -438,11 +441,11 @@ __global__ __launch_bounds__(SPREP) void attn_split_prep(
         if (mv) vmin = min(vmin, mv);
     }
     if (lane == 0) {
-        red[a][0] = kmax; red[a][1] = vmax; red[a][2] = kmin; red[a][3] = vmin;
+        red[wave][0] = kmax; red[wave][1] = vmax; red[wave][2] = kmin; red[wave][3] = vmin;
     }
     __syncthreads();
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < 8; ++w) {
         kmax = max(kmax, red[w][0]);
         vmax = max(vmax, red[w][1]);
         kmin = min(kmin, red[w][2]);
@@ -459,8 +462,8 @@ __global__ __launch_bounds__(SPREP) void attn_split_prep(
     // wave g.  Slot c of a fragment sits at c ^ swz(fragment) in LDS (bank
     // spread of the stores below); the copy out undoes it.
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int c16 = i < 4 ? 4 * a + i : 4 * a + i - 4, half = i >> 2;
+    for (int i = 0; i < 4; ++i) {
+        const int c16 = 4 * a + i;
         const int step = lane >> 3, g = (lane >> 1) & 3;
         const float x[4] = {kx[i].x * ks, kx[i].y * ks, kx[i].z * ks, kx[i].w * ks};
         f16x4 hi, lo;
@@ -475,21 +478,21 @@ __global__ __launch_bounds__(SPREP) void attn_split_prep(
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        f16x8 hi, lo;
+        f16x4 hi, lo;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < 4; ++i) {
             const float x = (j == 0 ? vx[i].x : j == 1 ? vx[i].y : j == 2 ? vx[i].z : vx[i].w) * vs;
             hi[i] = (_Float16)x;
             lo[i] = (_Float16)(x - (float)hi[i]);
         }
         const int db = lane >> 2, f = 32 + 2 * db, c = (16 * a + 4 * (lane & 3) + j) ^ db;
-        *reinterpret_cast<f16x8*>(&frag[f][c]) = hi;
-        *reinterpret_cast<f16x8*>(&frag[f + 1][c]) = lo;
+        reinterpret_cast<f16x4*>(&frag[f][c])[half] = hi;
+        reinterpret_cast<f16x4*>(&frag[f + 1][c])[half] = lo;
     }
     __syncthreads();
     uint4* dst = planes + ((size_t)kvh * ntile + tile) * SFRAGS * 64;
 #pragma unroll 4
-    for (int f = a; f < SFRAGS; f += 4) dst[64 * f + lane] = frag[f][lane ^ (f < 32 ? (f >> 1) & 7 : (f >> 1) & 15)];
+    for (int f = wave; f < SFRAGS; f += 8) dst[64 * f + lane] = frag[f][lane ^ (f < 32 ? (f >> 1) & 7 : (f >> 1) & 15)];
 }
 
 // Shape of one split launch.  A query block's key tiles go in chunks of
@@ -728,14 +731,18 @@ __global__ __launch_bounds__(64 * SWAVES, 2) void attn_split_flash(
     // waves of a SIMD (w, w + 4) take them in opposite orders, so one's VALU
     // work and LDS waits run beside the other's MFMAs.
     Scores S = {};
+    // t1 hidden from the optimizer: where it sees that a step always stages the
+    // next tile, it waits for those loads before it reads the tile it has.
+    int te = t1;
+    asm volatile("" : "+s"(te));
     auto step = [&](int t, auto first, auto more, auto masked) {
         const TileMeta mt = meta[t];
         // K of tile t + 1 and V of tile t have landed and every wave is past
         // tile t - 1; the next ones go out.
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lds_barrier();
-        if (t + 2 < t1) stage_k(t + 2);
-        if (t + 1 < t1) stage_v(t + 1);
+        if (t + 2 < te) stage_k(t + 2);
+        if (t + 1 < te) stage_v(t + 1);
         const float sc = qdesc * mt.kdesc;
         float st[2][4];
 #pragma unroll
