@@ -34,6 +34,7 @@ import synth  # noqa: E402
 HBM_PEAK = 8.0e12          # B/s, MI355X datasheet
 FP32_PEAK = 157.3e12       # FLOP/s, MI355X dense fp32 (matrix = vector)
 INT8_PEAK = 5.0e15         # OP/s, MI355X dense int8 matrix
+F16_PEAK = 2.5e15        # dense fp16 MFMA
 NK, NV, DK = 16, 32, 128
 NH, NKV, HD = 16, 4, 256
 CONV_DIM = 2 * NK * DK + NV * DK
@@ -702,7 +703,7 @@ def main():
         ms, kt = bench_attn_prefill(K, W)
         workloads["attn_prefill_2048"] = {
             "tokens_per_s": 2048 / (ms / 1e3), "ms": ms,
-            "mfma_frac": ATTN_PREFILL_FLOP / (ms / 1e3) / FP32_PEAK,
+            "mfma_frac": 3 * ATTN_PREFILL_FLOP / (ms / 1e3) / F16_PEAK,    # three fp16 products each
             "kernels_ms": {k: v[0] for k, v in kt.items()}}
         if not args.no_cpu:
             tok_s_cpu, sec = cpu_baseline_attn_prefill(threads)
