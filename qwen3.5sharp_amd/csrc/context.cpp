@@ -634,7 +634,7 @@ static int linear_q(q35m_ctx* ctx, int qtype, const void* w, const float* x, flo
         return fail(Q35M_ERR_INVALID, "weights and input must be 16-byte aligned");
     if ((r = check_linear_dims(n_in, n_out, tokens))) return r;
     if ((r = check_linear_type(qtype, n_in))) return r;
-    if (!q35::linear_q_fused(qtype, n_in, tokens))
+    if (!q35::linear_q_fused(qtype, x, y, n_in, n_out, tokens))
         HIP_TRY(q35::ensure_work(ctx, q35::linear_q_work_bytes(n_in, tokens)), "workspace");
     HIP_TRY(q35::launch_linear_q(ctx, qtype, w, x, y, n_in, n_out, tokens), "linear_q");
     return Q35M_OK;

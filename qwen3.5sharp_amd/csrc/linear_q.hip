@@ -1752,11 +1752,16 @@ hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const
 // One token of Q6_K keeps the quantizer apart where the row and four waves'
 // weights would leave one workgroup a CU (29.8 against 27.5 us at 16384 ->
 // 2560; Q4_K, whose weights are in registers, 19.5 against 23.2).
-bool linear_q_fused(int qtype, int n_in, int tokens) { return tokens == 1 && !(qtype == 6 && n_in > 40 * QK); }
+bool linear_q_fused(int qtype, const float* x, const float* y, int n_in, int n_out, int tokens) {
+    // Every workgroup of the fused form reads all of x while others store y.
+    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
+    const bool apart = ya >= xa + (size_t)n_in * sizeof(float) || xa >= ya + (size_t)n_out * sizeof(float);
+    return tokens == 1 && apart && !(qtype == 6 && n_in > 40 * QK);
+}
 
 hipError_t launch_linear_q(q35m_ctx* c, int qtype, const void* w, const float* x, float* y,
                            int n_in, int n_out, int tokens) {
-    if (linear_q_fused(qtype, n_in, tokens))
+    if (linear_q_fused(qtype, x, y, n_in, n_out, tokens))
         return launch_gemv(c, qtype, reinterpret_cast<const unsigned char*>(w), nullptr, x, y, n_in, n_out, 1, 0, 1);
     hipError_t e = launch_q8k_quantize(c, x, c->work, n_in, tokens);
     if (e != hipSuccess) return e;

@@ -212,8 +212,9 @@ hipError_t launch_linear_gemm(q35m_ctx* c, int qtype, const void* w, const void*
 hipError_t launch_add_rmsnorm(q35m_ctx* c, float* hidden, const float* delta, const float* w, float* y, void* q8,
                               int dim, int tokens, float eps);
 size_t linear_q_work_bytes(int n_in, int tokens);
-// Whether the projection quantizes its row itself and needs no workspace.
-bool linear_q_fused(int qtype, int n_in, int tokens);
+// Whether the projection quantizes its row itself and needs no workspace (one
+// token, x and y apart: an in-place call quantizes first).
+bool linear_q_fused(int qtype, const float* x, const float* y, int n_in, int n_out, int tokens);
 hipError_t launch_linear_f32(q35m_ctx* c, const float* w, const float* x, float* y, int n_in, int n_out,
                              int tokens);
 hipError_t launch_q8k_quantize(q35m_ctx* c, const float* x, void* q8, int n_in, int tokens);

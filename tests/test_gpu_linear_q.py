@@ -114,6 +114,34 @@ def test_linear_q_one_token_quantizes(ctx, qtype, n_in, n_out):
 
 
 @pytest.mark.parametrize("qtype", TYPES)
+@pytest.mark.parametrize("shift", [0, 256, -256])
+def test_linear_q_one_token_in_place(ctx, qtype, shift):
+    """y on top of x, or partly over its end or its start (shift floats): the
+    row is quantized as a whole before anything is stored.  Buffers that only
+    touch are apart."""
+    n_in = n_out = 5120
+    rng = np.random.default_rng(77 + qtype)
+    w = qb.random_blocks(rng, qtype, qb.nblocks(qtype, n_out * n_in))
+    x = rng.standard_normal((1, n_in)).astype(np.float32)
+    want = oracle.linear_q(qtype, w, x, n_in, n_out)
+    dw, buf = ctx.bytes_array(w), ctx.array((3, n_in))
+    view = lambda at: q35mix.DeviceView(buf, at, (1, n_in))  # noqa: E731
+    for at, fused in ((n_in + shift, False), (2 * n_in, True), (0, True)):
+        host = np.zeros((3, n_in), np.float32)
+        host[1] = x
+        buf.upload(host)
+        ctx.profile(True)
+        ctx.linear_q(qtype, dw, view(n_in), view(at), n_in, n_out, 1)
+        ran = ctx.profile_read()
+        ctx.profile(False)
+        assert ("q8k_quantize" not in ran) == fused
+        got = buf.download().reshape(-1)[at:at + n_out]
+        assert np.array_equal(got.view(np.uint32), want.reshape(-1).view(np.uint32))
+    dw.free()
+    buf.free()
+
+
+@pytest.mark.parametrize("qtype", TYPES)
 def test_linear_q_activation_edges(ctx, qtype):
     """Zero blocks (scale 0), a first extremum that is positive (negative
     scale) or repeated with both signs, ties at .5 after scaling, huge and tiny
