@@ -32,6 +32,7 @@
 // accumulation on 8 threads, one per reference lane, in block order.  Extra
 // tokens reuse the staged weights.
 #include "common.h"
+#include "f32_stage.h"
 #include "q35mix_internal.h"
 #include "quant_layout.h"
 
@@ -847,15 +848,15 @@ __global__ __launch_bounds__(256) void linear_f32(const float* __restrict__ w, c
     const int row0 = blockIdx.x * RW, tok0 = blockIdx.y * TW;
     const int main = n_in & ~15;                  // columns of the 16-wide strides
 
-    // Unit e of the staging: tile row e / C4 (weight rows, then tokens; past
-    // the end the last one again), lane e % 16 of 64-column run (e % C4) / 16.
-    // Columns past `main` read its last one and are not used.
+    // Rows and tokens past the end read the last one again, columns past
+    // `main` its last one; they are not used.
     float4 v[NL];
-    auto unit = [&](int i) { return NU % 256 ? min(tid + 256 * i, NU - 1) : tid + 256 * i; };
+    auto unit = [&](int i) { return f32_unit(tid, i, RW + TW, C4); };
     auto load = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
-            const int e = unit(i), r = e / C4, c = k0 + 64 * (e % C4 / 16) + l16;
+            const F32Unit u = unit(i);
+            const int r = u.row, c = k0 + u.col;
             const float* src = r < RW ? w + (size_t)min(row0 + r, n_out - 1) * n_in
                                       : x + (size_t)min(tok0 + r - RW, tokens - 1) * n_in;
             v[i] = make_float4(src[min(c, main - 1)], src[min(c + 16, main - 1)], src[min(c + 32, main - 1)],
@@ -864,7 +865,8 @@ __global__ __launch_bounds__(256) void linear_f32(const float* __restrict__ w, c
     };
     auto stage = [&] {
 #pragma unroll
-        for (int i = 0; i < NL; ++i) (&tile[0][0])[unit(i)] = v[i];
+        for (int i = 0; i < NL; ++i)
+            if (const F32Unit u = unit(i); u.store) (&tile[0][0])[u.slot] = v[i];
         __syncthreads();
     };
     float acc[RT][TT];
