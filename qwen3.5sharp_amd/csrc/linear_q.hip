@@ -931,6 +931,55 @@ __global__ __launch_bounds__(256) void linear_f32(const float* __restrict__ w, c
         }
 }
 
+// The same without LDS, for short rows and for a few tokens of many rows (see
+// launch_linear_f32): four threads an output row, thread q holding reference
+// lanes 4q .. 4q + 3 (a float4 of each stride when rows are 16-byte aligned),
+// 64 rows a workgroup, one token a grid row.  Rows past n_out compute the last
+// one and are not stored.
+template <bool VEC>
+__global__ __launch_bounds__(256) void linear_f32_direct(const float* __restrict__ w, const float* __restrict__ x,
+                                                         float* __restrict__ y, int n_in, int n_out) {
+#pragma clang fp contract(off)
+    const int tid = threadIdx.x, q = tid & 3, row = blockIdx.x * 64 + (tid >> 2), t = blockIdx.y;
+    const float* a = x + (size_t)t * n_in;
+    const float* b = w + (size_t)min(row, n_out - 1) * n_in;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    int i = 0;
+    for (; i + 16 <= n_in; i += 16) {
+        float av[4], bv[4];
+        if constexpr (VEC) {
+            const float4 a4 = *reinterpret_cast<const float4*>(a + i + 4 * q);
+            const float4 b4 = *reinterpret_cast<const float4*>(b + i + 4 * q);
+            av[0] = a4.x; av[1] = a4.y; av[2] = a4.z; av[3] = a4.w;
+            bv[0] = b4.x; bv[1] = b4.y; bv[2] = b4.z; bv[3] = b4.w;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { av[k] = a[i + 4 * q + k]; bv[k] = b[i + 4 * q + k]; }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[k] = fmaf(av[k], bv[k], acc[k]);
+    }
+    if (i + 8 <= n_in) {
+        if (q < 2)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[k] = fmaf(a[i + 4 * q + k], b[i + 4 * q + k], acc[k]);
+        i += 8;
+    }
+    // s_j = acc0_j + acc1_j (threads 0, 1 hold acc0's lanes 0-7, threads 2, 3
+    // acc1's), then HorizontalSum.
+    float u[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float s = acc[k] + row_xor<2>(acc[k]);
+        u[k] = s + row_xor<1>(s);
+    }
+    if (q == 0 && row < n_out) {
+        float sum = (u[0] + u[2]) + (u[1] + u[3]);
+        for (; i < n_in; ++i) sum += a[i] * b[i];
+        y[(size_t)t * n_out + row] = sum;
+    }
+}
+
 // ---------------------------------------------------------------- Q4_K, several tokens
 
 // The reference's Q4_K path for several tokens (MulMatQ4K.Gemm,
@@ -1791,6 +1840,25 @@ hipError_t launch_linear_f32(q35m_ctx* c, const float* w, const float* x, float*
         hipExtLaunchKernelGGL(kern, dim3((n_out + rw - 1) / rw, (tokens + tw - 1) / tw), dim3(256), 0, c->stream,
                               ps_.a, ps_.b, 0, w, x, y, n_in, n_out, tokens);
     };
+    // Short rows spend more on staging than on their chain, the tail of a row
+    // that is no multiple of 8 most of all, and a few tokens of many rows fill
+    // a corner of an 8 x 8 tile: they read global memory directly, while W,
+    // read once a token, comes from the caches.  Measured (us, direct / tiles):
+    // 4 -> 8192 at 256 tokens 17 / 52, 16 -> 65536 at 4 3.7 / 8.1, 100 -> 1024
+    // at 2048 53 / 68 (120, no tail: 60 / 42), 64 -> 65536 at 4 5.7 / 8.1, 300
+    // -> 32768 at 2 9.5 / 15.4, 600 -> 65536 at 1 22.9 / 28.2 (151936, past the
+    // 256 MiB cache: 108 / 71), 1000 -> 8192 at 1 21.7 / 7.9.
+    const size_t wb = (size_t)n_in * n_out * sizeof(float), mb = (size_t)1 << 20;
+    const bool direct = n_in < 32 || (n_in < 64 && wb <= 16 * mb) || (n_in <= 128 && (n_in & 7) && wb <= 10 * mb) ||
+                        (n_out > 4096 && ((tokens <= 4 && n_in <= 256 && tokens * wb <= 128 * mb) ||
+                                          (tokens <= 2 && n_in <= 384 && tokens * wb <= 160 * mb) ||
+                                          (tokens == 1 && n_in <= 1024 && n_out >= 32768 && wb <= 256 * mb)));
+    if (direct) {
+        const bool vec = n_in % 4 == 0 && ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15) == 0;
+        hipExtLaunchKernelGGL(vec ? linear_f32_direct<true> : linear_f32_direct<false>, dim3((n_out + 63) / 64, tokens),
+                              dim3(256), 0, c->stream, ps_.a, ps_.b, 0, w, x, y, n_in, n_out);
+        return hipGetLastError();
+    }
     // One token's rows, or one token a workgroup, while those workgroups fit
     // the CUs once; else 4 x 4 tiles, the most chains in flight, up to four
     // workgroups a CU; else 8 x 8 tiles, half the LDS reads a chain.  Measured
@@ -1804,7 +1872,9 @@ hipError_t launch_linear_f32(q35m_ctx* c, const float* w, const float* x, float*
     const long rows4 = (n_out + 3) / 4, toks4 = (tokens + 3) / 4;
     // A chunk is staged whole, so rows narrower than it take a smaller one.
     const bool few = rows4 * toks4 <= 4L * c->n_cu;
-    if (n_in > 512 && (tokens == 1 || rows4 * tokens <= c->n_cu)) go(linear_f32<1, 1, 4, 1, 2560>, 4, 1);
+    // (One token of rows that a 2560-column chunk would pad: 1000 -> 65536 62.8
+    // as 4 x 1, 41 as 8 x 8.)
+    if (n_in > 512 && (rows4 * tokens <= c->n_cu || (tokens == 1 && n_in >= 2048))) go(linear_f32<1, 1, 4, 1, 2560>, 4, 1);
     else if (n_in <= 128) few ? go(linear_f32<1, 1, 4, 4, 128>, 4, 4) : go(linear_f32<2, 2, 4, 4, 128>, 8, 8);
     else few ? go(linear_f32<1, 1, 4, 4, 512>, 4, 4) : go(linear_f32<2, 2, 4, 4, 256>, 8, 8);
     return hipGetLastError();

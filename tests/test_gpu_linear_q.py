@@ -231,11 +231,15 @@ def test_linear_f32_bit_exact(ctx, n_in, n_out, tokens):
 
 
 @pytest.mark.parametrize("n_in,n_out,tokens", [(2569, 5, 1), (5200, 3, 2), (64, 9, 33), (527, 261, 5), (600, 264, 70),
-                                               (283, 270, 65), (15, 300, 61), (256, 8, 4100), (129, 33, 9), (100, 300, 70)])
+                                               (283, 270, 65), (15, 300, 61), (256, 8, 4100), (129, 33, 9), (100, 300, 70),
+                                               (1, 9000, 3), (63, 65, 130), (64, 65, 130), (127, 301, 5), (128, 301, 5),
+                                               (256, 4097, 4), (257, 4097, 4), (384, 4161, 2), (1021, 32801, 1),
+                                               (1024, 32768, 1), (1500, 1027, 1), (2049, 1030, 1)])
 def test_linear_f32_tiles(ctx, n_in, n_out, tokens):
-    """Each tile shape of the F32 projection (4 rows x 1 token, 4 x 4, 8 x 8)
-    at ragged rows and tokens and around its staged column chunks (2560, 512,
-    256, 128), bit for bit."""
+    """Each form of the F32 projection (4 rows x 1 token, 4 x 4, 8 x 8, direct
+    from global memory) at ragged rows and tokens, around its staged column
+    chunks (2560, 512, 256, 128) and on both sides of the rules between the
+    forms, bit for bit."""
     rng = np.random.default_rng(n_in + 7 * n_out + tokens)
     w = rng.standard_normal((n_out, n_in)).astype(np.float32)
     x = rng.standard_normal((tokens, n_in)).astype(np.float32)
