@@ -648,7 +648,9 @@ hipError_t go(q35m_ctx* c, int kid, const unsigned char* w, const uint32_t* q8, 
         // tokens (256 tiles) 6.8 / 9.7 / 18 / 24.
         if (tiles <= (QT == 4 ? 400 : 640)) return split(linear_gemm_split<QT, 1, 1>, 1, 1);
         if (tiles <= (QT == 4 ? 1536 : 2304)) return split(linear_gemm_split<QT, 2, 2>, 2, 2);
-        if (tiles <= 4608) return whole(linear_gemm<QT, 2, 8>, 32, 8);
+        // (Up to 32 tokens fill no 64: 2560 -> 151936 at 8 tokens 78 / 113; rows
+        // of two blocks hardly load: 512 -> 151936 28 / 20 for Q2_0C.)
+        if (tiles <= 4608 || (tokens <= 32 && nb > 2)) return whole(linear_gemm<QT, 2, 8>, 32, 8);
         return whole(linear_gemm<QT, 4, 8>, 64, 8);
     }
 }

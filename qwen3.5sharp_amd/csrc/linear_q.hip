@@ -521,14 +521,17 @@ __device__ __forceinline__ void iq4xs_block_terms(const uint32_t* __restrict__ w
     }
 }
 
-// One token: a wave per group of up to 8 whole rows (at most 64 blocks, a
-// block a thread, held in registers); one wave a workgroup, or FW with FUSED
-// (see linear_q).  The token's Q8_K row is staged or formed in LDS, every thread forms its block's integer terms, and one thread
-// per row runs the reference's fp32 chain over the row's blocks in order.
+// A wave per group of up to 8 whole rows (at most 64 blocks, a block a thread,
+// held in registers): one wave a workgroup and tok_per_wg tokens after one
+// another, or FW waves and one token with FUSED (see linear_q).  Each token's
+// Q8_K row is staged or formed in LDS, every thread forms its block's integer
+// terms, and one thread per row runs the reference's fp32 chain over the row's
+// blocks in order.
 template <int QT, bool FUSED>
 __global__ __launch_bounds__(FUSED ? FW * LQ_THREADS : LQ_THREADS) void linear_qs(const unsigned char* __restrict__ w,
                                                         const uint32_t* __restrict__ q8, const float* __restrict__ x,
-                                                        float* __restrict__ y, int n_in, int n_out, int rows_per_wg) {
+                                                        float* __restrict__ y, int n_in, int n_out, int tokens,
+                                                        int rows_per_wg, int tok_per_wg) {
 #pragma clang fp contract(off)
     constexpr int BB = QT == 5 ? Q5K_BYTES : IQ4XS_BYTES;
     extern __shared__ uint4 smem[];
@@ -555,61 +558,65 @@ __global__ __launch_bounds__(FUSED ? FW * LQ_THREADS : LQ_THREADS) void linear_q
             for (int c = 0; c < BB / 8; ++c) reinterpret_cast<uint2*>(wb)[c] = reinterpret_cast<const uint2*>(src)[c];
         }
     }
-    if constexpr (FUSED) {
-        quantize_row<false>(rl, x, nb, q8s);
-    } else {
-        const uint4* src = reinterpret_cast<const uint4*>(q8);
-        uint4* dst = reinterpret_cast<uint4*>(q8s);
-        const int n4 = nb * (Q8K_WORDS / 4);
-        for (int i0 = 0; i0 < n4; i0 += 8 * LQ_THREADS) {
-            uint4 qv[8];
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                qv[c] = make_uint4(0u, 0u, 0u, 0u);
-                if (i0 + lane + LQ_THREADS * c < n4) qv[c] = src[i0 + lane + LQ_THREADS * c];
-            }
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-                if (i0 + lane + LQ_THREADS * c < n4) dst[i0 + lane + LQ_THREADS * c] = qv[c];
-        }
-    }
-    lds_barrier();
-    // Each thread forms its block's terms of the reference's chain (they do
-    // not depend on the running sum); one thread per row then adds them in
-    // order.
-    if (lane < nblk) {
-        const uint32_t* q8b = q8s + (lane % nb) * Q8K_WORDS;
-        const float yd = __builtin_bit_cast(float, q8b[0]);
-        float* out = terms + lane * QS_TLD;
-        if constexpr (QT == 5) {
-            int acc, sumi;
-            q5k_block_terms(wb, q8b, acc, sumi);
-            const float d = half_bits_to_float(wb[0] & 0xffff) * yd;
-            const float dmin = half_bits_to_float(wb[0] >> 16) * yd;
-            out[0] = d * (float)acc - dmin * (float)sumi;
+    const int t_end = FUSED ? 1 : min(tokens, ((int)blockIdx.y + 1) * tok_per_wg);
+    for (int t = FUSED ? 0 : blockIdx.y * tok_per_wg; t < t_end; ++t) {
+        if constexpr (FUSED) {
+            quantize_row<false>(rl, x, nb, q8s);
         } else {
-            int acc[8];
-            iq4xs_block_terms(wb, q8b, acc);
-            const uint32_t hdr = wb[0], sl = wb[1];
-            const float d = half_bits_to_float(hdr & 0xffff);
+            const uint4* src = reinterpret_cast<const uint4*>(q8 + (size_t)t * nb * Q8K_WORDS);
+            uint4* dst = reinterpret_cast<uint4*>(q8s);
+            const int n4 = nb * (Q8K_WORDS / 4);
+            for (int i0 = 0; i0 < n4; i0 += 8 * LQ_THREADS) {
+                uint4 qv[8];
 #pragma unroll
-            for (int ib = 0; ib < 8; ++ib) {
-                const int ls = (int)(((sl >> (8 * (ib >> 1) + 4 * (ib & 1))) & 0xf) |
-                                     (((hdr >> (16 + 2 * ib)) & 3) << 4));
-                const float dl = d * (float)(ls - 32);
-                out[ib] = dl * (float)acc[ib] * yd;
+                for (int c = 0; c < 8; ++c) {
+                    qv[c] = make_uint4(0u, 0u, 0u, 0u);
+                    if (i0 + lane + LQ_THREADS * c < n4) qv[c] = src[i0 + lane + LQ_THREADS * c];
+                }
+#pragma unroll
+                for (int c = 0; c < 8; ++c)
+                    if (i0 + lane + LQ_THREADS * c < n4) dst[i0 + lane + LQ_THREADS * c] = qv[c];
             }
         }
-    }
-    lds_barrier();
-    if (lane < nrows) {
-        constexpr int NTERM = QT == 5 ? 1 : 8;
-        float sumf = 0.0f;
-        const float* T = terms + lane * nb * QS_TLD;
-        for (int b = 0; b < nb; ++b)
+        lds_barrier();
+        // Each thread forms its block's terms of the reference's chain (they do
+        // not depend on the running sum); one thread per row then adds them in
+        // order.
+        if (lane < nblk) {
+            const uint32_t* q8b = q8s + (lane % nb) * Q8K_WORDS;
+            const float yd = __builtin_bit_cast(float, q8b[0]);
+            float* out = terms + lane * QS_TLD;
+            if constexpr (QT == 5) {
+                int acc, sumi;
+                q5k_block_terms(wb, q8b, acc, sumi);
+                const float d = half_bits_to_float(wb[0] & 0xffff) * yd;
+                const float dmin = half_bits_to_float(wb[0] >> 16) * yd;
+                out[0] = d * (float)acc - dmin * (float)sumi;
+            } else {
+                int acc[8];
+                iq4xs_block_terms(wb, q8b, acc);
+                const uint32_t hdr = wb[0], sl = wb[1];
+                const float d = half_bits_to_float(hdr & 0xffff);
 #pragma unroll
-            for (int k = 0; k < NTERM; ++k) sumf += T[b * QS_TLD + k];
-        y[row0 + lane] = sumf;
+                for (int ib = 0; ib < 8; ++ib) {
+                    const int ls = (int)(((sl >> (8 * (ib >> 1) + 4 * (ib & 1))) & 0xf) |
+                                         (((hdr >> (16 + 2 * ib)) & 3) << 4));
+                    const float dl = d * (float)(ls - 32);
+                    out[ib] = dl * (float)acc[ib] * yd;
+                }
+            }
+        }
+        lds_barrier();
+        if (lane < nrows) {
+            constexpr int NTERM = QT == 5 ? 1 : 8;
+            float sumf = 0.0f;
+            const float* T = terms + lane * nb * QS_TLD;
+            for (int b = 0; b < nb; ++b)
+#pragma unroll
+                for (int k = 0; k < NTERM; ++k) sumf += T[b * QS_TLD + k];
+            y[(size_t)t * n_out + row0 + lane] = sumf;
+        }
+        if (t + 1 < t_end) lds_barrier();
     }
 }
 
@@ -698,15 +705,16 @@ __device__ __forceinline__ int stq_unit_dot(const uint32_t* __restrict__ base, i
     return enc - q8k_bsum_total(q8b);
 }
 
-// One token: a wave per group of up to 8 whole rows (at most 64 units, one a
-// thread), one wave a workgroup, or FW with FUSED (see linear_q): the rows' contiguous weight bytes are staged in LDS
-// (as for Q6_K) and the token's Q8_K row, every thread forms its unit's T, and
-// one thread per row runs the chain.
+// A wave per group of up to 8 whole rows (at most 64 units, one a thread), one
+// wave a workgroup and tok_per_wg tokens, or FW waves and one token with FUSED
+// (see linear_q): the rows' contiguous weight bytes are staged in LDS (as for
+// Q6_K), then per token its Q8_K row, every thread forms its unit's T, and one
+// thread per row runs the chain.
 template <int QT, bool FUSED>
 __global__ __launch_bounds__(FUSED ? FW * LQ_THREADS : LQ_THREADS) void linear_qt(const unsigned char* __restrict__ w,
                                                         const uint32_t* __restrict__ q8, const float* __restrict__ x,
-                                                        float* __restrict__ y, int n_in, int n_out,
-                                                        int rows_per_wg, int panel_rows) {
+                                                        float* __restrict__ y, int n_in, int n_out, int tokens,
+                                                        int rows_per_wg, int tok_per_wg, int panel_rows) {
 #pragma clang fp contract(off)
     constexpr int UB = QT == 2 ? Q2_BYTES / 2 : STQ_BYTES;   // weight bytes per unit
     extern __shared__ uint4 smem[];
@@ -758,66 +766,70 @@ __global__ __launch_bounds__(FUSED ? FW * LQ_THREADS : LQ_THREADS) void linear_q
         }
     }
 
-    if constexpr (FUSED) {
-        quantize_row<QT == 2>(rl, x, nb, q8s);
-    } else {
-        const uint4* src = reinterpret_cast<const uint4*>(q8);
-        uint4* dst = reinterpret_cast<uint4*>(q8s);
-        const int n4 = nb * (Q8K_WORDS / 4);
-        for (int i0 = 0; i0 < n4; i0 += 8 * LQ_THREADS) {
-            uint4 qv[8];
+    const int t_end = FUSED ? 1 : min(tokens, ((int)blockIdx.y + 1) * tok_per_wg);
+    for (int t = FUSED ? 0 : blockIdx.y * tok_per_wg; t < t_end; ++t) {
+        if constexpr (FUSED) {
+            quantize_row<QT == 2>(rl, x, nb, q8s);
+        } else {
+            const uint4* src = reinterpret_cast<const uint4*>(q8 + (size_t)t * nb * Q8K_WORDS);
+            uint4* dst = reinterpret_cast<uint4*>(q8s);
+            const int n4 = nb * (Q8K_WORDS / 4);
+            for (int i0 = 0; i0 < n4; i0 += 8 * LQ_THREADS) {
+                uint4 qv[8];
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                qv[c] = make_uint4(0u, 0u, 0u, 0u);
-                if (i0 + lane + LQ_THREADS * c < n4) qv[c] = src[i0 + lane + LQ_THREADS * c];
-            }
+                for (int c = 0; c < 8; ++c) {
+                    qv[c] = make_uint4(0u, 0u, 0u, 0u);
+                    if (i0 + lane + LQ_THREADS * c < n4) qv[c] = src[i0 + lane + LQ_THREADS * c];
+                }
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const int i = i0 + lane + LQ_THREADS * c;
-                if (i < n4) {
-                    const int part = i % (Q8K_WORDS / 4);     // 1..16: qs, 0 and 17..18: d, bsums
-                    dst[i] = (QT == 2 && part >= 1 && part <= 16) ? byte_transpose(qv[c]) : qv[c];
+                for (int c = 0; c < 8; ++c) {
+                    const int i = i0 + lane + LQ_THREADS * c;
+                    if (i < n4) {
+                        const int part = i % (Q8K_WORDS / 4);     // 1..16: qs, 0 and 17..18: d, bsums
+                        dst[i] = (QT == 2 && part >= 1 && part <= 16) ? byte_transpose(qv[c]) : qv[c];
+                    }
                 }
             }
         }
-    }
-    lds_barrier();
-    if (lane < nunit) {
-        const int r = lane / nb, b = lane % nb;
-        const uint32_t* q8b = q8s + b * Q8K_WORDS;
-        if constexpr (QT == 2)
-            tv[lane] = q2_unit_dot(wbase, shift + (int)(r * row_bytes) + (b >> 1) * Q2_BYTES + 2 + 64 * (b & 1), q8b);
-        else
-            tv[lane] = stq_unit_dot(wbase, shift + (int)(r * row_bytes) + b * STQ_BYTES, q8b);
-    }
-    lds_barrier();
-    if (lane < nrows) {
-        const int row = row0 + lane;
-        const int* T = tv + lane * nb;
-        const int o = shift + (int)(lane * row_bytes);
-        float acc = 0.0f;
-        if (row < panel_rows) {
-            for (int b = 0; b < nb; ++b) {
-                const int dof = QT == 2 ? o + (b >> 1) * Q2_BYTES : o + b * STQ_BYTES + 40;
-                const float dw = half_bits_to_float(lds_word(wbase, dof) & 0xffff);
-                const float dx = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
-                acc = fmaf((float)T[b], dw * dx, acc);
-            }
-        } else if constexpr (QT == 2) {
-            for (int b = 0; b < nb; b += 2) {
-                const float dw = half_bits_to_float(lds_word(wbase, o + (b >> 1) * Q2_BYTES) & 0xffff);
-                const float dx0 = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
-                const float dx1 = __builtin_bit_cast(float, q8s[(b + 1) * Q8K_WORDS]);
-                acc = acc + dw * ((float)T[b] * dx0 + (float)T[b + 1] * dx1);
-            }
-        } else {
-            for (int b = 0; b < nb; ++b) {
-                const float dw = half_bits_to_float(lds_word(wbase, o + b * STQ_BYTES + 40) & 0xffff);
-                const float dx = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
-                acc = acc + (dw * dx) * (float)T[b];
-            }
+        lds_barrier();
+        if (lane < nunit) {
+            const int r = lane / nb, b = lane % nb;
+            const uint32_t* q8b = q8s + b * Q8K_WORDS;
+            if constexpr (QT == 2)
+                tv[lane] = q2_unit_dot(wbase, shift + (int)(r * row_bytes) + (b >> 1) * Q2_BYTES + 2 + 64 * (b & 1), q8b);
+            else
+                tv[lane] = stq_unit_dot(wbase, shift + (int)(r * row_bytes) + b * STQ_BYTES, q8b);
         }
-        y[row] = acc;
+        lds_barrier();
+        if (lane < nrows) {
+            const int row = row0 + lane;
+            const int* T = tv + lane * nb;
+            const int o = shift + (int)(lane * row_bytes);
+            float acc = 0.0f;
+            if (row < panel_rows) {
+                for (int b = 0; b < nb; ++b) {
+                    const int dof = QT == 2 ? o + (b >> 1) * Q2_BYTES : o + b * STQ_BYTES + 40;
+                    const float dw = half_bits_to_float(lds_word(wbase, dof) & 0xffff);
+                    const float dx = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
+                    acc = fmaf((float)T[b], dw * dx, acc);
+                }
+            } else if constexpr (QT == 2) {
+                for (int b = 0; b < nb; b += 2) {
+                    const float dw = half_bits_to_float(lds_word(wbase, o + (b >> 1) * Q2_BYTES) & 0xffff);
+                    const float dx0 = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
+                    const float dx1 = __builtin_bit_cast(float, q8s[(b + 1) * Q8K_WORDS]);
+                    acc = acc + dw * ((float)T[b] * dx0 + (float)T[b + 1] * dx1);
+                }
+            } else {
+                for (int b = 0; b < nb; ++b) {
+                    const float dw = half_bits_to_float(lds_word(wbase, o + b * STQ_BYTES + 40) & 0xffff);
+                    const float dx = __builtin_bit_cast(float, q8s[b * Q8K_WORDS]);
+                    acc = acc + (dw * dx) * (float)T[b];
+                }
+            }
+            y[(size_t)t * n_out + row] = acc;
+        }
+        if (t + 1 < t_end) lds_barrier();
     }
 }
 
@@ -1680,12 +1692,16 @@ hipError_t launch_q8k_quantize(q35m_ctx* c, const float* x, void* q8, int n_in, 
     return hipGetLastError();
 }
 
-// The one-token kernels, from the Q8_K row q8 or (q8 null) the fp32 row x; also
-// rows from row_base on of several tokens of Q4_K and Q6_K, tok_per_wg a
-// workgroup.
+// The GEMV kernels, from the Q8_K rows q8 or (q8 null) one token's fp32 row x:
+// rows from row_base on (0 but for Q4_K and Q6_K); rows below panel_rows take
+// the eight-row panel order (Q2_0C, STQ1_0).
 static hipError_t launch_gemv(q35m_ctx* c, int qtype, const unsigned char* w, const uint32_t* q8, const float* x, float* y,
-                              int n_in, int n_out, int tokens, int row_base, int tok_per_wg) {
+                              int n_in, int n_out, int tokens, int row_base, int panel_rows) {
     const int nb = n_in / QK, rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS), waves = q8 ? 1 : FW;
+    // Tokens a workgroup: one while the workgroups fit the CUs about once (a
+    // tiled call's last rows, many tokens of few rows, took 0.75 us a token).
+    const long groups = (n_out - row_base + rows_per_wg - 1) / rows_per_wg;
+    const int tok_per_wg = (int)((tokens * groups + 1499) / 1500);
     const dim3 grid(((n_out - row_base + rows_per_wg - 1) / rows_per_wg + waves - 1) / waves,
                     (tokens + tok_per_wg - 1) / tok_per_wg);
     const dim3 block(LQ_THREADS * waves);
@@ -1697,17 +1713,16 @@ static hipError_t launch_gemv(q35m_ctx* c, int qtype, const unsigned char* w, co
         return hipGetLastError();
     };
     if (qtype == 1 || qtype == 2) {
-        // Eight-row panels (see launch_linear_q_prequant) of one token.
         const int ub = qtype == 2 ? Q2_BYTES / 2 : STQ_BYTES;
         const size_t lds = 16 * (size_t)((rows_per_wg * nb * ub + 31) / 16 + 1) + LQ_THREADS * 4;
-        const int kid = qtype == 2 ? K_Q2_0C_LINEAR : K_STQ1_0_LINEAR, panel_rows = n_out & ~7;
-        if (qtype == 2) return go(q8 ? linear_qt<2, false> : linear_qt<2, true>, kid, lds, rows_per_wg, panel_rows);
-        return go(q8 ? linear_qt<1, false> : linear_qt<1, true>, kid, lds, rows_per_wg, panel_rows);
+        const int kid = qtype == 2 ? K_Q2_0C_LINEAR : K_STQ1_0_LINEAR;
+        auto kern = qtype == 2 ? (q8 ? linear_qt<2, false> : linear_qt<2, true>) : q8 ? linear_qt<1, false> : linear_qt<1, true>;
+        return go(kern, kid, lds, tokens, rows_per_wg, tok_per_wg, panel_rows);
     }
     if (qtype == 5 || qtype == 14) {
         const size_t lds = (size_t)LQ_THREADS * QS_TLD * 4;
-        if (qtype == 5) return go(q8 ? linear_qs<5, false> : linear_qs<5, true>, K_Q5K_LINEAR, lds, rows_per_wg);
-        return go(q8 ? linear_qs<14, false> : linear_qs<14, true>, K_IQ4XS_LINEAR, lds, rows_per_wg);
+        auto kern = qtype == 5 ? (q8 ? linear_qs<5, false> : linear_qs<5, true>) : q8 ? linear_qs<14, false> : linear_qs<14, true>;
+        return go(kern, qtype == 5 ? K_Q5K_LINEAR : K_IQ4XS_LINEAR, lds, tokens, rows_per_wg, tok_per_wg);
     }
     const int bb = qtype == 4 ? Q4K_BYTES : Q6K_BYTES;
     const size_t lds = 16 * (size_t)lq_wave_chunks(qtype, rows_per_wg, nb, bb);
@@ -1721,22 +1736,45 @@ static hipError_t launch_gemv(q35m_ctx* c, int qtype, const unsigned char* w, co
               : pick(linear_q<6, 10, true>, linear_q<6, 16, true>, linear_q<6, 0, true>, K_Q6K_LINEAR);
 }
 
+// Whether a few tokens of Q5_K, IQ4_XS, Q2_0C or STQ1_0 take the GEMV, which
+// costs by the token and the row group (about 0.4 ns for Q5_K, 1 for STQ1_0),
+// or linear_gemm, which costs by its tiles, filled or not.  While every tile
+// has its own workgroup, the line lies at so many row-group tokens a block of a
+// row and round of the CUs; past that, at so many tokens.  Measured (us, GEMV /
+// matrix cores): Q5_K 2560 -> 8192 at 3 tokens 9.2 / 9.2, at 4 10.3 / 9.3;
+// 2560 -> 12288 at 8 15 / 18; 4096 -> 65536 at 4 49 / 62; 16384 -> 1024 at 2 10
+// / 24; IQ4_XS 2560 -> 12288 at 8 19 / 22; 2560 -> 151936 at 2 47 / 113; Q2_0C
+// 4096 -> 32768 at 4 40 / 52; 9728 -> 65536 at 2 248 / 78; STQ1_0 4096 -> 8192
+// at 2 12 / 10, 2560 -> 12288 at 2 11 / 15.
+static bool few_tokens_gemv(int qtype, int n_in, int n_out, int tokens) {
+    struct Line { int groups, blocks, mid, mid_blocks, mid_long, wide, short_rows; };
+    const Line l = qtype == 5 ? Line{260, 32, 8, 100, 3, 4, 2} : qtype == 14 ? Line{282, 22, 8, 100, 2, 6, 4}
+                 : qtype == 2 ? Line{140, 36, 4, 64, 1, 2, 1} : Line{60, 36, 2, 24, 1, 1, 1};
+    const int nb = n_in / QK, rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
+    const long groups = (n_out + rows_per_wg - 1) / rows_per_wg, tiles = (n_out + 15) / 16;
+    if (nb <= 2 || tokens > 16) return false;
+    if (tiles <= 640) return nb > 4 && tokens * groups <= (long)l.groups * min(nb, l.blocks) * ((tiles + 255) / 256);
+    if (nb <= 4) return tokens <= l.short_rows;
+    if (nb > 24) return tiles <= 2304 && tokens <= l.mid_long;
+    if (tiles <= 2304) return tokens <= l.mid && tokens * nb <= l.mid_blocks;
+    return tokens <= l.wide && tokens * nb <= 64;
+}
+
 hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const void* q8, float* y,
                                     int n_in, int n_out, int tokens) {
     const int nb = n_in / QK;
     const unsigned char* wb = reinterpret_cast<const unsigned char*>(w);
     const uint32_t* qb = reinterpret_cast<const uint32_t*>(q8);
-    if (tokens == 1) return launch_gemv(c, qtype, wb, qb, nullptr, y, n_in, n_out, 1, 0, 1);
-    if (qtype == 1 || qtype == 2) {
-        // Which rows take the eight-row panel order (MulMatQ2.cs:25-40,
-        // MulMatSTQ.cs:25-64): the first n_out & ~7, except STQ1_0 with
-        // several tokens: all rows when tokens % 4 == 0 and n_out % 8 == 0,
-        // else none.
-        int panel_rows = n_out & ~7;
-        if (qtype == 1) panel_rows = ((tokens & 3) == 0 && (n_out & 7) == 0) ? n_out : 0;
+    // Which rows take the eight-row panel order (MulMatQ2.cs:25-40,
+    // MulMatSTQ.cs:25-64): the first n_out & ~7, except STQ1_0 with several
+    // tokens: all rows when tokens % 4 == 0 and n_out % 8 == 0, else none.
+    int panel_rows = n_out & ~7;
+    if (qtype == 1 && tokens > 1) panel_rows = ((tokens & 3) == 0 && (n_out & 7) == 0) ? n_out : 0;
+    if (tokens == 1) return launch_gemv(c, qtype, wb, qb, nullptr, y, n_in, n_out, 1, 0, panel_rows);
+    if (qtype != 4 && qtype != 6) {
+        if (few_tokens_gemv(qtype, n_in, n_out, tokens)) return launch_gemv(c, qtype, wb, qb, nullptr, y, n_in, n_out, tokens, 0, panel_rows);
         return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, n_out, tokens, panel_rows);
     }
-    if (qtype == 5 || qtype == 14) return launch_linear_gemm(c, qtype, w, q8, y, n_in, n_out, n_out, tokens, 0);
     // The tiled kernels address their operands through buffer descriptors
     // (32-bit offsets): calls with more than 2 GiB of weight rows or of
     // activations go in pieces of whole row and token tiles (even rows), each
@@ -1793,11 +1831,7 @@ hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const
         else e = tiled(q6k_gemm, K_Q6K_GEMM, Q6K_BYTES, SGR, SGT, 256, row_base);
     }
     if (e != hipSuccess || row_base == n_out) return e;
-    // Tokens a workgroup: one while the workgroups fit the CUs about once (a
-    // tiled call's last rows, many tokens of few rows, took 0.75 us a token).
-    const int grid = (n_out - row_base + rows_per_wg - 1) / rows_per_wg;
-    const int tok_per_wg = (int)(((long)tokens * grid + 1499) / 1500);
-    return launch_gemv(c, qtype, wb, qb, nullptr, y, n_in, n_out, tokens, row_base, tok_per_wg);
+    return launch_gemv(c, qtype, wb, qb, nullptr, y, n_in, n_out, tokens, row_base, 0);
 }
 
 // One token of Q6_K keeps the quantizer apart where the row and four waves'
@@ -1813,7 +1847,8 @@ bool linear_q_fused(int qtype, const float* x, const float* y, int n_in, int n_o
 hipError_t launch_linear_q(q35m_ctx* c, int qtype, const void* w, const float* x, float* y,
                            int n_in, int n_out, int tokens) {
     if (linear_q_fused(qtype, x, y, n_in, n_out, tokens))
-        return launch_gemv(c, qtype, reinterpret_cast<const unsigned char*>(w), nullptr, x, y, n_in, n_out, 1, 0, 1);
+        return launch_gemv(c, qtype, reinterpret_cast<const unsigned char*>(w), nullptr, x, y, n_in, n_out, 1, 0,
+                           n_out & ~7);
     hipError_t e = launch_q8k_quantize(c, x, c->work, n_in, tokens);
     if (e != hipSuccess) return e;
     return launch_linear_q_prequant(c, qtype, w, c->work, y, n_in, n_out, tokens);

@@ -91,6 +91,35 @@ def test_linear_gemm_tiles(ctx, qtype, n_in, n_out, tokens):
     assert np.array_equal(got.view(np.uint32), oracle.linear_q(qtype, w, x, n_in, n_out).view(np.uint32))
 
 
+GEMV_NAME = {1: "linear_qt<1>", 2: "linear_qt<2>", 4: "linear_q<4>", 5: "linear_qs<5>", 6: "linear_q<6>", 14: "linear_qs<14>"}
+
+
+def run_named(ctx, qtype, n_in, n_out, tokens, seed):
+    """One projection against the oracle, bit for bit; the kernels it ran."""
+    rng = np.random.default_rng(seed + 31 * qtype + n_in + n_out + tokens)
+    w = qb.random_blocks(rng, qtype, qb.nblocks(qtype, n_out * n_in))
+    x = rng.standard_normal((tokens, n_in)).astype(np.float32)
+    ctx.profile(True)
+    got = run(ctx, qtype, w, x, n_in, n_out)
+    ran = ctx.profile_read()
+    ctx.profile(False)
+    assert np.array_equal(got.view(np.uint32), oracle.linear_q(qtype, w, x, n_in, n_out).view(np.uint32))
+    return ran
+
+
+@pytest.mark.parametrize("qtype", [5, 14, 2, 1])
+@pytest.mark.parametrize("n_in,n_out,tokens,gemv", [(4096, 257, 2, True), (4096, 30, 16, True), (4096, 30, 17, False),
+                                                    (9728, 41, 5, True), (16384, 19, 4, True), (3584, 331, 3, True),
+                                                    (2560, 10300, 2, True), (2560, 10300, 12, False), (512, 40, 2, False),
+                                                    (1024, 8200, 3, False), (2560, 40000, 17, False), (9728, 10300, 4, False)])
+def test_linear_few_tokens(ctx, qtype, n_in, n_out, tokens, gemv):
+    """A few tokens of the formats that run per token: the GEMV over several
+    tokens a workgroup, and the matrix cores on the other side of the rule
+    (32-token tiles of wide outputs among them)."""
+    ran = run_named(ctx, qtype, n_in, n_out, tokens, 900)
+    assert (GEMV_NAME[qtype] in ran) == gemv and (f"linear_gemm<{qtype}>" in ran) != gemv
+
+
 @pytest.mark.parametrize("qtype", TYPES)
 @pytest.mark.parametrize("n_in,n_out", [(512, 1), (512, 33), (4096, 17), (4608, 129), (10240, 5), (10752, 9), (16384, 3)])
 def test_linear_q_one_token_quantizes(ctx, qtype, n_in, n_out):
