@@ -201,7 +201,7 @@ const char* kernel_name(int id) {
         "q4k_gemm", "q6k_gemm", "add_rmsnorm", "linear_qs<5>", "linear_qs<14>", "linear_f32", "linear_qt<2>",
         "linear_qt<1>", "attn_decode_partial<4,16>", "attn_decode_partial<8,16>", "q6k_gemm_blk",
         "linear_gemm<5>", "linear_gemm<14>", "linear_gemm<2>", "linear_gemm<1>",
-        "attn_split_prep", "attn_split_flash", "attn_split_merge"};
+        "attn_split_prep", "attn_split_flash", "attn_split_merge", "linear_gemm<4>", "linear_gemm<6>"};
     return (id >= 0 && id < K_COUNT) ? names[id] : nullptr;
 }
 

@@ -645,12 +645,13 @@ hipError_t go(q35m_ctx* c, int kid, const unsigned char* w, const uint32_t* q8, 
     } else {
         // Q4_K at 16 tokens 10.9 / 9.3 / 18 / 25, at 64 34 / 17.6 / 18 / 25, at
         // 128 66 / 32 / 19 / 26, at 256 131 / 63 / 34 / 27; 2560 -> 1024 at 64
-        // tokens (256 tiles) 6.8 / 9.7 / 18 / 24.
+        // tokens (256 tiles) 6.8 / 9.7 / 18 / 24; 512 -> 12288 at 96 (4608) - / -
+        // / 15 / 11.
         if (tiles <= (QT == 4 ? 400 : 640)) return split(linear_gemm_split<QT, 1, 1>, 1, 1);
         if (tiles <= (QT == 4 ? 1536 : 2304)) return split(linear_gemm_split<QT, 2, 2>, 2, 2);
         // (Up to 32 tokens fill no 64: 2560 -> 151936 at 8 tokens 78 / 113; rows
         // of two blocks hardly load: 512 -> 151936 28 / 20 for Q2_0C.)
-        if (tiles <= 4608 || (tokens <= 32 && nb > 2)) return whole(linear_gemm<QT, 2, 8>, 32, 8);
+        if (tiles <= (QT == 4 ? 4096 : 4608) || (tokens <= 32 && nb > 2)) return whole(linear_gemm<QT, 2, 8>, 32, 8);
         return whole(linear_gemm<QT, 4, 8>, 64, 8);
     }
 }
@@ -662,8 +663,8 @@ hipError_t launch_linear_gemm(q35m_ctx* c, int qtype, const void* w, const void*
     const unsigned char* wb = reinterpret_cast<const unsigned char*>(w);
     const uint32_t* qb = reinterpret_cast<const uint32_t*>(q8);
     switch (qtype) {
-        case 4: return go<4>(c, K_Q4K_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, 0);
-        case 6: return go<6>(c, K_Q6K_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, 0);
+        case 4: return go<4>(c, K_Q4K_SMALL, wb, qb, y, n_in, n_rows, n_out, tokens, 0);
+        case 6: return go<6>(c, K_Q6K_SMALL, wb, qb, y, n_in, n_rows, n_out, tokens, 0);
         case 5: return go<5>(c, K_Q5K_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, 0);
         case 14: return go<14>(c, K_IQ4XS_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, 0);
         case 2: return go<2>(c, K_Q2_0C_GEMM, wb, qb, y, n_in, n_rows, n_out, tokens, panel_rows);

@@ -1804,28 +1804,36 @@ hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const
     // the end of it.
     const int rows_per_wg = min(LQ_THREADS / nb, LQ_MAX_ROWS);
     int row_base = 0;
-    // The GEMV takes a few tokens while its workgroups fit the CUs about
-    // once; the matrix cores the rest: linear_gemm's small tiles while they
-    // are few, else 64-token tiles.  Measured (us; GEMV / small / 64-token
-    // tiles): Q6_K 4096 -> 2560 at 2 tokens 6.8 / 12 / 29, at 4 9.8 / 12 /
-    // 29, at 8 17 / 12 / 29, at 32 - / 22 / 29; 2560 -> 8192 at 2 11 / 16.5
-    // / 20, at 16 - / 16.5 / 20, at 32 - / 36 / 20; 2560 -> 1024 at 4 6.0 /
-    // 9.3 / 19, at 16 10.4 / 9.5 / 19 (a workgroup's tokens one after the
-    // other: 11.6 at 4, 47 at 15 of 2560 -> 8192).  Q4_K (GEMV order in no
-    // whole panel: small tiles / 64-token tiles) 2560 -> 8192 at 8 9.1 / 30,
-    // at 128 19 / 32, at 256 27 / 32, at 500 49 / 44.
-    const long groups = (n_out + rows_per_wg - 1) / rows_per_wg;
-    const long tiles = (long)((n_out + 15) / 16) * ((tokens + 15) / 16);
+    // Q6_K by what a call costs in each form (us; GEMV / small tiles / 64-token
+    // tiles).  The GEMV: tokens times row groups, in rounds of the CUs as the
+    // tiles' own: 4096 -> 2560 at 2 tokens 9 / 13 / 31, at 4 12 / 14 / 32; 2560
+    // -> 8192 at 4 17 / 20 / 22, at 6 23 / 20 / 22; 16384 -> 1024 at 4 28 / 36 /
+    // 112; past 8192 outputs, where the small tiles have no advantage left, 3
+    // tokens: 2560 -> 151936 148 / 275 / 175, at 4 186 / 283 / 175; 2560 ->
+    // 12288 at 6 24 / 27 / 27.  Rows of more than 24 blocks leave it two tokens:
+    // 9728 -> 8192 61 / 43 / 69.  The small tiles up to two a CU (4096 -> 8192 at
+    // 16 26 / 32, 2560 at 64 36 / 32), three while they are one token tile of
+    // long rows (9728 -> 12288 at 8 70 / 88), one for rows of three blocks (512
+    // -> 8192 at 64 17 / 9).
+    // Q4_K (GEMV order in no whole panel: small / 64-token tiles): 2560 -> 8192
+    // at 8 tokens 9.1 / 30, at 128 19 / 32, at 256 27 / 32, at 500 49 / 44;
+    // but 65536 outputs at 17-32 52 / 44 (at 16 of 512 inputs 14.6 / 12.4).
+    const long groups = (n_out + rows_per_wg - 1) / rows_per_wg, row_tiles = (n_out + 15) / 16;
+    const long tiles = row_tiles * ((tokens + 15) / 16);
+    bool gemv = tokens <= 16;
+    if (row_tiles <= 512) gemv &= tokens * groups <= min(275 * nb, 5000) * ((row_tiles + 255) / 256);
+    else gemv &= nb > 2 && nb <= 24 && (tokens <= 3 || (nb >= 8 && nb <= 12 && row_tiles <= 768 && tokens * groups <= 12500));
     if (qtype == 4) {
         row_base = n_out & ~7;
     } else if (c->proj_order == Q35M_PROJ_BLOCK && tokens >= 16 && (((size_t)n_out * nb) & 1) == 0) {
         return tiled(q6k_gemm_blk, K_Q6K_GEMM_BLK, Q6K_BYTES, BR, BT, BTHREADS, n_out);
-    } else if (groups * tokens > 4000 || tokens > 16) {
+    } else if (!gemv) {
         row_base = n_out - (int)(((size_t)n_out * nb) & 1);
     }
     hipError_t e = hipSuccess;
     if (row_base > 0) {
-        const bool small = qtype == 4 ? tiles <= 8192 : tiles * nb <= 5120;
+        const bool small = qtype == 4 ? tiles <= (tokens > 32 ? 8192 : nb > 2 || tokens > 16 ? 4096 : 2048)
+                                      : tiles <= (nb <= 3 ? 256 : tokens <= 16 && nb >= 16 ? 768 : 512);
         if (small) e = launch_linear_gemm(c, qtype, w, q8, y, n_in, row_base, n_out, tokens, 0);
         else if (qtype == 4) e = tiled(q4k_gemm, K_Q4K_GEMM, Q4K_BYTES, GR, GT, GTHREADS, row_base);
         else e = tiled(q6k_gemm, K_Q6K_GEMM, Q6K_BYTES, SGR, SGT, 256, row_base);

@@ -98,6 +98,8 @@ enum KernelId {
     K_ATTN_SPLIT_PREP,
     K_ATTN_SPLIT_FLASH,
     K_ATTN_SPLIT_MERGE,
+    K_Q4K_SMALL,                 // linear_gemm and linear_gemm_split of Q4_K, Q6_K
+    K_Q6K_SMALL,
     K_COUNT
 };
 const char* kernel_name(int id);

@@ -120,6 +120,31 @@ def test_linear_few_tokens(ctx, qtype, n_in, n_out, tokens, gemv):
     assert (GEMV_NAME[qtype] in ran) == gemv and (f"linear_gemm<{qtype}>" in ran) != gemv
 
 
+@pytest.mark.parametrize("n_in,n_out,tokens,kernels", [
+    (2560, 8192, 3, ["linear_q<6>"]), (2560, 2053, 8, ["linear_q<6>"]), (2560, 1000, 17, ["linear_gemm<6>"]),
+    (16384, 521, 5, ["linear_q<6>"]), (2560, 12001, 2, ["linear_q<6>"]), (2560, 12001, 7, ["q6k_gemm"]),
+    (2560, 16390, 3, ["linear_q<6>"]), (2560, 16390, 4, ["q6k_gemm"]), (9728, 8200, 2, ["linear_gemm<6>"]),
+    (5376, 8203, 4, ["linear_gemm<6>", "linear_q<6>"]), (5376, 4101, 33, ["q6k_gemm", "linear_q<6>"]),
+    (768, 2051, 100, ["q6k_gemm", "linear_q<6>"]), (768, 33, 20, ["linear_gemm<6>", "linear_q<6>"]),
+    (512, 4120, 17, ["q6k_gemm"]), (512, 4080, 16, ["linear_gemm<6>"])])
+def test_linear_q6k_forms(ctx, n_in, n_out, tokens, kernels):
+    """Q6_K of several tokens on both sides of the rules between the GEMV, the
+    small tiles and the 64-token tiles; with an odd number of blocks the last
+    row goes to the GEMV."""
+    ran = run_named(ctx, 6, n_in, n_out, tokens, 1900)
+    assert sorted(k for k in ran if k != "q8k_quantize") == sorted(kernels)
+
+
+@pytest.mark.parametrize("n_in,n_out,tokens,kernels", [
+    (512, 32768, 16, ["linear_gemm<4>"]), (512, 32776, 16, ["q4k_gemm"]), (768, 65529, 2, ["linear_gemm<4>", "linear_q<4>"]),
+    (768, 32776, 18, ["q4k_gemm"]), (1280, 12291, 90, ["linear_gemm<4>", "linear_q<4>"]), (768, 3009, 800, ["q4k_gemm", "linear_q<4>"])])
+def test_linear_q4k_forms(ctx, n_in, n_out, tokens, kernels):
+    """The same for Q4_K: small tiles and 64-token tiles, the GEMV for the last
+    n_out % 8 rows."""
+    ran = run_named(ctx, 4, n_in, n_out, tokens, 2900)
+    assert sorted(k for k in ran if k != "q8k_quantize") == sorted(kernels)
+
+
 @pytest.mark.parametrize("qtype", TYPES)
 @pytest.mark.parametrize("n_in,n_out", [(512, 1), (512, 33), (4096, 17), (4608, 129), (10240, 5), (10752, 9), (16384, 3)])
 def test_linear_q_one_token_quantizes(ctx, qtype, n_in, n_out):
