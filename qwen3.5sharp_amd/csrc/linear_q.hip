@@ -31,6 +31,8 @@
 // L2, forms one block's integer lanes per thread, and runs each row's fp32
 // accumulation on 8 threads, one per reference lane, in block order.  Extra
 // tokens reuse the staged weights.
+#include <climits>
+
 #include "common.h"
 #include "f32_stage.h"
 #include "q35mix_internal.h"
@@ -1842,14 +1844,28 @@ hipError_t launch_linear_q_prequant(q35m_ctx* c, int qtype, const void* w, const
     return launch_gemv(c, qtype, wb, qb, nullptr, y, n_in, n_out, tokens, row_base, 0);
 }
 
-// One token of Q6_K keeps the quantizer apart where the row and four waves'
-// weights would leave one workgroup a CU (29.8 against 27.5 us at 16384 ->
-// 2560; Q4_K, whose weights are in registers, 19.5 against 23.2).
+// Where quantizing the row in every workgroup costs more than a launch of the
+// quantizer (us, in the projection / apart).  Many workgroups of short rows,
+// and IQ4_XS, whose decode leaves no issue slots: Q5_K 512 -> 151936 23 / 17,
+// IQ4_XS 2560 -> 151936 45 / 38 (at 65536 22.5 / 21.6, at 12288 7.1 / 8.5),
+// STQ1_0 43 / 40.  Rows of more than 24 blocks are quantized in more than two
+// passes and leave few workgroups a CU: 9728 -> 2560 Q4_K 13.4 / 10.9 (8192 25
+// / 29), Q5_K 9.5 / 8.9 (1024 5.8 / 6.9), IQ4_XS 13.9 / 12.4, Q2_0C 12.0 / 10.9
+// (4111 15.6 / 16.3), STQ1_0 14.1 / 12.0; above 40 blocks Q6_K, with its weights
+// in LDS too, 29.8 / 27.5 at 16384 -> 2560, the others the better the more rows
+// (16384 -> 8192 Q4_K 35 / 54, Q5_K 25 / 29; 250 12.9 / 11.4, 6.5 / 7.2).
+static bool fuse_pays(int qtype, int nb, int n_out) {
+    if (nb <= 24) return n_out <= (qtype == 4 ? INT_MAX : nb <= 4 || qtype == 14 ? 49152 : qtype == 1 ? 98304 : INT_MAX);
+    if (nb <= 40)
+        return qtype == 6 || n_out <= (qtype == 4 ? 4 : 1536) || (qtype == 4 && n_out >= 6144) || (qtype == 2 && n_out >= 3072);
+    return qtype == 5 || qtype == 2 || (qtype != 6 && (n_out <= 4 || n_out >= 1024));
+}
+
 bool linear_q_fused(int qtype, const float* x, const float* y, int n_in, int n_out, int tokens) {
     // Every workgroup of the fused form reads all of x while others store y.
     const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
     const bool apart = ya >= xa + (size_t)n_in * sizeof(float) || xa >= ya + (size_t)n_out * sizeof(float);
-    return tokens == 1 && apart && !(qtype == 6 && n_in > 40 * QK);
+    return tokens == 1 && apart && fuse_pays(qtype, n_in / QK, n_out);
 }
 
 hipError_t launch_linear_q(q35m_ctx* c, int qtype, const void* w, const float* x, float* y,

@@ -107,6 +107,18 @@ def run_named(ctx, qtype, n_in, n_out, tokens, seed):
     return ran
 
 
+@pytest.mark.parametrize("qtype,n_in,n_out,fused", [
+    (4, 512, 50000, True), (5, 1024, 49152, True), (5, 1024, 49153, False), (6, 512, 50001, False), (2, 1536, 50000, True),
+    (14, 1280, 49153, False), (1, 1280, 98305, False), (4, 6400, 5, False), (4, 6400, 6145, True), (6, 6400, 2051, True),
+    (5, 9728, 1536, True), (5, 9728, 1537, False), (2, 9728, 2049, False), (2, 9728, 3073, True), (1, 9728, 4097, False),
+    (5, 10496, 100, True), (14, 10496, 100, False), (14, 10496, 1025, True), (6, 10496, 100, False), (4, 16384, 3, True)])
+def test_linear_one_token_forms(ctx, qtype, n_in, n_out, fused):
+    """One token on both sides of the rule for quantizing its row inside the
+    projection."""
+    ran = run_named(ctx, qtype, n_in, n_out, 1, 500)
+    assert GEMV_NAME[qtype] in ran and ("q8k_quantize" not in ran) == fused
+
+
 @pytest.mark.parametrize("qtype", [5, 14, 2, 1])
 @pytest.mark.parametrize("n_in,n_out,tokens,gemv", [(4096, 257, 2, True), (4096, 30, 16, True), (4096, 30, 17, False),
                                                     (9728, 41, 5, True), (16384, 19, 4, True), (3584, 331, 3, True),
