@@ -348,7 +348,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_flash(
 //
 // Scales need the magnitudes within 2^12 of each other: V rows of one kv head
 // (their scale is shared across the whole sum), and K and V rows of a tile;
-// and everything finite and below 2^40.  attn_split_prep records what it saw
+// and everything finite and below 2^40, V rows not below 2^-41.  attn_split_prep records what it saw
 // of a tile; a query block that meets anything else runs the fp32 form.
 //
 //  1. attn_split_prep: RoPE / norm of the new K rows as attn_prefill_prep, and
@@ -452,7 +452,9 @@ __global__ __launch_bounds__(SPREP) void attn_split_prep(
         vmin = min(vmin, red[w][3]);
     }
     const int ek = exp_of(kmax), ev = exp_of(vmax), ekm = kmin == ~0u ? ek : exp_of(kmin), evm = vmin == ~0u ? ev : exp_of(vmin);
-    const bool bad = ek > kMaxExp || ev > kMaxExp || ek - ekm > kMaxSpread;
+    // (V below the range of exp_of would be lost; small K only bring scores near 0.)
+    const bool tiny = vmin != ~0u && (int)(vmin >> 23) - 126 < kMinExp;
+    const bool bad = ek > kMaxExp || ev > kMaxExp || ek - ekm > kMaxSpread || tiny;
     if (threadIdx.x == 0) meta[(size_t)kvh * ntile + tile] = TileMeta{pow2(min(ek, kMaxExp) - kScaleTop), ev, evm, bad};
     const float ks = pow2(kScaleTop - min(ek, kMaxExp)), vs = pow2(kScaleTop - min(ev, kMaxExp));
 

@@ -238,9 +238,10 @@ def test_deltanet_prefill_long_context():
         np.testing.assert_array_equal(c.state_read(0, 0, q35mix.STATE_CONV), cs_ref)
 
 
-def _attn_prefill_case(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None):
+def _attn_prefill_case(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None, new_v=1.0):
     """One attention prefill of T tokens behind `start` cached rows against
-    the oracle; kmul / vmul scale single cached rows, (row, factor)."""
+    the oracle; kmul / vmul scale single cached rows, (row, factor), new_v the
+    new rows of V."""
     dims = oracle.dims(n_heads=nh, n_kv_heads=nkv)
     rng = np.random.default_rng(1000 * nh + 10 * start + T)
     wts = synth.attn_weights(256)
@@ -254,6 +255,7 @@ def _attn_prefill_case(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None):
         for row, f in mul or ():
             arr[row] *= np.float32(f)
     x = synth.attn_inputs(T, nh, nkv, 256, salt=3 + T)
+    x["v"] = x["v"] * np.float32(new_v)
     with q35mix.Context(q35mix.qwen35_config(num_layers=1, num_heads=nh, num_kv_heads=nkv, is_recurrent=[0]), n_seqs=1,
                         kv_capacity=start + T) as c:
         c.set_attn_weights(0, wts)
@@ -300,3 +302,15 @@ def test_attn_prefill_value_ranges(case):
             e = np.max(np.abs(got - want)[fin]) / np.max(np.abs(want[fin]))
             say(f"attn_prefill {case} start {start}: {e:.2e}")
             assert e <= 1e-5
+
+
+@pytest.mark.parametrize("start,T", [(0, 40), (200, 40), (3000, 37)])
+@pytest.mark.parametrize("exp", [-38, -45, -60, -90])
+def test_attn_prefill_small_values(start, T, exp):
+    """V rows of one small magnitude, in and below the range of the fp16
+    split: nothing is lost."""
+    f = 2.0 ** exp
+    got, want = _attn_prefill_case(16, 4, start, T, vmul=[(r, f) for r in range(start)], new_v=f)
+    e = np.max(np.abs(got - want)) / np.max(np.abs(want))
+    say(f"attn_prefill V of 2^{exp}, start {start}: {e:.2e}")
+    assert e <= 1e-5
