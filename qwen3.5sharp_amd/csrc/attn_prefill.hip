@@ -348,6 +348,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_flash(
 //
 // Scales need the magnitudes within 2^12 of each other: V rows of one kv head
 // (their scale is shared across the whole sum), and K and V rows of a tile;
+// the columns of a tile within 2^16 (a column of small values is a dim of the
+// output, or meets large ones of q: 2^20 apart it had 4.4e-6 in place of 1.3e-6);
 // and everything finite and below 2^40, V rows not below 2^-41.  attn_split_prep records what it saw
 // of a tile; a query block that meets anything else runs the fp32 form.
 //
@@ -367,7 +369,7 @@ constexpr int SPREP = 512, SWAVES = 8;
 // Largest workspace the split form takes (a sequence's planes are as large as
 // its K and V rows); calls past it take the fp32 form.
 constexpr size_t kSplitMaxBytes = (size_t)2 << 30;
-constexpr int kScaleTop = 14, kPTop = 10, kMinExp = -40, kMaxExp = 40, kMaxSpread = 12;
+constexpr int kScaleTop = 14, kPTop = 10, kMinExp = -40, kMaxExp = 40, kMaxSpread = 12, kMaxColSpread = 16;
 
 // What attn_split_prep saw in a tile of one kv head.
 struct TileMeta {
@@ -404,7 +406,8 @@ __global__ __launch_bounds__(SPREP) void attn_split_prep(
     float* __restrict__ V, const float* __restrict__ rope_cos, const float* __restrict__ rope_sin,
     uint4* __restrict__ planes, TileMeta* __restrict__ meta, int start, int T, int nkv, int cap, float eps) {
     __shared__ uint4 frag[SFRAGS][64];
-    __shared__ uint32_t red[8][4];
+    __shared__ uint32_t red[8][4], colexp[8][2][64];
+    __shared__ int badcol[2];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int a = wave & 3, half = wave >> 2;
     const int len = start + T, ntile = (len + ST - 1) / ST;
@@ -443,6 +446,16 @@ __global__ __launch_bounds__(SPREP) void attn_split_prep(
     if (lane == 0) {
         red[wave][0] = kmax; red[wave][1] = vmax; red[wave][2] = kmin; red[wave][3] = vmin;
     }
+    // The biased exponents of the largest values of the lane's four columns.
+    auto exps = [](const float4 (&x)[4]) {
+        auto top = [](float a, float b, float c, float d) {
+            return max(max(abs_bits(a), abs_bits(b)), max(abs_bits(c), abs_bits(d))) >> 23;
+        };
+        return top(x[0].x, x[1].x, x[2].x, x[3].x) | top(x[0].y, x[1].y, x[2].y, x[3].y) << 8 |
+               top(x[0].z, x[1].z, x[2].z, x[3].z) << 16 | top(x[0].w, x[1].w, x[2].w, x[3].w) << 24;
+    };
+    colexp[wave][0][lane] = exps(kx);
+    colexp[wave][1][lane] = exps(vx);
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < 8; ++w) {
@@ -455,7 +468,20 @@ __global__ __launch_bounds__(SPREP) void attn_split_prep(
     // (V below the range of exp_of would be lost; small K only bring scores near 0.)
     const bool tiny = vmin != ~0u && (int)(vmin >> 23) - 126 < kMinExp;
     const bool bad = ek > kMaxExp || ev > kMaxExp || ek - ekm > kMaxSpread || tiny;
-    if (threadIdx.x == 0) meta[(size_t)kvh * ntile + tile] = TileMeta{pow2(min(ek, kMaxExp) - kScaleTop), ev, evm, bad};
+    // Waves 0 and 1: K's and V's smallest nonzero column.  (A tile of one row
+    // has only its own values.)
+    if (wave < 2) {
+        int low = 255;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            int e = 0;
+#pragma unroll
+            for (int w = 0; w < 8; ++w) e = max(e, (int)((colexp[w][wave][lane] >> (8 * c)) & 255));
+            if (e) low = min(low, e);
+        }
+        low = 255 - (int)wave_umax((uint32_t)(255 - low));
+        if (lane == 0) badcol[wave] = len - ST * tile > 1 && (int)((wave ? vmax : kmax) >> 23) - low > kMaxColSpread;
+    }
     const float ks = pow2(kScaleTop - min(ek, kMaxExp)), vs = pow2(kScaleTop - min(ev, kMaxExp));
 
     // Fragments as the flash kernel's operands: 16 bytes a lane (c16, g).  K,
@@ -492,6 +518,8 @@ __global__ __launch_bounds__(SPREP) void attn_split_prep(
         reinterpret_cast<f16x4*>(&frag[f + 1][c])[half] = lo;
     }
     __syncthreads();
+    if (threadIdx.x == 0)
+        meta[(size_t)kvh * ntile + tile] = TileMeta{pow2(min(ek, kMaxExp) - kScaleTop), ev, evm, bad || badcol[0] || badcol[1]};
     uint4* dst = planes + ((size_t)kvh * ntile + tile) * SFRAGS * 64;
 #pragma unroll 4
     for (int f = wave; f < SFRAGS; f += 8) dst[64 * f + lane] = frag[f][lane ^ (f < 32 ? (f >> 1) & 7 : (f >> 1) & 15)];

@@ -238,15 +238,17 @@ def test_deltanet_prefill_long_context():
         np.testing.assert_array_equal(c.state_read(0, 0, q35mix.STATE_CONV), cs_ref)
 
 
-def _attn_prefill_case(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None, new_v=1.0):
+def _attn_prefill_case(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None, new_v=1.0, k_norm=None):
     """One attention prefill of T tokens behind `start` cached rows against
     the oracle; kmul / vmul scale single cached rows, (row, factor), new_v the
-    new rows of V."""
+    new rows of V (a number, or one a dim)."""
     dims = oracle.dims(n_heads=nh, n_kv_heads=nkv)
     rng = np.random.default_rng(1000 * nh + 10 * start + T)
     wts = synth.attn_weights(256)
     if q_norm is not None:
-        wts["q_norm"] = np.full(256, q_norm, np.float32)
+        wts["q_norm"] = np.full(256, q_norm, np.float32) if np.isscalar(q_norm) else q_norm
+    if k_norm is not None:
+        wts["k_norm"] = k_norm
     ck = np.zeros((start + T, nkv * 256), np.float32)
     cv = np.zeros_like(ck)
     ck[:start] = rng.standard_normal((start, nkv * 256))
@@ -255,7 +257,7 @@ def _attn_prefill_case(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None, new
         for row, f in mul or ():
             arr[row] *= np.float32(f)
     x = synth.attn_inputs(T, nh, nkv, 256, salt=3 + T)
-    x["v"] = x["v"] * np.float32(new_v)
+    x["v"] = x["v"] * np.tile(np.broadcast_to(np.asarray(new_v, np.float32), 256), nkv)
     with q35mix.Context(q35mix.qwen35_config(num_layers=1, num_heads=nh, num_kv_heads=nkv, is_recurrent=[0]), n_seqs=1,
                         kv_capacity=start + T) as c:
         c.set_attn_weights(0, wts)
@@ -314,3 +316,23 @@ def test_attn_prefill_small_values(start, T, exp):
     e = np.max(np.abs(got - want)) / np.max(np.abs(want))
     say(f"attn_prefill V of 2^{exp}, start {start}: {e:.2e}")
     assert e <= 1e-5
+
+
+@pytest.mark.parametrize("which", ["v", "k"])
+@pytest.mark.parametrize("exp", [15, 20, 24])
+def test_attn_prefill_column_ranges(which, exp):
+    """Dims of V, or of K with those of q the other way round, whose magnitudes
+    lie 2^exp apart: every dim of the output keeps the precision of its own
+    values (each row's largest error against the oracle over that dim's rms)."""
+    start, T = 0, 300
+    col = np.exp2(-exp * np.arange(256) / 255).astype(np.float32)
+    if which == "v":
+        got, want = _attn_prefill_case(16, 4, start, T, new_v=col)
+        e = np.max(np.abs(got - want).reshape(T, 16, 256) / np.sqrt(np.mean(want.reshape(T, 16, 256) ** 2, axis=(0, 1))))
+    else:
+        got, want = _attn_prefill_case(16, 4, start, T, k_norm=2 * col - 1, q_norm=2 / col - 1)
+        e = np.max(np.abs(got - want)) / np.sqrt(np.mean(want ** 2))
+    say(f"attn_prefill {which} columns 2^{exp} apart: {e:.2e}")
+    # Twice the 2.7e-5 that fp32 products leave here (the split alone: 2.8e-4 for
+    # V and 5.7e-4 for K at 2^24).
+    assert e <= 5e-5
