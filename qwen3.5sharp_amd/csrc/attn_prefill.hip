@@ -366,6 +366,7 @@ typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 constexpr int ST = 32;                       // key rows a tile
 constexpr int SFRAGS = 64;                   // 1 KiB operand fragments a tile: 32 K, 32 V
 constexpr int SPREP = 512, SWAVES = 8;
+constexpr int LDO = kHd + 4;                 // padded LDS row stride of the output rows
 // Largest workspace the split form takes (a sequence's planes are as large as
 // its K and V rows); calls past it take the fp32 form.
 constexpr size_t kSplitMaxBytes = (size_t)2 << 30;
@@ -548,15 +549,21 @@ __device__ __forceinline__ f32x4 mfma_h(f16x8 a, f16x8 b, f32x4 c) { return __bu
 // A part's floats in the workspace: O as each wave's registers, then (m, l) a lane.
 constexpr size_t kPartFloats = (size_t)SWAVES * 64 * 64 + (size_t)SWAVES * 64 * 2;
 
-// out = O inv sigmoid(gate) for the lane's column: registers r of block db are dims 16 db + 4 g + r.
-__device__ __forceinline__ void store_gated(float* __restrict__ orow, const float* __restrict__ grow, int d0, f32x4 o, float inv) {
-    const float4 gt = *reinterpret_cast<const float4*>(grow + d0);
-    float4 r;
-    r.x = o[0] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-gt.x));
-    r.y = o[1] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-gt.y));
-    r.z = o[2] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-gt.z));
-    r.w = o[3] * inv * __builtin_amdgcn_rcpf(1.0f + __expf(-gt.w));
-    *reinterpret_cast<float4*>(orow + d0) = r;
+// 1 / (1 + e^-x) to fp32 precision in a dozen instructions: the exponential
+// with the rounding error of its base-2 argument made good, the reciprocal
+// with one Newton step (expf and a division are 45).
+__device__ __forceinline__ float sigmoid_full(float x) {
+    const float n = __builtin_amdgcn_fmed3f(-x, -88.0f, 88.0f);    // (past it 0 and 1 in any case)
+    const float l2 = 1.44269502e+0f, l2lo = 1.92596303e-8f, ln2 = 0.693147182f;   // log2(e) as a sum, ln 2
+    const float t = n * l2, d = fmaf(n, l2lo, fmaf(n, l2, -t));
+    const float p = __builtin_amdgcn_exp2f(t), s = 1.0f + fmaf(p * ln2, d, p);
+    const float r = __builtin_amdgcn_rcpf(s);
+    return x != x ? x : fmaf(fmaf(-s, r, 1.0f), r, r);
+}
+
+__device__ __forceinline__ float4 gated(float4 o, float4 gate) {
+    return make_float4(o.x * sigmoid_full(gate.x), o.y * sigmoid_full(gate.y), o.z * sigmoid_full(gate.z),
+                       o.w * sigmoid_full(gate.w));
 }
 
 // Slot of a block's chunk in the parts.
@@ -577,10 +584,12 @@ __global__ __launch_bounds__(64 * SWAVES, 2) void attn_split_flash(
     const uint4* __restrict__ planes, const TileMeta* __restrict__ meta, QRows Q, const float* __restrict__ K,
     const float* __restrict__ V, int cap, float* __restrict__ out, float* __restrict__ parts, int* __restrict__ fp32_done,
     SplitPlan P, SplitItems items) {
-    // K and V operands of two tiles (128 KiB), or the fp32 form's tiles.
+    // K and V operands of two tiles (128 KiB), or the fp32 form's tiles, or the
+    // waves' output rows.
     __shared__ union {
         struct { uint4 k[2][SFRAGS / 2][64], v[2][SFRAGS / 2][64]; } t;
         Tiles fp32[2];
+        float rows[SWAVES][16][LDO];
     } lds;
     __shared__ int red[4][SWAVES];
     const float* q_gate = Q.q_gate;
@@ -854,12 +863,45 @@ __global__ __launch_bounds__(64 * SWAVES, 2) void attn_split_flash(
     l_run = xor16_sum(l_run);
     l_run = xor32_sum(l_run);
     if (n <= P.chunk) {
-        if (row < P.T) {
-            const float inv = pow2(evmax - kPTop - kScaleTop) / l_run;
-            const float* grow = q_gate + ((size_t)row * P.nh + h) * 2 * kHd + kHd;
-            float* orow = out + ((size_t)row * P.nh + h) * kHd;
+        // The item's rows go through LDS (the tiles', once every wave is past
+        // them) and on to the waves in turn, so that a gate load and a store
+        // cover a whole row and a few rows share all waves; four rows a step,
+        // in a loop, as code that runs once costs its fetch (stored from the
+        // accumulators' own lanes, a call of one token took 6 us more).
+        const float inv = pow2(evmax - kPTop - kScaleTop) / l_run;
+        const int hs = __builtin_ctz(P.hg), t_base = P.rows * qb, n_rows = min(P.rows, P.T - t_base) << hs;
+        struct RowAt { size_t at; int lds; };
+        auto row_at = [&](int step, int i) {
+            const int q = min(wave + SWAVES * (4 * step + i), n_rows - 1), t = q >> hs, hh = q & (P.hg - 1);
+            return RowAt{((size_t)(t_base + t) * P.nh + P.hg * y + hh) * kHd, (((t >> 4) * P.hg + hh) * 16 + (t & 15)) * LDO};
+        };
+        float4 gate[4];
+        auto load_gates = [&](int step) {
 #pragma unroll
-            for (int db = 0; db < 16; ++db) store_gated(orow, grow, 16 * db + 4 * g, O[db], inv);
+            for (int i = 0; i < 4; ++i) gate[i] = *reinterpret_cast<const float4*>(q_gate + 2 * row_at(step, i).at + kHd + 4 * lane);
+        };
+        load_gates(0);
+        lds_barrier();
+#pragma unroll
+        for (int db = 0; db < 16; ++db)
+            *reinterpret_cast<f32x4*>(&lds.rows[wave][c16][16 * db + 4 * g]) = O[db] * inv;
+        lds_barrier();
+        const float* rows = &lds.rows[0][0][0];
+#pragma unroll 1
+        for (int step = 0; wave + SWAVES * 4 * step < n_rows; ++step) {
+            const float4 now[4] = {gate[0], gate[1], gate[2], gate[3]};
+            load_gates(step + 1);
+            float4 o[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = *reinterpret_cast<const float4*>(rows + row_at(step, i).lds + 4 * lane);
+            // The first position (a wave's first row) attends to itself alone: its V as it is.
+            if (P.start + t_base + step == 0 && wave < P.hg)
+                o[0] = *reinterpret_cast<const float4*>(V + (size_t)kvh * cap * kHd + 4 * lane);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                o[i] = gated(o[i], now[i]);
+                if (wave + SWAVES * (4 * step + i) < n_rows) *reinterpret_cast<float4*>(out + row_at(step, i).at + 4 * lane) = o[i];
+            }
         }
     } else {
         float* po = parts + part_slot(P, qb, c, y);
@@ -929,10 +971,15 @@ __global__ __launch_bounds__(256) void attn_split_merge(const TileMeta* __restri
         add(xml[i][lane], x);
     }
     const float inv = pow2(ev - kPTop - kScaleTop) / l;
-    const float* grow = q_gate + ((size_t)row * P.nh + h) * 2 * kHd + kHd;
-    float* orow = out + ((size_t)row * P.nh + h) * kHd;
+    const float* grow = q_gate + ((size_t)row * P.nh + h) * 2 * kHd + kHd + 64 * d4 + 4 * g;
+    float* orow = out + ((size_t)row * P.nh + h) * kHd + 64 * d4 + 4 * g;
+    float4 gate[4];
 #pragma unroll
-    for (int d = 0; d < 4; ++d) store_gated(orow, grow, 16 * (4 * d4 + d) + 4 * g, o[d], inv);
+    for (int d = 0; d < 4; ++d) gate[d] = *reinterpret_cast<const float4*>(grow + 16 * d);
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+        *reinterpret_cast<float4*>(orow + 16 * d) =
+            gated(make_float4(o[d][0] * inv, o[d][1] * inv, o[d][2] * inv, o[d][3] * inv), gate[d]);
 }
 
 }  // namespace
