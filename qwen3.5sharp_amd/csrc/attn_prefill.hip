@@ -376,7 +376,7 @@ constexpr int kScaleTop = 14, kPTop = 10, kMinExp = -40, kMaxExp = 40, kMaxSprea
 struct TileMeta {
     float kdesc;          // 2^(ek - 14): K = (hi + lo) kdesc
     int ev;               // exponent of V's largest value: V = (hi + lo) 2^(ev - 14)
-    int ev_min;           // exponent of the smallest nonzero row of V
+    int ev_min;           // exponent of the smallest nonzero row of V (kMaxExp: none)
     int bad;              // a value outside the range above
 };
 
@@ -465,7 +465,8 @@ __global__ __launch_bounds__(SPREP) void attn_split_prep(
         kmin = min(kmin, red[w][2]);
         vmin = min(vmin, red[w][3]);
     }
-    const int ek = exp_of(kmax), ev = exp_of(vmax), ekm = kmin == ~0u ? ek : exp_of(kmin), evm = vmin == ~0u ? ev : exp_of(vmin);
+    const int ek = exp_of(kmax), ev = exp_of(vmax), ekm = kmin == ~0u ? ek : exp_of(kmin);
+    const int evm = vmin == ~0u ? kMaxExp : exp_of(vmin);      // (rows of zeros have no place in the spread)
     // (V below the range of exp_of would be lost; small K only bring scores near 0.)
     const bool tiny = vmin != ~0u && (int)(vmin >> 23) - 126 < kMinExp;
     const bool bad = ek > kMaxExp || ev > kMaxExp || ek - ekm > kMaxSpread || tiny;

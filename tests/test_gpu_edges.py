@@ -7,6 +7,7 @@ import sys
 import numpy as np
 import pytest
 
+import f64_model
 import oracle
 import q35mix
 import synth
@@ -238,11 +239,8 @@ def test_deltanet_prefill_long_context():
         np.testing.assert_array_equal(c.state_read(0, 0, q35mix.STATE_CONV), cs_ref)
 
 
-def _attn_prefill_case(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None, new_v=1.0, k_norm=None):
-    """One attention prefill of T tokens behind `start` cached rows against
-    the oracle; kmul / vmul scale single cached rows, (row, factor), new_v the
-    new rows of V (a number, or one a dim)."""
-    dims = oracle.dims(n_heads=nh, n_kv_heads=nkv)
+def _attn_prefill_data(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None, new_v=1.0, k_norm=None):
+    """Inputs, weights and cached rows (keys, values) of an attention prefill."""
     rng = np.random.default_rng(1000 * nh + 10 * start + T)
     wts = synth.attn_weights(256)
     if q_norm is not None:
@@ -258,6 +256,15 @@ def _attn_prefill_case(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None, new
             arr[row] *= np.float32(f)
     x = synth.attn_inputs(T, nh, nkv, 256, salt=3 + T)
     x["v"] = x["v"] * np.tile(np.broadcast_to(np.asarray(new_v, np.float32), 256), nkv)
+    return x, wts, ck, cv
+
+
+def _attn_prefill_case(nh, nkv, start, T, kmul=None, vmul=None, q_norm=None, new_v=1.0, k_norm=None):
+    """One attention prefill of T tokens behind `start` cached rows against
+    the oracle; kmul / vmul scale single cached rows, (row, factor), new_v the
+    new rows of V (a number, or one a dim)."""
+    dims = oracle.dims(n_heads=nh, n_kv_heads=nkv)
+    x, wts, ck, cv = _attn_prefill_data(nh, nkv, start, T, kmul, vmul, q_norm, new_v, k_norm)
     with q35mix.Context(q35mix.qwen35_config(num_layers=1, num_heads=nh, num_kv_heads=nkv, is_recurrent=[0]), n_seqs=1,
                         kv_capacity=start + T) as c:
         c.set_attn_weights(0, wts)
@@ -336,3 +343,24 @@ def test_attn_prefill_column_ranges(which, exp):
     # Twice the 2.7e-5 that fp32 products leave here (the split alone: 2.8e-4 for
     # V and 5.7e-4 for K at 2^24).
     assert e <= 5e-5
+
+
+def _attn_f64_error(start, T, got, **kw):
+    """2-norm of the difference to the float64 model over the model's."""
+    x, wts, ck, cv = _attn_prefill_data(16, 4, start, T, **kw)
+    want, _, _ = f64_model.attn(start, x["q_gate"], x["k"], x["v"], wts, ck, cv, 16, 4, 256)
+    want = want.reshape(T, -1)
+    return np.linalg.norm(got - want) / np.linalg.norm(want)
+
+
+def test_attn_prefill_zero_tile_stays_split():
+    """A tile of 32 zero V rows is within the split's range: the result keeps
+    the split's distance to 64 bits, about half of the fp32 products' (5.8e-7
+    and 1.2e-6 at this size), and so does one with half of them zero."""
+    start, T = 3000, 37
+    for rows in (range(64, 96), range(64, 80)):
+        kw = {"vmul": [(r, 0.0) for r in rows]}
+        got, _ = _attn_prefill_case(16, 4, start, T, **kw)
+        e = _attn_f64_error(start, T, got, **kw)
+        say(f"attn_prefill {len(rows)} zero V rows: {e:.2e}")
+        assert e <= 8e-7
