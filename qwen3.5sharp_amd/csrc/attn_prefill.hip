@@ -698,13 +698,13 @@ __global__ __launch_bounds__(64 * SWAVES, 2) void attn_split_flash(
                 ql[k][j] = (_Float16)(v - (float)hi);
             }
     }
-    // The V scale of the sum, the kv head's largest exponent; and whether
-    // everything is within the split's range, the same for all of a block's
-    // chunks.
+    // The V scale of the sum, the largest exponent of the tiles that the block
+    // reads; and whether they are within the split's range, the same for all
+    // of a block's chunks.
     int evmax = kMinExp;
     {
         int evmin = kMaxExp;
-        for (int i = tid; i < P.ntile; i += 64 * SWAVES) {
+        for (int i = tid; i < n; i += 64 * SWAVES) {
             evmax = max(evmax, meta[i].ev);
             evmin = min(evmin, meta[i].ev_min);
             bad |= meta[i].bad != 0;
@@ -925,7 +925,7 @@ __global__ __launch_bounds__(256) void attn_split_merge(const TileMeta* __restri
     const int row0 = P.rows * qb + 16 * (wave / P.hg), row = row0 + c16;
     const int h = P.hg * y + wave % P.hg;
     if (row0 >= P.T || fp32_done[blockIdx.z * P.groups + y]) return;
-    const int kvh = y * P.hg / (P.nh / P.nkv), nch = (P.tiles(qb) + P.chunk - 1) / P.chunk;
+    const int kvh = y * P.hg / (P.nh / P.nkv), n = P.tiles(qb), nch = (n + P.chunk - 1) / P.chunk;
     float m = -1e30f, l = 0.0f;
     f32x4 o[4];
 #pragma unroll
@@ -959,7 +959,7 @@ __global__ __launch_bounds__(256) void attn_split_merge(const TileMeta* __restri
     }
     int ev = kMinExp;
     if (w == 0) {
-        for (int i = lane; i < P.ntile; i += kWave) ev = max(ev, meta[(size_t)kvh * P.ntile + i].ev);
+        for (int i = lane; i < n; i += kWave) ev = max(ev, meta[(size_t)kvh * P.ntile + i].ev);
         ev = min((int)wave_umax((uint32_t)(ev + 1024)) - 1024, kMaxExp);
     }
     __syncthreads();

@@ -364,3 +364,28 @@ def test_attn_prefill_zero_tile_stays_split():
         e = _attn_f64_error(start, T, got, **kw)
         say(f"attn_prefill {len(rows)} zero V rows: {e:.2e}")
         assert e <= 8e-7
+
+
+@pytest.mark.parametrize("start,T", [(0, 300), (500, 200), (6000, 100)])
+@pytest.mark.parametrize("value", [2.0 ** 30, 2.0 ** 60, 2.0 ** -60, np.inf])
+def test_attn_prefill_late_values(start, T, value):
+    """V outside the split's range in the last row: the query blocks (32 rows)
+    that do not read its tile (32 rows from row 0 of the cache) have the bits
+    they have without it."""
+    import unittest.mock
+    real = synth.attn_inputs
+
+    def late(*a, **k):
+        x = real(*a, **k)
+        x["v"] = x["v"].copy()
+        x["v"][-1] *= np.float32(value)
+        return x
+
+    plain, _ = _attn_prefill_case(16, 4, start, T)
+    with unittest.mock.patch.object(synth, "attn_inputs", late):
+        got, want = _attn_prefill_case(16, 4, start, T)
+    before = max(32 * b for b in range(T // 32 + 1) if (start + 32 * b + 31) // 32 <= (start + T - 1) // 32)
+    assert before > 0 and np.array_equal(got[:before].view(np.uint32), plain[:before].view(np.uint32))
+    if np.isfinite(value):      # (an infinity times the 0 of a masked weight is NaN for the rows of its 16)
+        for t in range(before, T):
+            assert np.max(np.abs(got[t] - want[t])) <= 1e-5 * np.max(np.abs(want[t]))
