@@ -90,10 +90,11 @@ struct QRows {
     float eps;
 };
 
-// Query block qb of head group y; every thread of the workgroup's 8 waves.
+// Query block qb (16 subs rows) of head group y; every thread of the
+// workgroup's 8 waves.  With subs > 1 the spare waves take further 16 rows.
 __device__ __forceinline__ void flash_fp32_block(
     Tiles* smem, const QRows& Q, const float* __restrict__ K, const float* __restrict__ V,
-    float* __restrict__ out, int start, int T, int nh, int nkv, int hg, int cap, int qb, int y) {
+    float* __restrict__ out, int start, int T, int nh, int nkv, int hg, int cap, int qb, int y, int subs) {
     const float* q_gate = Q.q_gate;
     const int kvh = y * hg / (nh / nkv);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -102,10 +103,10 @@ __device__ __forceinline__ void flash_fp32_block(
     const int half = __builtin_amdgcn_readfirstlane(tid >> 8);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, htid = tid & 255;
     const int g = lane >> 4, c16 = lane & 15;
-    const bool stores = wave < hg;           // uniform per wave
-    const int h = hg * y + min(wave, hg - 1);
-    const int r0 = qb * QR;
-    const int blk_len = start + min(T - 1, r0 + QR - 1) + 1;
+    const bool stores = wave < hg * subs;    // uniform per wave
+    const int unit = min(wave, hg * subs - 1), h = hg * y + unit % hg;
+    const int r0 = (qb * subs + unit / hg) * QR;
+    const int blk_len = start + min(T - 1, (qb + 1) * subs * QR - 1) + 1;
     const int my_t = min(r0 + c16, T - 1);
     const int my_len = start + my_t + 1;
     // Key tiles of this half: [t_begin, t_begin + n_iter), the last one past
@@ -334,7 +335,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_flash(
     __shared__ Tiles smem[2];
     const int groups = nh / hg, nqb = (T + QR - 1) / QR;
     const int rank = blockIdx.x;                 // heaviest query blocks first
-    flash_fp32_block(smem, Q, K, V, out, start, T, nh, nkv, hg, cap, nqb - 1 - rank / groups, rank % groups);
+    flash_fp32_block(smem, Q, K, V, out, start, T, nh, nkv, hg, cap, nqb - 1 - rank / groups, rank % groups, 1);
 }
 
 // ---------------------------------------------------------------- split fp16
@@ -729,11 +730,16 @@ __global__ __launch_bounds__(64 * SWAVES, 2) void attn_split_flash(
     }
     if (c == 0 && tid == 0 && n > P.chunk) fp32_done[(qb - P.first_multi) * P.groups + y] = bad;
     if (bad) {
-        if (c > 0) return;
+        // The block's rows in two halves, one to each of its first two chunks'
+        // workgroups (133 tokens behind 8000 rows of 4 q heads a kv head 1160
+        // us, of one 1174; all in the first chunk's, 16 rows after another, 2299
+        // and 9078; the fp32 kernels alone 1097).  A block of one chunk has
+        // them after one another (64 tokens 62, the fp32 kernels 25).
+        const int subs = 4 / P.hg, nch = (n + P.chunk - 1) / P.chunk;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        for (int b = P.rows / QR * qb; b < P.rows / QR * (qb + 1) && b * QR < P.T; ++b) {
+        for (int b = c; b < 2 && (2 * qb + b) * subs * QR < P.T; b += nch) {
             __syncthreads();
-            flash_fp32_block(lds.fp32, Q, K, V, out, P.start, P.T, P.nh, P.nkv, P.hg, cap, b, y);
+            flash_fp32_block(lds.fp32, Q, K, V, out, P.start, P.T, P.nh, P.nkv, P.hg, cap, 2 * qb + b, y, subs);
         }
         return;
     }

@@ -389,3 +389,16 @@ def test_attn_prefill_late_values(start, T, value):
     if np.isfinite(value):      # (an infinity times the 0 of a masked weight is NaN for the rows of its 16)
         for t in range(before, T):
             assert np.max(np.abs(got[t] - want[t])) <= 1e-5 * np.max(np.abs(want[t]))
+
+
+@pytest.mark.parametrize("nh,nkv", [(16, 4), (8, 4), (4, 4), (8, 1)])
+@pytest.mark.parametrize("start,T", [(0, 1), (0, 17), (3, 130), (2500, 34), (2500, 131)])
+def test_attn_prefill_all_out_of_range(nh, nkv, start, T):
+    """Every query block in the fp32 form (a row 2^20 times the others in the
+    first tile), in one chunk and shared out over several, for 1, 2 and 4 q
+    heads a workgroup."""
+    kw = {"vmul": [(1, 2.0 ** 20)]} if start else {"new_v": np.exp2(np.where(np.arange(256) % 2, 20, 0))}
+    got, want = _attn_prefill_case(nh, nkv, start, T, **kw)
+    e = np.max(np.abs(got - want)) / np.max(np.abs(want))
+    say(f"attn_prefill fp32 form {nh}/{nkv} start {start} T {T}: {e:.2e}")
+    assert e <= 1e-5
