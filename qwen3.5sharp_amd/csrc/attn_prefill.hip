@@ -993,6 +993,9 @@ __global__ __launch_bounds__(256) void attn_split_merge(const TileMeta* __restri
 
 namespace {
 
+// Parts of a head group's chunked query blocks at most.
+long max_parts(const SplitPlan& p, int slots) { return 2L * (slots + p.nqb); }
+
 // Chunks from the share of one workgroup a CU, longer until the items of more
 // than half a chunk fit the CUs once (two of them would share one).
 SplitPlan plan_split(const Dims& d, int n_cu, int start, int T) {
@@ -1014,12 +1017,13 @@ SplitPlan plan_split(const Dims& d, int n_cu, int start, int T) {
     if (p.nqb >= 2 * slots) chunk = p.ntile;
     chunk = std::max(chunk, (p.ntile + 63) / 64);              // the item list's 6 bits
     for (; chunk < p.ntile; chunk += std::max(1, chunk / 32)) {
-        int big = 0;
+        int big = 0, multi = 0;
         for (int q = 0; q < p.nqb; ++q) {
             const int n = p.tiles(q);
             big += n / chunk + (2 * (n % chunk) > chunk);
+            multi += n > chunk;
         }
-        if (big <= slots) break;
+        if (big <= slots && (long)multi * ((p.ntile + chunk - 1) / chunk) <= max_parts(p, slots)) break;
     }
     p.chunk = std::min(chunk, p.ntile);
     p.maxch = (p.ntile + p.chunk - 1) / p.chunk;
@@ -1059,19 +1063,37 @@ struct SplitWork {
     }
 };
 
-}  // namespace
-
-// The split form's workspace, 0 where the call takes the fp32 form (which needs none).
-size_t attn_prefill_split_bytes(const q35m_ctx* c, int start, int T) {
-    const SplitPlan p = plan_split(c->d, c->n_cu, start, T);
-    const SplitWork w(p);
-    // A kv head's planes are addressed through one buffer descriptor.
-    if ((size_t)p.ntile * SFRAGS * 1024 > c->tile_limit || w.bytes > kSplitMaxBytes) return 0;
-    return w.bytes;
+// Workspace of any split call of T tokens on this context: one of its
+// capacity, so that it is allocated once and not again as a sequence grows
+// (nor under a stream capture after one call of as many tokens).
+size_t split_reserve(const q35m_ctx* c, const SplitPlan& p) {
+    const int slots = std::max(1, c->n_cu / p.groups);
+    const long ntile = ((long)c->cap + ST - 1) / ST, chunks = (ntile + 3) / 4;
+    const long parts = chunks > 1 && p.nqb < 2 * slots ? std::min<long>(max_parts(p, slots), p.nqb * chunks) : 0;
+    const size_t bytes = align256((size_t)p.nqb * p.groups * sizeof(int)) + align256((size_t)p.nkv * ntile * sizeof(TileMeta)) +
+                         (size_t)p.nkv * ntile * SFRAGS * 1024 + (size_t)parts * p.groups * kPartFloats * sizeof(float) + 768;
+    return std::min(bytes, kSplitMaxBytes);
 }
 
+// Whether the call takes the split form, with its workspace in place.  A size
+// that could not be had is not asked for again.
+bool split_ready(q35m_ctx* c, const SplitPlan& p, size_t bytes) {
+    // A kv head's planes are addressed through one buffer descriptor.
+    if ((size_t)p.ntile * SFRAGS * 1024 > c->tile_limit || bytes > kSplitMaxBytes) return false;
+    for (const size_t n : {std::max(bytes, split_reserve(c, p)), bytes}) {
+        if (n <= c->work_bytes) return true;
+        if (n >= c->split_refused) continue;
+        if (ensure_work(c, n) == hipSuccess) return true;
+        (void)hipGetLastError();
+        c->split_refused = n;
+    }
+    return false;
+}
+
+}  // namespace
+
 hipError_t launch_attn_prefill(q35m_ctx* c, int layer, int seq, int start, int T,
-                               const float* q_gate, const float* k, const float* v, float* out, bool split) {
+                               const float* q_gate, const float* k, const float* v, float* out) {
     const Dims& d = c->d;
     const AttnLayer& L = c->full[layer];
     float* K = L.k_cache + (size_t)seq * c->cap * d.kv_dim;
@@ -1079,9 +1101,9 @@ hipError_t launch_attn_prefill(q35m_ctx* c, int layer, int seq, int start, int T
     const QRows Q{q_gate, L.q_norm, c->rope_cos, c->rope_sin, d.eps};
     // Head groups of up to 4 q heads of one kv head.
     const int g = d.nh / d.nkv, hg = g < 4 ? g : 4;
-    if (split) {
-        const SplitPlan p = plan_split(d, c->n_cu, start, T);
-        const SplitWork wk(p);
+    const SplitPlan p = plan_split(d, c->n_cu, start, T);
+    const SplitWork wk(p);
+    if (split_ready(c, p, wk.bytes)) {
         char* base = reinterpret_cast<char*>(c->work);
         int* fp32_done = reinterpret_cast<int*>(base + wk.fp32_done);
         TileMeta* meta = reinterpret_cast<TileMeta*>(base + wk.meta);

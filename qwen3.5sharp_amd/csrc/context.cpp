@@ -602,11 +602,7 @@ int q35m_attn_prefill(q35m_ctx* ctx, int layer, int seq, int T, const float* q_g
     if ((long)start + T > q35::kPrefillMaxRows)
         return fail(Q35M_ERR_UNSUPPORTED, "attention prefill reads at most %d cached rows (sequence %d "
                     "would reach %d)", q35::kPrefillMaxRows, seq, start + T);
-    // Without room for the split form's workspace the call takes the fp32 form.
-    const size_t split = q35::attn_prefill_split_bytes(ctx, start, T);
-    const bool ok = split && q35::ensure_work(ctx, split) == hipSuccess;
-    if (!ok) (void)hipGetLastError();
-    HIP_TRY(q35::launch_attn_prefill(ctx, layer, seq, start, T, q_gate, k, v, out, ok), "attn_prefill");
+    HIP_TRY(q35::launch_attn_prefill(ctx, layer, seq, start, T, q_gate, k, v, out), "attn_prefill");
     return Q35M_OK;
 }
 

@@ -148,6 +148,7 @@ struct q35m_ctx {
     int rope_cap = 0;
     float* work = nullptr;             // scratch for split-K partials and prefill
     size_t work_bytes = 0;
+    size_t split_refused = ~(size_t)0;   // smallest workspace of the split attention prefill that could not be had
     float* noalloc_scratch = nullptr;  // the device's fixed scratch (q35m_attn_decode_noalloc)
     // Largest weight or activation piece (bytes) one tiled-projection launch
     // addresses: 2 GiB (32-bit buffer offsets); the environment variable
@@ -201,10 +202,7 @@ constexpr size_t kNoAllocScratchBytes = Q35M_NOALLOC_SCRATCH_BYTES;
 // current; each device has its own copy).
 hipError_t attn_decode_scratch_address(float** ptr);
 hipError_t launch_attn_prefill(q35m_ctx* c, int layer, int seq, int start, int T,
-                               const float* q_gate, const float* k, const float* v, float* out, bool split);
-// Workspace of the split-fp16 form (0: the call takes the fp32 form, which
-// needs none).
-size_t attn_prefill_split_bytes(const q35m_ctx* c, int start, int T);
+                               const float* q_gate, const float* k, const float* v, float* out);
 hipError_t launch_linear_q(q35m_ctx* c, int qtype, const void* w, const float* x, float* y,
                            int n_in, int n_out, int tokens);
 // Q5_K, IQ4_XS, Q2_0C and STQ1_0 projections of several tokens on the matrix

@@ -2,6 +2,7 @@
 every branch of the prefill scan's loop, the 64-sequence decode batch, the
 last KV row and the limits the ABI enforces.  Parity gate as in
 test_gpu_mixers.py: max|gpu - oracle| / max|oracle| <= 1e-4."""
+import ctypes
 import sys
 
 import numpy as np
@@ -402,3 +403,72 @@ def test_attn_prefill_all_out_of_range(nh, nkv, start, T):
     e = np.max(np.abs(got - want)) / np.max(np.abs(want))
     say(f"attn_prefill fp32 form {nh}/{nkv} start {start} T {T}: {e:.2e}")
     assert e <= 1e-5
+
+
+def _turns_context(cap):
+    c = q35mix.Context(q35mix.qwen35_config(num_layers=1, num_heads=16, num_kv_heads=4, is_recurrent=[0]), n_seqs=1,
+                       kv_capacity=cap)
+    c.set_attn_weights(0, synth.attn_weights(256))
+    k, v = synth.kv_prefill(cap, 1024, salt=77)
+    c.state_write(0, 0, q35mix.STATE_KEYS, k)
+    c.state_write(0, 0, q35mix.STATE_VALUES, v)
+    c.truncate(0, 0)
+    x = synth.attn_inputs(20, 16, 4, 256, salt=5)
+    args = [c.array((20, 8192), x["q_gate"]), c.array((20, 1024), x["k"]), c.array((20, 1024), x["v"]), c.array((20, 4096))]
+    return c, args
+
+
+def test_attn_prefill_workspace_allocated_once():
+    """The turns of a growing conversation need no more device memory than
+    its first one: the workspace is one of the context's capacity."""
+    hip = q35mix.hip()
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    c, args = _turns_context(6000)
+    with c:
+        c.attn_prefill(0, 0, 20, *args)
+        c.sync()
+        first = free()
+        for start in (900, 3000, 5980):
+            c.advance(0, start - c.kv_len(0))
+            c.attn_prefill(0, 0, 20, *args)
+            c.sync()
+            assert free() == first
+
+
+def test_attn_prefill_under_graph_capture():
+    """A turn captured into a HIP graph behind more rows than the call that
+    warmed the context up: three replays, with eager work between them, each
+    equal bit for bit to the eager call."""
+    hip = q35mix.hip()
+    c, args = _turns_context(4100)
+    with c:
+        c.attn_prefill(0, 0, 20, *args)
+        c.sync()
+        c.advance(0, 4000)
+        stream, graph, exe = ctypes.c_void_p(c.stream), ctypes.c_void_p(), ctypes.c_void_p()
+        assert hip.hipStreamBeginCapture(stream, 0) == 0
+        try:
+            c.attn_prefill(0, 0, 20, *args)
+        finally:
+            r_end = hip.hipStreamEndCapture(stream, ctypes.byref(graph))
+        assert r_end == 0
+        assert hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)) == 0
+        try:
+            for rep in range(3):
+                args[3].upload(np.zeros((20, 4096), np.float32))
+                assert hip.hipGraphLaunch(exe, stream) == 0
+                c.sync()
+                got = args[3].download()
+                args[3].upload(np.zeros((20, 4096), np.float32))
+                c.attn_prefill(0, 0, 20, *args)
+                c.sync()
+                assert np.array_equal(got.view(np.uint32), args[3].download().view(np.uint32))
+                assert np.any(got)
+        finally:
+            assert hip.hipGraphExecDestroy(exe) == 0
+            assert hip.hipGraphDestroy(graph) == 0
