@@ -298,8 +298,8 @@ def test_attn_prefill_chunks(nh, nkv, start, T):
 @pytest.mark.parametrize("case", ["v_spread", "k_spread", "v_zero_rows", "huge_v", "q_huge", "v_inf", "v_nan"])
 def test_attn_prefill_value_ranges(case):
     """Cached rows whose magnitudes lie far apart, huge or not finite, and q
-    beyond the split's range: the query blocks that meet them take the fp32
-    form (one chunk and many), the others keep theirs."""
+    beyond the split's range: the query blocks that read them take the fp32
+    form (one chunk and many); a tile of zero rows stays."""
     for start, T in ((200, 40), (3000, 37)):
         kw = {"v_spread": {"vmul": [(50, 2.0 ** 20)]}, "k_spread": {"kmul": [(60, 2.0 ** -15)]},
               "v_zero_rows": {"vmul": [(r, 0.0) for r in range(64, 96)]}, "huge_v": {"vmul": [(r, 1e25) for r in range(start)]},
@@ -472,3 +472,66 @@ def test_attn_prefill_under_graph_capture():
         finally:
             assert hip.hipGraphExecDestroy(exe) == 0
             assert hip.hipGraphDestroy(graph) == 0
+
+
+@pytest.mark.parametrize("nh,nkv,start,T", [(16, 4, 0, 1), (16, 4, 31, 33), (16, 4, 300, 65), (4, 4, 100, 129), (8, 4, 63, 65),
+                                            (8, 1, 700, 40), (16, 2, 0, 34)])
+def test_attn_prefill_fp32_kernels(monkeypatch, nh, nkv, start, T):
+    """The kernels that take a call without room for the split form's
+    workspace (here by a 1-byte limit on what a descriptor covers): output and
+    new cache rows, 1, 2, 4 and 8 q heads a kv head."""
+    monkeypatch.setenv("Q35M_TILE_LIMIT_BYTES", "1")
+    dims = oracle.dims(n_heads=nh, n_kv_heads=nkv)
+    x, wts, ck, cv = _attn_prefill_data(nh, nkv, start, T)
+    with q35mix.Context(q35mix.qwen35_config(num_layers=1, num_heads=nh, num_kv_heads=nkv, is_recurrent=[0]), n_seqs=1,
+                        kv_capacity=start + T) as c:
+        c.set_attn_weights(0, wts)
+        if start:
+            c.state_write(0, 0, q35mix.STATE_KEYS, ck[:start])
+            c.state_write(0, 0, q35mix.STATE_VALUES, cv[:start])
+            if c.kv_len(0) < start:
+                c.advance(0, start - c.kv_len(0))
+        out = c.array((T, nh * 256))
+        c.profile(True)
+        c.attn_prefill(0, 0, T, c.array((T, 2 * nh * 256), x["q_gate"]), c.array((T, nkv * 256), x["k"]),
+                       c.array((T, nkv * 256), x["v"]), out)
+        ran = c.profile_read()
+        c.profile(False)
+        assert sorted(ran) == ["attn_prefill_flash", "attn_prefill_prep"]
+        got = out.download()
+        rows = [c.state_read(0, 0, kind, start + T)[start:] for kind in (q35mix.STATE_KEYS, q35mix.STATE_VALUES)]
+    want, k_all, _ = oracle.attn_prefill(dims, start, T, x["q_gate"], x["k"], x["v"], wts, ck, cv, n_threads=8)
+    e = np.max(np.abs(got - want)) / np.max(np.abs(want))
+    say(f"attn_prefill fp32 kernels {nh}/{nkv} start {start} T {T}: {e:.2e}")
+    assert e <= 1e-5
+    k_new = k_all.reshape(start + T, -1)[start:]
+    assert np.max(np.abs(rows[0].reshape(T, -1) - k_new)) <= 1e-5 * np.max(np.abs(k_new))
+    assert np.array_equal(rows[1].reshape(T, -1), x["v"].reshape(T, -1))
+
+
+def test_attn_prefill_long_prompt():
+    """A prompt of more query blocks than the item list holds (the grid goes
+    block by block): rows of its first, middle and last blocks against the
+    oracle run from there over the cache's own earlier rows."""
+    nh, nkv, T = 4, 1, 16500
+    dims = oracle.dims(n_heads=nh, n_kv_heads=nkv)
+    wts = synth.attn_weights(256)
+    x = synth.attn_inputs(T, nh, nkv, 256, salt=91)
+    with q35mix.Context(q35mix.qwen35_config(num_layers=1, num_heads=nh, num_kv_heads=nkv, is_recurrent=[0]), n_seqs=1,
+                        kv_capacity=T) as c:
+        c.set_attn_weights(0, wts)
+        out = c.array((T, nh * 256))
+        c.attn_prefill(0, 0, T, c.array((T, 2 * nh * 256), x["q_gate"]), c.array((T, nkv * 256), x["k"]),
+                       c.array((T, nkv * 256), x["v"]), out)
+        got = out.download()
+        keys, values = (c.state_read(0, 0, kind, T).reshape(T, nkv * 256) for kind in (q35mix.STATE_KEYS, q35mix.STATE_VALUES))
+    assert np.array_equal(values, x["v"].reshape(T, -1))
+    for t0, n in ((0, 40), (8170, 40), (16384, 20), (T - 33, 33)):
+        sl = slice(t0, t0 + n)
+        want, k_all, _ = oracle.attn_prefill(dims, t0, n, x["q_gate"][sl], x["k"][sl], x["v"][sl], wts, keys[:t0 + n].copy(),
+                                             values[:t0 + n].copy(), n_threads=8)
+        e = np.max(np.abs(got[sl] - want)) / np.max(np.abs(want))
+        say(f"attn_prefill rows {t0}..{t0 + n} of {T}: {e:.2e}")
+        assert e <= 1e-5
+        k_new = k_all.reshape(t0 + n, -1)[t0:]
+        assert np.max(np.abs(keys[sl] - k_new)) <= 1e-5 * np.max(np.abs(k_new))

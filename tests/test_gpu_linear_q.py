@@ -77,12 +77,14 @@ def test_linear_q_bit_exact(ctx, qtype, n_in, n_out, tokens):
 @pytest.mark.parametrize("n_in,n_out,tokens", [(512, 15, 2), (2560, 63, 16), (4608, 65, 17), (1024, 130, 32),
                                                (3584, 17, 33), (512, 257, 64), (5120, 34, 65), (1536, 129, 191),
                                                (512, 8190, 33), (1024, 2047, 100), (512, 3001, 700), (2304, 2111, 20),
-                                               (16384, 4111, 3), (2560, 1701, 16)])
+                                               (16384, 4111, 3), (2560, 1701, 16), (2560, 63, 20), (16384, 1031, 18),
+                                               (9728, 10260, 2)])
 def test_linear_gemm_tiles(ctx, qtype, n_in, n_out, tokens):
-    """The matrix-core tiles of each rule at the edges of their rows (16 a
-    wave), tokens (16, 32, 64) and block pipelines, and the rows the tiles
-    leave to the GEMV, bit for bit (STQ1_0: panel and raw row orders by the
-    token count)."""
+    """The matrix-core tiles at the edges of their rows (16 a wave), tokens
+    (16, 32, 64) and block pipelines, the rows the tiles leave to the GEMV, and
+    the shapes that the GEMV takes whole, bit for bit (STQ1_0: panel and raw
+    row orders by the token count).  Which kernel a shape takes:
+    test_linear_few_tokens, test_linear_q6k_forms, test_linear_q4k_forms."""
     n_in += -n_in % qb.VALUES[qtype]
     rng = np.random.default_rng(31 * qtype + n_in + n_out + tokens)
     w = qb.random_blocks(rng, qtype, qb.nblocks(qtype, n_out * n_in))
@@ -149,7 +151,8 @@ def test_linear_q6k_forms(ctx, n_in, n_out, tokens, kernels):
 
 @pytest.mark.parametrize("n_in,n_out,tokens,kernels", [
     (512, 32768, 16, ["linear_gemm<4>"]), (512, 32776, 16, ["q4k_gemm"]), (768, 65529, 2, ["linear_gemm<4>", "linear_q<4>"]),
-    (768, 32776, 18, ["q4k_gemm"]), (1280, 12291, 90, ["linear_gemm<4>", "linear_q<4>"]), (768, 3009, 800, ["q4k_gemm", "linear_q<4>"])])
+    (768, 32776, 18, ["q4k_gemm"]), (1280, 12291, 90, ["linear_gemm<4>", "linear_q<4>"]), (768, 3009, 800, ["q4k_gemm", "linear_q<4>"]),
+    (2560, 1041, 2050, ["q4k_gemm", "linear_q<4>"])])
 def test_linear_q4k_forms(ctx, n_in, n_out, tokens, kernels):
     """The same for Q4_K: small tiles and 64-token tiles, the GEMV for the last
     n_out % 8 rows."""
@@ -316,26 +319,33 @@ def test_linear_f32_tiles(ctx, n_in, n_out, tokens):
         a.free()
 
 
-@pytest.mark.parametrize("qtype", [4, 6])
-def test_tiled_pieces_match_whole_launch(monkeypatch, qtype):
-    """The tiled Q4_K / Q6_K kernels go in pieces of whole row and token tiles
-    when a call holds more than 2 GiB of weight rows or activations; a context
-    created with a 256 KiB piece limit splits ordinary shapes the same way
-    (several row and token pieces here), and the results stay bit-identical to
-    the oracle."""
+@pytest.fixture()
+def pieces_ctx(monkeypatch):
+    """A context whose kernels take at most 256 KiB of an operand at once, in
+    place of 2 GiB."""
     monkeypatch.setenv("Q35M_TILE_LIMIT_BYTES", str(256 * 1024))
     c = q35mix.Context(q35mix.qwen35_config(num_layers=1, is_recurrent=[1]), n_seqs=1, kv_capacity=16)
-    try:
-        n_in, n_out, tokens = (2560, 520, 200) if qtype == 4 else (2560, 424, 200)
-        say(f"pieces {NAMES[qtype]} n_in={n_in} n_out={n_out} tokens={tokens}")
-        rng = np.random.default_rng(4242 + qtype)
-        w = qb.random_blocks(rng, qtype, qb.nblocks(qtype, n_out * n_in))
-        x = rng.standard_normal((tokens, n_in)).astype(np.float32)
-        got = run(c, qtype, w, x, n_in, n_out)
-        want = oracle.linear_q(qtype, w, x, n_in, n_out)
-        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
-    finally:
-        c.close()
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("qtype,n_in,n_out,tokens", [(4, 512, 1104, 2000), (6, 1024, 424, 700), (6, 768, 425, 700)])
+def test_tiled_pieces_match_whole_launch(pieces_ctx, qtype, n_in, n_out, tokens):
+    """The 64-token-tile Q4_K / Q6_K kernels go in pieces of whole row and
+    token tiles when a call holds more than 2 GiB of weight rows or
+    activations; with a 256 KiB piece limit ordinary shapes split the same way
+    (several row and token pieces here), bit-identical to the oracle."""
+    ran = run_named(pieces_ctx, qtype, n_in, n_out, tokens, 4242)
+    assert ran["q4k_gemm" if qtype == 4 else "q6k_gemm"][1] >= 6
+
+
+@pytest.mark.parametrize("qtype,n_in,n_out,tokens", [(q, 2560, n, 200) for q in TYPES for n in (520, 424)] +
+                         [(q, 512, 2100, 1100) for q in (5, 14, 2, 1)] + [(4, 512, 2100, 450), (6, 1024, 60, 1900)])
+def test_small_tile_pieces_match_whole_launch(pieces_ctx, qtype, n_in, n_out, tokens):
+    """The same for linear_gemm's token pieces, in its split form and its 32-
+    and 64-token tiles."""
+    ran = run_named(pieces_ctx, qtype, n_in, n_out, tokens, 4243)
+    assert ran[f"linear_gemm<{qtype}>"][1] > 1
 
 
 BLOCK_SHAPES = [(2560, 8192, 2048), (4096, 2560, 2048), (2560, 520, 70), (512, 33, 5), (4096, 136, 130),
