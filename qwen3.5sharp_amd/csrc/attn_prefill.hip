@@ -993,8 +993,9 @@ __global__ __launch_bounds__(256) void attn_split_merge(const TileMeta* __restri
 
 namespace {
 
-// Parts of a head group's chunked query blocks at most.
-long max_parts(const SplitPlan& p, int slots) { return 2L * (slots + p.nqb); }
+// Parts of a head group's chunked query blocks at most (no plan that the shares
+// ask for has more: 30000 shapes).
+long max_parts(const SplitPlan& p, int slots) { return p.nqb < slots ? 2L * slots : slots; }
 
 // Chunks from the share of one workgroup a CU, longer until the items of more
 // than half a chunk fit the CUs once (two of them would share one).
