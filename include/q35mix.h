@@ -332,7 +332,8 @@ int q35m_device_count(int* count);
  * GEMM (MulMatQ4K.Gemm, MulMatQ4K.cs:45-127 -> GemmQ4K.GemmAvx2Tile,
  * GemmQ4K.Avx2.cs:39-207) for the first n_out & ~7 outputs and the GEMV for
  * the rest, as the reference splits them.  w and x must be 16-byte aligned;
- * n_in a multiple of 256 up to 16384. */
+ * n_in a multiple of 256 up to 16384.  y may overlap x: the rows are quantized
+ * before anything is stored. */
 int q35m_linear_q4k(q35m_ctx* ctx, const void* w, const float* x, float* y, int n_in, int n_out,
                     int tokens);
 int q35m_linear_q6k(q35m_ctx* ctx, const void* w, const float* x, float* y, int n_in, int n_out,
@@ -364,7 +365,7 @@ int q35m_linear_stq1_0(q35m_ctx* ctx, const void* w, const float* x, float* y, i
 /* F32 weights W [n_out][n_in] row-major in device memory (Qwen35Model.F32Gemm,
  * src/Qwen35Sharp.Model/Qwen35Model.Decode.cs:129-140, the reference's Linear
  * and DecodeLinear for F32 tensors): y[t][o] = Ops.DotF32(x[t], W[o])
- * (Ops.cs:418-449), bit-identical to it; any n_in >= 1. */
+ * (Ops.cs:418-449), bit-identical to it; any n_in >= 1; y and x apart. */
 int q35m_linear_f32(q35m_ctx* ctx, const float* w, const float* x, float* y, int n_in, int n_out,
                     int tokens);
 

@@ -204,6 +204,7 @@ __device__ __forceinline__ void flash_fp32_block(
         lds_barrier();
         Q35_STORE_ROW(0) Q35_STORE_ROW(1) Q35_STORE_ROW(2) Q35_STORE_ROW(3)
         Q35_STORE_ROW(4) Q35_STORE_ROW(5) Q35_STORE_ROW(6) Q35_STORE_ROW(7)
+        __builtin_amdgcn_sched_barrier(0);
 
         // S^T for positions p0 + 16 pb + (4g + r), queries c16.
         f32x4 st[2];
@@ -211,13 +212,7 @@ __device__ __forceinline__ void flash_fp32_block(
             f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
             float4 a0 = *reinterpret_cast<const float4*>(&Ks[c16][64 * g]);
             float4 a1 = *reinterpret_cast<const float4*>(&Ks[16 + c16][64 * g]);
-#pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                float4 n0 = a0, n1 = a1;
-                if (u < 15) {
-                    n0 = *reinterpret_cast<const float4*>(&Ks[c16][64 * g + 4 * (u + 1)]);
-                    n1 = *reinterpret_cast<const float4*>(&Ks[16 + c16][64 * g + 4 * (u + 1)]);
-                }
+            auto products = [&](int u) {
                 acc0 = mfma16(a0.x, qreg[4 * u], acc0);
                 acc1 = mfma16(a1.x, qreg[4 * u], acc1);
                 acc0 = mfma16(a0.y, qreg[4 * u + 1], acc0);
@@ -226,16 +221,25 @@ __device__ __forceinline__ void flash_fp32_block(
                 acc1 = mfma16(a1.z, qreg[4 * u + 2], acc1);
                 acc0 = mfma16(a0.w, qreg[4 * u + 3], acc0);
                 acc1 = mfma16(a1.w, qreg[4 * u + 3], acc1);
+            };
+#pragma unroll
+            for (int u = 0; u < 15; ++u) {
+                const float4 n0 = *reinterpret_cast<const float4*>(&Ks[c16][64 * g + 4 * (u + 1)]);
+                const float4 n1 = *reinterpret_cast<const float4*>(&Ks[16 + c16][64 * g + 4 * (u + 1)]);
+                products(u);
                 a0 = n0; a1 = n1;
             }
+            // Every wave has its last operands (the K tile is free) and the V
+            // tile is stored: refill K, load the next V into registers.  The
+            // last products run behind the barrier.
+            lds_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            if (it + 1 < n_iter) {
+                load_k(p0 + KT);
+                Q35_LOAD_TILE(p0 + KT)
+            }
+            products(15);
             st[0] = acc0; st[1] = acc1;
-        }
-        // Every wave is past S (the K tile is free) and the V tile is
-        // stored: refill K, load the next V into registers.
-        lds_barrier();
-        if (it + 1 < n_iter) {
-            load_k(p0 + KT);
-            Q35_LOAD_TILE(p0 + KT)
         }
 #undef Q35_LOAD_ROW
 #undef Q35_LOAD_TILE
@@ -577,11 +581,13 @@ __device__ __forceinline__ size_t part_slot(const SplitPlan& P, int qb, int c, i
 // hg of the block, with its q rows (RoPE and norm as rope_norm_row, then split)
 // and output accumulators in registers and the tiles, two buffers of 64 KiB,
 // shared by the eight waves.  A step (one tile) is 96 MFMAs and 64 KiB of LDS
-// reads a wave; it takes 2.9 us where its MFMAs alone take 2.1 (with the loads,
-// half the LDS reads and the softmax left out).  T = 2048 behind nothing 122 us
-// (fp32 MFMA 315), T = 4096 370 (1175), T = 133 behind 8000 rows 70 (1085, 36
-// workgroups).  32 rows a wave, one wave a SIMD, halves the LDS reads but moves
-// registers to and from the accumulation file: 508 us at T = 4096.
+// reads a wave and takes 2.9 us; the matrix pipes are busy 36 % of the kernel's
+// SIMD cycles at T = 2048, 47 % of those in which a CU has work
+// (profiles/tiled_kernels_counters.md), the rest is the softmax and the operand
+// reads in front of each product.  T = 2048 behind nothing 122-129 us (fp32 MFMA
+// 315), T = 4096 370 (1175), T = 133 behind 8000 rows 70 (1085, 36 workgroups).
+// 32 rows a wave, one wave a SIMD, halves the LDS reads but moves registers to
+// and from the accumulation file: 508 us at T = 4096.
 __global__ __launch_bounds__(64 * SWAVES, 2) void attn_split_flash(
     const uint4* __restrict__ planes, const TileMeta* __restrict__ meta, QRows Q, const float* __restrict__ K,
     const float* __restrict__ V, int cap, float* __restrict__ out, float* __restrict__ parts, int* __restrict__ fp32_done,

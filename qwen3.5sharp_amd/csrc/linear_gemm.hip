@@ -26,8 +26,9 @@
 // the chain's own operations.  The workgroup's waves share the tokens, CH
 // blocks at a time through two LDS buffers filled by buffer loads straight
 // into LDS while the other one is worked on.  Bound by instruction issue: Q5_K
-// at 500 tokens of 2560 -> 8192 issues on 98 % of its cycles, 448 VALU and 40
-// MFMA instructions a block of 16 rows x 64 tokens.
+// at 500 tokens of 2560 -> 8192 takes 451 VALU and 40 MFMA instructions a block
+// of 16 rows x 64 tokens and issues on 68 % of all SIMD cycles, 84 % of those
+// in which its CU has work (profiles/tiled_kernels_counters.md).
 #include <algorithm>
 
 #include "common.h"
