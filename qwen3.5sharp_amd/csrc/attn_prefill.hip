@@ -27,6 +27,18 @@
 namespace q35 {
 namespace {
 
+// 1 / (1 + e^-x) to fp32 precision in a dozen instructions: the exponential
+// with the rounding error of its base-2 argument made good, the reciprocal
+// with one Newton step (expf and a division are 45).
+__device__ __forceinline__ float sigmoid_full(float x) {
+    const float n = __builtin_amdgcn_fmed3f(-x, -88.0f, 88.0f);    // (past it 0 and 1 in any case)
+    const float l2 = 1.44269502e+0f, l2lo = 1.92596303e-8f, ln2 = 0.693147182f;   // log2(e) as a sum, ln 2
+    const float t = n * l2, d = fmaf(n, l2lo, fmaf(n, l2, -t));
+    const float p = __builtin_amdgcn_exp2f(t), s = 1.0f + fmaf(p * ln2, d, p);
+    const float r = __builtin_amdgcn_rcpf(s);
+    return x != x ? x : fmaf(fmaf(-s, r, 1.0f), r, r);
+}
+
 __global__ __launch_bounds__(kWave) void attn_prefill_prep(
     const float* __restrict__ knew, const float* __restrict__ vnew, const float* __restrict__ k_norm,
     float* __restrict__ K, float* __restrict__ V, const float* __restrict__ rope_cos,
@@ -92,6 +104,8 @@ struct QRows {
 
 // Query block qb (16 subs rows) of head group y; every thread of the
 // workgroup's 8 waves.  With subs > 1 the spare waves take further 16 rows.
+// KEYS false: the halves take a block each, 2 qb and 2 qb + 1, and all its keys.
+template <bool KEYS>
 __device__ __forceinline__ void flash_fp32_block(
     Tiles* smem, const QRows& Q, const float* __restrict__ K, const float* __restrict__ V,
     float* __restrict__ out, int start, int T, int nh, int nkv, int hg, int cap, int qb, int y, int subs) {
@@ -105,14 +119,14 @@ __device__ __forceinline__ void flash_fp32_block(
     const int g = lane >> 4, c16 = lane & 15;
     const bool stores = wave < hg * subs;    // uniform per wave
     const int unit = min(wave, hg * subs - 1), h = hg * y + unit % hg;
-    const int r0 = (qb * subs + unit / hg) * QR;
-    const int blk_len = start + min(T - 1, (qb + 1) * subs * QR - 1) + 1;
+    const int r0 = ((KEYS ? qb : 2 * qb + half) * subs + unit / hg) * QR;
+    const int blk_len = start + min(T - 1, (qb + 1) * (KEYS ? 1 : 2) * subs * QR - 1) + 1;
     const int my_t = min(r0 + c16, T - 1);
     const int my_len = start + my_t + 1;
     // Key tiles of this half: [t_begin, t_begin + n_iter), the last one past
     // blk_len (fully masked) when half 1 has one tile fewer.
-    const int n_tiles = (blk_len + KT - 1) / KT, n_iter = (n_tiles + 1) / 2;
-    const int p_begin = half * n_iter * KT;
+    const int n_tiles = (blk_len + KT - 1) / KT, n_iter = KEYS ? (n_tiles + 1) / 2 : n_tiles;
+    const int p_begin = KEYS ? half * n_iter * KT : 0;
     // Head-major cache: kv head kvh's rows are [cap][256] from kvh * cap * 256.
     const float* Kh = K + (size_t)kvh * cap * kHd;
     const float* Vh = V + (size_t)kvh * cap * kHd;
@@ -293,42 +307,53 @@ __device__ __forceinline__ void flash_fp32_block(
                 for (int d = 0; d < 4; ++d) O[4 * dq + d] = mfma16(v[d].w, st[pb][3], O[4 * dq + d]);
             }
     }
-    // Merge: half 1 hands (m, l, O) to half 0 through LDS (the tile buffers,
-    // free after the last barrier of the loop).
-    static_assert(4 * 64 * 66 * sizeof(float) <= sizeof(Tiles), "merge exchange fits one half's tiles");
-    float* xch = &smem[0].k[0][0];
-    float* xo = xch + (size_t)(wave * 64 + lane) * 64;
-    float* xml = xch + (size_t)4 * 64 * 64 + (size_t)(wave * 64 + lane) * 2;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (half == 1) {
+    float inv;
+    if constexpr (KEYS) {
+        // Merge: half 1 hands (m, l, O) to half 0 through LDS (the tile
+        // buffers, free after the last barrier of the loop).
+        static_assert(4 * 64 * 66 * sizeof(float) <= sizeof(Tiles), "merge exchange fits one half's tiles");
+        float* xch = &smem[0].k[0][0];
+        float* xo = xch + (size_t)(wave * 64 + lane) * 64;
+        float* xml = xch + (size_t)4 * 64 * 64 + (size_t)(wave * 64 + lane) * 2;
+        __syncthreads();
+        if (half == 1) {
 #pragma unroll
-        for (int db = 0; db < 16; ++db)
-            *reinterpret_cast<float4*>(xo + 4 * db) = make_float4(O[db][0], O[db][1], O[db][2], O[db][3]);
-        xml[0] = m_run;
-        xml[1] = l_run;
+            for (int db = 0; db < 16; ++db)
+                *reinterpret_cast<float4*>(xo + 4 * db) = make_float4(O[db][0], O[db][1], O[db][2], O[db][3]);
+            xml[0] = m_run;
+            xml[1] = l_run;
+        }
+        __syncthreads();
+        if (half == 1) return;
+        const float m1 = xml[0], l1 = xml[1];
+        const float m = fmaxf(m_run, m1);
+        const float a0 = __expf(m_run - m), a1 = m1 == -INFINITY ? 0.0f : __expf(m1 - m);
+        inv = 1.0f / (l_run * a0 + l1 * a1);
+#pragma unroll
+        for (int db = 0; db < 16; ++db) {
+            const float4 o1 = *reinterpret_cast<const float4*>(xo + 4 * db);
+            O[db][0] = O[db][0] * a0 + o1.x * a1;
+            O[db][1] = O[db][1] * a0 + o1.y * a1;
+            O[db][2] = O[db][2] * a0 + o1.z * a1;
+            O[db][3] = O[db][3] * a0 + o1.w * a1;
+        }
+    } else {
+        inv = 1.0f / l_run;
     }
-    __syncthreads();
-    if (half == 1) return;
-    const float m1 = xml[0], l1 = xml[1];
-    const float m = fmaxf(m_run, m1);
-    const float a0 = __expf(m_run - m), a1 = m1 == -INFINITY ? 0.0f : __expf(m1 - m);
-    const float l = l_run * a0 + l1 * a1;
     const int t = r0 + c16;
     if (t >= T || !stores) return;
-    const float inv = 1.0f / l;
-    const float* grow = q_gate + (size_t)t * 2 * nh * kHd + (size_t)h * 2 * kHd + kHd;
+    const float* grow = q_gate + ((size_t)t * nh + h) * 2 * kHd + kHd;
     float* orow = out + ((size_t)t * nh + h) * kHd;
 #pragma unroll
     for (int db = 0; db < 16; ++db) {
         const int d0 = 16 * db + 4 * g;
-        const float4 o1 = *reinterpret_cast<const float4*>(xo + 4 * db);
         const float4 gt = *reinterpret_cast<const float4*>(grow + d0);
         float4 r;
-        r.x = (O[db][0] * a0 + o1.x * a1) * inv * (1.0f / (1.0f + expf(-gt.x)));
-        r.y = (O[db][1] * a0 + o1.y * a1) * inv * (1.0f / (1.0f + expf(-gt.y)));
-        r.z = (O[db][2] * a0 + o1.z * a1) * inv * (1.0f / (1.0f + expf(-gt.z)));
-        r.w = (O[db][3] * a0 + o1.w * a1) * inv * (1.0f / (1.0f + expf(-gt.w)));
+        r.x = O[db][0] * inv * sigmoid_full(gt.x);
+        r.y = O[db][1] * inv * sigmoid_full(gt.y);
+        r.z = O[db][2] * inv * sigmoid_full(gt.z);
+        r.w = O[db][3] * inv * sigmoid_full(gt.w);
         *reinterpret_cast<float4*>(orow + d0) = r;
     }
 }
@@ -339,7 +364,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_flash(
     __shared__ Tiles smem[2];
     const int groups = nh / hg, nqb = (T + QR - 1) / QR;
     const int rank = blockIdx.x;                 // heaviest query blocks first
-    flash_fp32_block(smem, Q, K, V, out, start, T, nh, nkv, hg, cap, nqb - 1 - rank / groups, rank % groups, 1);
+    flash_fp32_block<true>(smem, Q, K, V, out, start, T, nh, nkv, hg, cap, nqb - 1 - rank / groups, rank % groups, 1);
 }
 
 // ---------------------------------------------------------------- split fp16
@@ -555,18 +580,6 @@ __device__ __forceinline__ f32x4 mfma_h(f16x8 a, f16x8 b, f32x4 c) { return __bu
 // A part's floats in the workspace: O as each wave's registers, then (m, l) a lane.
 constexpr size_t kPartFloats = (size_t)SWAVES * 64 * 64 + (size_t)SWAVES * 64 * 2;
 
-// 1 / (1 + e^-x) to fp32 precision in a dozen instructions: the exponential
-// with the rounding error of its base-2 argument made good, the reciprocal
-// with one Newton step (expf and a division are 45).
-__device__ __forceinline__ float sigmoid_full(float x) {
-    const float n = __builtin_amdgcn_fmed3f(-x, -88.0f, 88.0f);    // (past it 0 and 1 in any case)
-    const float l2 = 1.44269502e+0f, l2lo = 1.92596303e-8f, ln2 = 0.693147182f;   // log2(e) as a sum, ln 2
-    const float t = n * l2, d = fmaf(n, l2lo, fmaf(n, l2, -t));
-    const float p = __builtin_amdgcn_exp2f(t), s = 1.0f + fmaf(p * ln2, d, p);
-    const float r = __builtin_amdgcn_rcpf(s);
-    return x != x ? x : fmaf(fmaf(-s, r, 1.0f), r, r);
-}
-
 __device__ __forceinline__ float4 gated(float4 o, float4 gate) {
     return make_float4(o.x * sigmoid_full(gate.x), o.y * sigmoid_full(gate.y), o.z * sigmoid_full(gate.z),
                        o.w * sigmoid_full(gate.w));
@@ -737,16 +750,17 @@ __global__ __launch_bounds__(64 * SWAVES, 2) void attn_split_flash(
     if (c == 0 && tid == 0 && n > P.chunk) fp32_done[(qb - P.first_multi) * P.groups + y] = bad;
     if (bad) {
         // The block's rows in two halves, one to each of its first two chunks'
-        // workgroups (133 tokens behind 8000 rows of 4 q heads a kv head 1160
-        // us, of one 1174; all in the first chunk's, 16 rows after another, 2299
-        // and 9078; the fp32 kernels alone 1097).  A block of one chunk has
-        // them after one another (64 tokens 62, the fp32 kernels 25).
+        // workgroups (133 tokens behind 8000 rows of 4 q heads a kv head 1150
+        // us, of one 1162; all in the first chunk's, 16 rows after another, 2299
+        // and 9078; the fp32 kernels alone 1090), or one to each half of a
+        // single chunk's (64 tokens 47, one after the other 62; 25).
         const int subs = 4 / P.hg, nch = (n + P.chunk - 1) / P.chunk;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        for (int b = c; b < 2 && (2 * qb + b) * subs * QR < P.T; b += nch) {
-            __syncthreads();
-            flash_fp32_block(lds.fp32, Q, K, V, out, P.start, P.T, P.nh, P.nkv, P.hg, cap, 2 * qb + b, y, subs);
-        }
+        __syncthreads();
+        if (nch == 1)
+            flash_fp32_block<false>(lds.fp32, Q, K, V, out, P.start, P.T, P.nh, P.nkv, P.hg, cap, qb, y, subs);
+        else if (c < 2 && (2 * qb + c) * subs * QR < P.T)
+            flash_fp32_block<true>(lds.fp32, Q, K, V, out, P.start, P.T, P.nh, P.nkv, P.hg, cap, 2 * qb + c, y, subs);
         return;
     }
 
