@@ -153,7 +153,7 @@ __global__ __launch_bounds__(NT, 2) void attn_decode_partial(
             const float4 qj = q_s[h][l16 + 16 * j];                                              \
             t += qj.x * kk[m][j].x + qj.y * kk[m][j].y + qj.z * kk[m][j].z + qj.w * kk[m][j].w;  \
         }                                                                                        \
-        a[m][h] = row_sum_shuffle(t);                                                              \
+        a[m][h] = row_sum_shuffle(t);                                                           \
     }
     // With one sub-chunk a workgroup, its rows are scored in load order (row
     // block m outer), so the first blocks are scored while later K rows are

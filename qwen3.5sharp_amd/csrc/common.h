@@ -13,8 +13,6 @@ __device__ __forceinline__ float silu(float x) {
     return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x));
 }
 
-__device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + __expf(-x)); }
-
 // Qwen35Ops.SoftplusScalar / Log1pSafe (src/Qwen35Sharp.Model/Qwen35Ops.cs:
 // 121-142): identity above 20, exp below -10, otherwise log(1 + e^x) with a
 // 4-term Taylor series whenever e^x < 0.5.  The series is part of the
@@ -110,10 +108,6 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
-// Non-temporal 16-byte load and store (global_load / global_store_dwordx4 with
-// the nt bit): for data streamed through once per call, such as decode states
-// and KV rows, so that it does not evict from L2 and MALL what the following
-// kernels read.
 // Buffer loads straight into LDS (no registers): lane l's 4 or 16 bytes at
 // voff + soff of the descriptor's range go to lds + size * l; offsets past
 // the range read as zero.  Completion is waited for with vmcnt.
@@ -126,6 +120,10 @@ __device__ __forceinline__ void dma_b128(__amdgpu_buffer_rsrc_t rs, void* lds, u
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)lds, 16, voff, soff, 0, 0);
 }
 
+// Non-temporal 16-byte load and store (global_load / global_store_dwordx4 with
+// the nt bit): for data streamed through once per call, such as decode states
+// and KV rows, so that it does not evict from L2 and MALL what the following
+// kernels read.
 typedef float nt_f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float4 load_nt(const float* p) {
     const nt_f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const nt_f32x4*>(p));

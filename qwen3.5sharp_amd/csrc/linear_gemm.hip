@@ -126,30 +126,6 @@ template <> struct RowBlock<1> {       // d; slots and signs of chunk lg (16 gro
     }
 };
 
-// Four IQ4_XS grid values (IQ4XS.cs:15-18) of four 4-bit indices, one a byte.
-__device__ __forceinline__ uint32_t iq4_grid(uint32_t idx) {
-    // grid bytes: -127 -104 -83 -65 | -49 -35 -22 -10 | 1 13 25 38 | 53 69 89 113
-    const uint32_t g0 = 0xBFAD9881u, g1 = 0xF6EADDCFu, g2 = 0x26190D01u, g3 = 0x71594535u;
-    const uint32_t sel = idx & 0x07070707u;
-    const uint32_t m = ((idx >> 3) & 0x01010101u) * 0xffu;
-    const uint32_t lo = __builtin_amdgcn_perm(g1, g0, sel), hi = __builtin_amdgcn_perm(g3, g2, sel);
-    return (lo & ~m) | (hi & m);
-}
-
-// The four-lane patterns of STQ1_0 groups 4 i .. + 3 of a chunk, one a byte
-// (see stq_unit_dot in linear_q.hip): h the groups' 4-bit slots, s4 their signs.
-__device__ __forceinline__ uint32_t stq_patterns(uint32_t h, uint32_t s4) {
-    constexpr uint32_t L0 = 0x092989A9u, L1 = 0x062686A6u, L2 = 0x121A929Au, L3 = 0x424A626Au;
-    constexpr uint32_t H0 = 0xA1812101u, H1 = 0xA4842404u, H2 = 0x98901810u, H3 = 0x68604840u;
-    const uint32_t idx = (h & 0xfu) | ((h & 0xf0u) << 4) | ((h & 0xf00u) << 8) | ((h & 0xf000u) << 12);
-    const uint32_t sel = idx & 0x07070707u;
-    const uint32_t hib = ((idx >> 3) & 0x01010101u) * 0xffu;
-    const uint32_t lo = (__builtin_amdgcn_perm(L1, L0, sel) & ~hib) | (__builtin_amdgcn_perm(L3, L2, sel) & hib);
-    const uint32_t hi = (__builtin_amdgcn_perm(H1, H0, sel) & ~hib) | (__builtin_amdgcn_perm(H3, H2, sel) & hib);
-    const uint32_t neg = ((s4 * 0x00204081u) & 0x01010101u) * 0xffu;
-    return (lo & ~neg) | (hi & neg);
-}
-
 // v of the four 16-lane groups, in every lane.
 __device__ __forceinline__ void lane_groups(uint32_t v, uint32_t (&r)[4]) {
     const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);

@@ -493,31 +493,21 @@ __device__ __forceinline__ void q5k_block_terms(const uint32_t* __restrict__ wb,
 
 // IQ4_XS x Q8_K block: acc[ib] = q8 . grid[idx] over sub-block ib (16 bytes:
 // low nibbles pair with q8 bytes 32 ib .. + 15, high nibbles with 32 ib +
-// 16 ..).  The grid (IQ4XS.cs:15-18) is looked up 4 bytes at a time with two
-// byte permutes (entries 0-7 and 8-7) and a select on the index's bit 3.
-// wb: the block's 34 dwords.
+// 16 ..), the grid looked up 4 bytes at a time.  wb: the block's 34 dwords.
 __device__ __forceinline__ void iq4xs_block_terms(const uint32_t* __restrict__ wb,
                                                   const uint32_t* __restrict__ q8b, int (&acc)[8]) {
-    // grid bytes: -127 -104 -83 -65 | -49 -35 -22 -10 | 1 13 25 38 | 53 69 89 113
-    const uint32_t g0 = 0xBFAD9881u, g1 = 0xF6EADDCFu, g2 = 0x26190D01u, g3 = 0x71594535u;
     uint4 qv[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) qv[i] = reinterpret_cast<const uint4*>(q8b + Q8K_QS)[i];
     const uint32_t* q8 = reinterpret_cast<const uint32_t*>(qv);
-    auto lookup = [&](uint32_t idx) {      // idx: four 4-bit indices, one a byte
-        const uint32_t sel = idx & 0x07070707u;
-        const uint32_t m = ((idx >> 3) & 0x01010101u) * 0xffu;
-        const uint32_t lo = __builtin_amdgcn_perm(g1, g0, sel), hi = __builtin_amdgcn_perm(g3, g2, sel);
-        return (lo & ~m) | (hi & m);
-    };
 #pragma unroll
     for (int ib = 0; ib < 8; ++ib) {
         int a = 0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const uint32_t wv = wb[2 + 4 * ib + k];
-            a = __builtin_amdgcn_sdot4((int)lookup(wv & 0x0f0f0f0fu), (int)q8[8 * ib + k], a, false);
-            a = __builtin_amdgcn_sdot4((int)lookup((wv >> 4) & 0x0f0f0f0fu), (int)q8[8 * ib + 4 + k], a, false);
+            a = __builtin_amdgcn_sdot4((int)iq4_grid(wv & 0x0f0f0f0fu), (int)q8[8 * ib + k], a, false);
+            a = __builtin_amdgcn_sdot4((int)iq4_grid((wv >> 4) & 0x0f0f0f0fu), (int)q8[8 * ib + 4 + k], a, false);
         }
         acc[ib] = a;
     }
@@ -670,15 +660,9 @@ __device__ __forceinline__ int q2_unit_dot(const uint32_t* __restrict__ base, in
 }
 
 // STQ1_0 block at byte offset o times a Q8_K block: encoded - S.  Four groups
-// at a time: their slots (nibbles of one 16-bit half of qs) spread to bytes,
-// looked up in the two 16-byte codebook halves with byte permutes, the half
-// chosen per byte by the group's sign bit; lane L of the four patterns then
-// meets activations chunk * 64 + 16 L + 4 i .. + 3.
+// at a time (stq_patterns): lane L of the four patterns meets activations chunk * 64 + 16 L + 4 i .. + 3.
 __device__ __forceinline__ int stq_unit_dot(const uint32_t* __restrict__ base, int o,
                                             const uint32_t* __restrict__ q8b) {
-    // STQ1_0.Codebook, entries 0-15 (sign 0) and 16-31 (sign 1), 4 a dword
-    constexpr uint32_t L0 = 0x092989A9u, L1 = 0x062686A6u, L2 = 0x121A929Au, L3 = 0x424A626Au;
-    constexpr uint32_t H0 = 0xA1812101u, H1 = 0xA4842404u, H2 = 0x98901810u, H3 = 0x68604840u;
     uint32_t qs[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) qs[j] = lds_word(base, o + 4 * j);
@@ -691,13 +675,7 @@ __device__ __forceinline__ int stq_unit_dot(const uint32_t* __restrict__ base, i
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t h = (qs[2 * c + (i >> 1)] >> (16 * (i & 1))) & 0xffffu;
-            const uint32_t idx = (h & 0xfu) | ((h & 0xf0u) << 4) | ((h & 0xf00u) << 8) | ((h & 0xf000u) << 12);
-            const uint32_t sel = idx & 0x07070707u;
-            const uint32_t hib = ((idx >> 3) & 0x01010101u) * 0xffu;
-            const uint32_t lo = (__builtin_amdgcn_perm(L1, L0, sel) & ~hib) | (__builtin_amdgcn_perm(L3, L2, sel) & hib);
-            const uint32_t hi = (__builtin_amdgcn_perm(H1, H0, sel) & ~hib) | (__builtin_amdgcn_perm(H3, H2, sel) & hib);
-            const uint32_t neg = ((((s16 >> (4 * i)) & 0xfu) * 0x00204081u) & 0x01010101u) * 0xffu;
-            const uint32_t p = (lo & ~neg) | (hi & neg);
+            const uint32_t p = stq_patterns(h, (s16 >> (4 * i)) & 0xfu);
 #pragma unroll
             for (int L = 0; L < 4; ++L)
                 enc = __builtin_amdgcn_sdot4((int)((p >> (2 * L)) & 0x03030303u), (int)q8[16 * c + 4 * L + i], enc,
