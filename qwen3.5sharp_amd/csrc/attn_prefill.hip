@@ -595,12 +595,12 @@ __device__ __forceinline__ size_t part_slot(const SplitPlan& P, int qb, int c, i
 // and output accumulators in registers and the tiles, two buffers of 64 KiB,
 // shared by the eight waves.  A step (one tile) is 96 MFMAs and 64 KiB of LDS
 // reads a wave and takes 2.9 us; the matrix pipes are busy 36 % of the kernel's
-// SIMD cycles at T = 2048, 47 % of those in which a CU has work
-// (profiles/tiled_kernels_counters.md), the rest is the softmax and the operand
-// reads in front of each product.  T = 2048 behind nothing 122-129 us (fp32 MFMA
-// 315), T = 4096 370 (1175), T = 133 behind 8000 rows 70 (1085, 36 workgroups).
-// 32 rows a wave, one wave a SIMD, halves the LDS reads but moves registers to
-// and from the accumulation file: 508 us at T = 4096.
+// SIMD cycles at T = 2048, 47 % of those in which a CU has work, the rest is the
+// softmax and the operand reads in front of each product.  T = 2048 behind
+// nothing 122-129 us (fp32 MFMA 315), T = 4096 370 (1175), T = 133 behind 8000
+// rows 70 (1085, 36 workgroups).  32 rows a wave, one wave a SIMD, halves the
+// LDS reads but moves registers to and from the accumulation file: 508 us at
+// T = 4096.
 __global__ __launch_bounds__(64 * SWAVES, 2) void attn_split_flash(
     const uint4* __restrict__ planes, const TileMeta* __restrict__ meta, QRows Q, const float* __restrict__ K,
     const float* __restrict__ V, int cap, float* __restrict__ out, float* __restrict__ parts, int* __restrict__ fp32_done,

@@ -28,7 +28,7 @@
 // into LDS while the other one is worked on.  Bound by instruction issue: Q5_K
 // at 500 tokens of 2560 -> 8192 takes 451 VALU and 40 MFMA instructions a block
 // of 16 rows x 64 tokens and issues on 68 % of all SIMD cycles, 84 % of those
-// in which its CU has work (profiles/tiled_kernels_counters.md).
+// in which its CU has work.
 #include <algorithm>
 
 #include "common.h"
